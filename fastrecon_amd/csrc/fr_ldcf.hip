@@ -40,10 +40,10 @@
 // and multiplies by W2^T held as eight A fragments; the D fragments (lane l:
 // sample l%16, outputs 16mt+4(l/16)+i) feed SiLU and the 64 -> 1 layer, whose
 // four partial sums per sample are added across lane groups in a fixed order.
-// Training recomputes this forward, back-propagates in FP32 and accumulates
-// each wave's weight gradient in registers; per-wave partials are summed in
-// wave order by a second kernel (deterministic), then Adam updates the FP32
-// master weights and refreshes the BF16 copies.
+// Training recomputes this forward, back-propagates in FP32 on the matrix
+// cores and accumulates each wave's weight gradient in registers; one partial
+// per workgroup, summed in a fixed order by a second kernel (deterministic),
+// then Adam updates the FP32 master weights and refreshes the BF16 copies.
 #include "fr_internal.h"
 
 #include <algorithm>
@@ -624,42 +624,6 @@ struct mlp_dev {
     const uint16_t *w3;      // [64] BF16
 };
 
-// W2^T as A fragments: fragment (mt, ks), lane l holds W2[k][m] for
-// m = 16 mt + l%16, k = 32 ks + 8 (l/16) + j, j = 0..7.
-__device__ inline void load_a(const mlp_dev &W, int lane, u32x4 (&a)[4][2])
-{
-    const int m0 = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            uint32_t w[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) w[j] = W.w2[(32 * ks + 8 * g + j) * H + 16 * mt + m0];
-            a[mt][ks] = u32x4{w[0] | (w[1] << 16), w[2] | (w[3] << 16), w[4] | (w[5] << 16), w[6] | (w[7] << 16)};
-        }
-}
-
-// Forward for the 16 samples of one wave.  Lane l: sample l%16.
-// Outputs: z1[ks][j] (unit 32ks+8g+j), h1b (BF16-rounded h1 as float),
-// z2[mt][i] (output 16mt+4g+i), h2, y (identical in the 4 lanes of a sample).
-struct fwd_state {
-    float z1[2][8], h1[2][8];
-    float z2[4][4], h2[4][4];
-    float y;
-};
-
-// Where the forward reads the layer-1 weights, the biases and w3: straight
-// from the device parameters, or from a workgroup's LDS copy (same values).
-struct wsrc_global {
-    const mlp_dev &W;
-    __device__ float w1(int i, int k) const { return bf2f(W.w1[i * H + k]); }
-    __device__ float b1(int k) const { return W.p[O_B1 + k]; }
-    __device__ float b2(int o) const { return W.p[O_B2 + o]; }
-    __device__ float w3(int o) const { return bf2f(W.w3[o]); }
-    __device__ float b3() const { return W.p[O_B3]; }
-};
-
 struct lds_weights {
     float w1[NF][H];
     float b1[H], b2[H], w3[H];
@@ -686,55 +650,6 @@ __device__ inline void stage_weights(const mlp_dev &W, lds_weights &L)
     if (threadIdx.x == 0) L.b3 = W.p[O_B3];
 }
 
-template <class WS>
-__device__ inline void mlp_forward16(const WS &W, const u32x4 (&a)[4][2], const float *x, int lane, fwd_state &F)
-{
-    const int g = lane >> 4;
-    u32x4 b[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        float h[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = 32 * ks + 8 * g + j;
-            float z = W.b1(k);
-#pragma unroll
-            for (int i = 0; i < NF; ++i) z = fmaf(x[i], W.w1(i, k), z);
-            F.z1[ks][j] = z;
-            h[j] = silu(z);
-        }
-        uint32_t hb[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            hb[j] = pack_bf16(h[2 * j], h[2 * j + 1]);
-            F.h1[ks][2 * j] = bf2f(hb[j] & 0xffffu);
-            F.h1[ks][2 * j + 1] = bf2f(hb[j] >> 16);
-        }
-        b[ks] = u32x4{hb[0], hb[1], hb[2], hb[3]};
-    }
-    float part = 0.f;
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[mt][0]),
-                                                     __builtin_bit_cast(bf16x8, b[0]), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[mt][1]),
-                                                     __builtin_bit_cast(bf16x8, b[1]), acc, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int o = 16 * mt + 4 * g + i;
-            const float z = __fadd_rn(acc[i], W.b2(o));
-            F.z2[mt][i] = z;
-            F.h2[mt][i] = silu(z);
-            part = fmaf(F.h2[mt][i], W.w3(o), part);
-        }
-    }
-    // the four lane groups hold the partial sums of the same sample
-    const float p1 = __fadd_rn(part, __shfl_xor(part, 16));
-    const float p2 = __fadd_rn(p1, __shfl_xor(p1, 32));
-    F.y = __fadd_rn(p2, W.b3());
-}
-
 // ------------------------------------------------------------- inference
 // Inference runs both dense layers on MFMA.  Layer 1 (FP32 16x16x4, two K
 // steps of four features): A = W1^T fragments (lane l: W1[4s + l/16][16mt +
@@ -744,8 +659,7 @@ __device__ inline void mlp_forward16(const WS &W, const u32x4 (&a)[4][2], const 
 // units in the order that puts exactly those sixteen units into lane l's
 // BF16 B operand: K position 32ks + 8(l/16) + j holds unit hidden_of(...)
 // = 16(2ks + j/4) + 4(l/16) + j%4, and W2's A fragments are loaded in the
-// same order.  Against the training forward (mlp_forward16, sequential FMAs
-// in layer 1) only the FP32 summation order of z1 differs.
+// same order.  The training pass runs the same forward.
 __device__ inline int hidden_of(int k)
 {
     const int ks = k >> 5, g = (k >> 3) & 3, j = k & 7;
@@ -811,13 +725,6 @@ __device__ inline float mlp_infer16(const WS &W, const infer_frags &F, float x0,
     const float p1 = __fadd_rn(part, __shfl_xor(part, 16));
     const float p2 = __fadd_rn(p1, __shfl_xor(p1, 32));
     return __fadd_rn(p2, W.b3());
-}
-
-__device__ inline void load_x(const float *__restrict__ feat, int64_t row, float *x)
-{
-    const float4 *r = reinterpret_cast<const float4 *>(feat + row * FSTRIDE);
-    const float4 a = r[0], b = r[1];
-    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
 }
 
 // mode 0: y; mode 1: the DCF exp(mu + sigma y - lb), lb = 8 x_k for a
@@ -891,128 +798,241 @@ __global__ void __launch_bounds__(256) k_ldcf_dcf(mlp_dev W, const float *__rest
 }
 
 // Training pass over a batch: forward, MSE loss against t (normalised
-// targets), back-propagation; each wave writes its gradient partial
-// (NPARAM floats) and loss partial to its slot.  Every wave runs the same
-// number of 16-sample groups (groups past the batch are masked), so the
-// block barriers match.
+// targets), back-propagation.  Each wave takes groups of 16 samples; every
+// contraction runs on the matrix cores, the FP32 ones on v_mfma_f32_16x16x4.
+//
+// Two layouts of a 16-sample tile of hidden values:
+//   "by unit":   lane (g, j) holds unit 16 mt + 4 g + r of sample j, the
+//                forward's (mlp_infer16);
+//   "by sample": lane (g, j) holds unit 16 nt + j of sample 4 g + r, what the
+//                same products give with their operands swapped.
+// A register of either is, without any exchange between lanes, an operand of
+// a K = 4 product: by unit for a sum over units (dh1 = W2 dz2), by sample
+// for a sum over samples (the weight gradients), K position g standing for
+// unit 16 mt + 4 g + r or sample 4 g + r.  So both layers run twice (16
+// products and 32 SiLUs a lane more per group) and nothing goes through LDS.
+// b1's gradient is row 8 of W1's: feature "8" is 1.
+//
+// The waves of a workgroup add their sums in LDS in a fixed order and write
+// one slot per workgroup, one workgroup per CU.  Bound by the FP32 matrix
+// products (160 of 32 cycles per group: 9 us for 65,536 rows) and the serial
+// start and end of a wave's four groups.  65,536 rows: 217 -> 31 us, and the
+// slot sums 958 -> 4 us (before: VALU products through LDS and one slot per
+// wave, 79 MB of them, added by one thread per parameter).
 constexpr int TB_WAVES = 4;
-struct wave_lds {
-    float x[16][NF];
-    float h1[16][H];
-    float h2[16][H];
-    float dz2[16][H];
-    float dz1[16][H];
-    float dy[16];
-};
+constexpr int TB_VALUES = 64 + 16 + 10;      // a lane's sums: W2, W1 (and b1), b2, w3, b3, loss
 
-__global__ void __launch_bounds__(256) k_mlp_backward(mlp_dev W, const float *__restrict__ feat,
-                                                      const float *__restrict__ targ, const int64_t *__restrict__ idx,
-                                                      int64_t B, int iters, float *__restrict__ partial)
+__global__ void __launch_bounds__(64 * TB_WAVES, 1) k_mlp_backward(mlp_dev W, const float *__restrict__ feat,
+                                                               const float *__restrict__ targ,
+                                                               const int64_t *__restrict__ idx, int64_t B,
+                                                               float *__restrict__ partial)
 {
-    __shared__ wave_lds L[TB_WAVES];
-    __shared__ float w2f[H][H + 1];
+    __shared__ lds_weights LW;
+    __shared__ float red[TB_WAVES / 2 * TB_VALUES * 64];
+    stage_weights(W, LW);
     const int lane = threadIdx.x & 63;
     const int wv = threadIdx.x >> 6;
-    const int64_t wave = (int64_t)blockIdx.x * TB_WAVES + wv;
+    const int g = lane >> 4, j = lane & 15;
     const int64_t nwaves = (int64_t)gridDim.x * TB_WAVES;
-    for (int q = threadIdx.x; q < H * H; q += blockDim.x) w2f[q / H][q % H] = bf2f(W.w2[q]);
-    u32x4 a[4][2];
-    load_a(W, lane, a);
-    __syncthreads();
-
-    const int g = lane >> 4, sl = lane & 15;
-    float gW2[H];
+    infer_frags F;
+    load_infer_frags(W, lane, F);
+    uint2 wb[4][4];                          // W2[16 nt + j][16 mt + 4 g + 0..3], BF16
 #pragma unroll
-    for (int o = 0; o < H; ++o) gW2[o] = 0.f;
-    float gW1[NF];
-#pragma unroll
-    for (int i = 0; i < NF; ++i) gW1[i] = 0.f;
-    float gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, gl = 0.f;
-    const float inv2B = 2.0f / (float)B;
-    wave_lds &S = L[wv];
-
-    for (int it = 0; it < iters; ++it) {
-        const int64_t gi = wave + (int64_t)it * nwaves;
-        const int64_t b = gi * 16 + sl;
-        const bool valid = b < B;
-        const int64_t row = valid ? (idx ? idx[b] : b) : (idx ? idx[0] : 0);
-        float x[NF];
-        load_x(feat, row, x);
-        fwd_state F;
-        mlp_forward16(wsrc_global{W}, a, x, lane, F);
-        const float r = valid ? __fsub_rn(F.y, targ[row]) : 0.f;
-        const float dy = __fmul_rn(inv2B, r);
-        // dz2 for the lane's outputs; stage the per-sample rows in LDS
+    for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
         for (int mt = 0; mt < 4; ++mt)
+            wb[nt][mt] = *reinterpret_cast<const uint2 *>(W.w2 + (16 * nt + j) * H + 16 * mt + 4 * g);
+    __syncthreads();
+    const wsrc_lds ws{LW};
+
+    union {
+        struct {
+            f32x4 w2[4][4], w1[4];           // tile (mt, nt) of W2's, nt of W1's: row 4 g + r, column j
+            float b2[4], w3[4], b3, loss;
+        };
+        float v[TB_VALUES];
+    } G;
+#pragma unroll
+    for (int i = 0; i < TB_VALUES; ++i) G.v[i] = 0.f;
+    const float inv2B = 2.0f / (float)B;
+    const int64_t groups = (B + 15) / 16;
+
+    for (int64_t gi = (int64_t)blockIdx.x * TB_WAVES + wv; gi < groups; gi += nwaves) {
+        const int64_t b = gi * 16 + j;
+        const bool valid = b < B;
+        const int64_t row = valid ? (idx ? idx[b] : b) : (idx ? idx[0] : 0);
+        const float x0 = feat[row * FSTRIDE + g], x1 = feat[row * FSTRIDE + 4 + g];
+        const float t = targ[row];
+        // layer 1 by unit (layer 2's operand) and by sample (h1 and SiLU')
+        uint32_t hb[4][2];
+        float h1[4][4], d1[4][4];
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            const int u = 16 * mt + 4 * g;
+            f32x4 z = {ws.b1(u), ws.b1(u + 1), ws.b1(u + 2), ws.b1(u + 3)};
+            z = __builtin_amdgcn_mfma_f32_16x16x4f32(F.a1[mt][0], x0, z, 0, 0, 0);
+            z = __builtin_amdgcn_mfma_f32_16x16x4f32(F.a1[mt][1], x1, z, 0, 0, 0);
+            hb[mt][0] = pack_bf16(silu(z[0]), silu(z[1]));
+            hb[mt][1] = pack_bf16(silu(z[2]), silu(z[3]));
+            const float bj = ws.b1(16 * mt + j);
+            f32x4 zs = {bj, bj, bj, bj};
+            zs = __builtin_amdgcn_mfma_f32_16x16x4f32(x0, F.a1[mt][0], zs, 0, 0, 0);
+            zs = __builtin_amdgcn_mfma_f32_16x16x4f32(x1, F.a1[mt][1], zs, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const uint32_t h = pack_bf16(silu(zs[r]), silu(zs[r + 1]));
+                h1[mt][r] = bf2f(h & 0xffffu);
+                h1[mt][r + 1] = bf2f(h >> 16);
+                d1[mt][r] = dsilu(zs[r]);
+                d1[mt][r + 1] = dsilu(zs[r + 1]);
+            }
+        }
+        bf16x8 h[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+            h[ks] = __builtin_bit_cast(bf16x8, u32x4{hb[2 * ks][0], hb[2 * ks][1], hb[2 * ks + 1][0], hb[2 * ks + 1][1]});
+        // layer 2 by unit: the output and w3 SiLU'
+        float dz2[4][4];
+        float part = 0.f;
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt) {
+            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, F.a2[mt][0]), h[0], z, 0, 0, 0);
+            z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, F.a2[mt][1]), h[1], z, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int o = 16 * mt + 4 * g + i;
-                S.h2[sl][o] = F.h2[mt][i];
-                S.dz2[sl][o] = __fmul_rn(__fmul_rn(dy, bf2f(W.w3[o])), dsilu(F.z2[mt][i]));
+                const float zi = __fadd_rn(z[i], ws.b2(o));
+                part = fmaf(silu(zi), ws.w3(o), part);
+                dz2[mt][i] = __fmul_rn(ws.w3(o), dsilu(zi));
+            }
+        }
+        const float p1 = __fadd_rn(part, __shfl_xor(part, 16));
+        const float y = __fadd_rn(__fadd_rn(p1, __shfl_xor(p1, 32)), ws.b3());
+        const float res = valid ? __fsub_rn(y, t) : 0.f;
+        const float dy = __fmul_rn(inv2B, res);
+        float dys[4], xs[4];                 // sample 4 g + r: its dy, its feature j (1 for j = 8, 0 above)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            dys[r] = __shfl(dy, 4 * g + r);
+            const int src = 16 * (j & 3) + 4 * g + r;
+            const float v0 = __shfl(x0, src), v1 = __shfl(x1, src);
+            xs[r] = j < 4 ? v0 : (j < 8 ? v1 : (j == 8 ? 1.f : 0.f));
+        }
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dz2[mt][i] = __fmul_rn(dy, dz2[mt][i]);
+        // layer 2 by sample: gradients of b2, w3 and W2
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            f32x4 z = {0.f, 0.f, 0.f, 0.f};
+            z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h[0], __builtin_bit_cast(bf16x8, F.a2[nt][0]), z, 0, 0, 0);
+            z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h[1], __builtin_bit_cast(bf16x8, F.a2[nt][1]), z, 0, 0, 0);
+            const float bj = ws.b2(16 * nt + j), wj = ws.w3(16 * nt + j);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float zr = __fadd_rn(z[r], bj);
+                G.w3[nt] = fmaf(silu(zr), dys[r], G.w3[nt]);
+                z[r] = __fmul_rn(dys[r], __fmul_rn(wj, dsilu(zr)));
+                G.b2[nt] = __fadd_rn(G.b2[nt], z[r]);
             }
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
+            for (int r = 0; r < 4; ++r)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) S.h1[sl][32 * ks + 8 * g + j] = F.h1[ks][j];
+                for (int mt = 0; mt < 4; ++mt)
+                    G.w2[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(h1[mt][r], z[r], G.w2[mt][nt], 0, 0, 0);
+        }
+        // dh1 by sample, then dz1 and W1's gradient
+        f32x4 dh[4];
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) dh[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int nt = 0; nt < 4; ++nt) {
+                    const uint32_t w = i < 2 ? wb[nt][mt].x : wb[nt][mt].y;
+                    const float wf = (i & 1) ? __uint_as_float(w & 0xffff0000u) : bf2f(w);
+                    dh[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(dz2[mt][i], wf, dh[nt], 0, 0, 0);
+                }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt)
+                G.w1[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xs[r], __fmul_rn(dh[nt][r], d1[nt][r]), G.w1[nt], 0, 0, 0);
         if (g == 0) {
-#pragma unroll
-            for (int i = 0; i < NF; ++i) S.x[sl][i] = x[i];
-            S.dy[sl] = dy;
-            gl = __fadd_rn(gl, __fmul_rn(r, r));
+            G.loss = fmaf(res, res, G.loss);
+            G.b3 = __fadd_rn(G.b3, dy);
         }
+    }
+    // the waves' sums, upper half onto lower half until one is left
+#pragma unroll 1
+    for (int half = TB_WAVES / 2; half >= 1; half >>= 1) {
+        if (wv >= half && wv < 2 * half)
+#pragma unroll
+            for (int i = 0; i < TB_VALUES; ++i) red[((wv - half) * TB_VALUES + i) * 64 + lane] = G.v[i];
         __syncthreads();
-        // dh1 = dz2 W2^T for the lane's units, then dz1
+        if (wv < half)
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int k = 32 * ks + 8 * g + j;
-                float dh = 0.f;
-                for (int o = 0; o < H; ++o) dh = __fadd_rn(dh, __fmul_rn(S.dz2[sl][o], w2f[k][o]));
-                S.dz1[sl][k] = __fmul_rn(dh, dsilu(F.z1[ks][j]));
-            }
-        __syncthreads();
-        // lane l owns row l of W2 (input unit l), column l of W1, and index l
-        // of b1, b2, w3
-        for (int s2 = 0; s2 < 16; ++s2) {
-            const float h1s = S.h1[s2][lane];
-#pragma unroll
-            for (int o = 0; o < H; ++o) gW2[o] = __fadd_rn(gW2[o], __fmul_rn(h1s, S.dz2[s2][o]));
-            const float d1 = S.dz1[s2][lane];
-#pragma unroll
-            for (int i = 0; i < NF; ++i) gW1[i] = __fadd_rn(gW1[i], __fmul_rn(S.x[s2][i], d1));
-            gb1 = __fadd_rn(gb1, d1);
-            gb2 = __fadd_rn(gb2, S.dz2[s2][lane]);
-            gw3 = __fadd_rn(gw3, __fmul_rn(S.h2[s2][lane], S.dy[s2]));
-            gb3 = __fadd_rn(gb3, S.dy[s2]);
-        }
+            for (int i = 0; i < TB_VALUES; ++i) G.v[i] = __fadd_rn(G.v[i], red[(wv * TB_VALUES + i) * 64 + lane]);
         __syncthreads();
     }
-    // loss partial: lanes 0..15 hold one sample each
-    float l1 = gl;
+    if (wv != 0) return;
+    float *P = partial + (size_t)blockIdx.x * SLOT;
 #pragma unroll
-    for (int m = 8; m >= 1; m >>= 1) l1 = __fadd_rn(l1, __shfl_xor(l1, m));
-    float *P = partial + (size_t)wave * SLOT;
+    for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-    for (int i = 0; i < NF; ++i) P[O_W1 + i * H + lane] = gW1[i];
-    P[O_B1 + lane] = gb1;
+        for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-    for (int o = 0; o < H; ++o) P[O_W2 + lane * H + o] = gW2[o];
-    P[O_B2 + lane] = gb2;
-    P[O_W3 + lane] = gw3;
+            for (int r = 0; r < 4; ++r) P[O_W2 + (16 * mt + 4 * g + r) * H + 16 * nt + j] = G.w2[mt][nt][r];
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+        const int u = 16 * nt + j;
+        if (g < 2)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) P[O_W1 + (4 * g + r) * H + u] = G.w1[nt][r];
+        if (g == 2) P[O_B1 + u] = G.w1[nt][0];
+        float b2 = __fadd_rn(G.b2[nt], __shfl_xor(G.b2[nt], 16)), w3 = __fadd_rn(G.w3[nt], __shfl_xor(G.w3[nt], 16));
+        b2 = __fadd_rn(b2, __shfl_xor(b2, 32));
+        w3 = __fadd_rn(w3, __shfl_xor(w3, 32));
+        if (g == 0) {
+            P[O_B2 + u] = b2;
+            P[O_W3 + u] = w3;
+        }
+    }
+    // lanes 0..15 hold one sample's share each, the others 0
+    float gb3 = G.b3, gl = G.loss;
+#pragma unroll
+    for (int m = 8; m >= 1; m >>= 1) {
+        gb3 = __fadd_rn(gb3, __shfl_xor(gb3, m));
+        gl = __fadd_rn(gl, __shfl_xor(gl, m));
+    }
     if (lane == 0) {
         P[O_B3] = gb3;
-        P[NPARAM] = l1;
+        P[NPARAM] = gl;
     }
 }
 
-__global__ void k_reduce_slots(const float *__restrict__ partial, int64_t nslots, float *__restrict__ out)
+// out[p] = sum of the slots' values p: wave w of a workgroup adds slots w, w
+// + RED_WAVES, .. for 64 parameters, then the waves' sums in order
+constexpr int RED_WAVES = 16;
+__global__ void __launch_bounds__(64 * RED_WAVES) k_reduce_slots(const float *__restrict__ partial, int nslots,
+                                                                 float *__restrict__ out)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= SLOT) return;
+    __shared__ float sums[RED_WAVES][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int p = blockIdx.x * 64 + lane;
     float a = 0.f;
-    for (int64_t w = 0; w < nslots; ++w) a = __fadd_rn(a, partial[(size_t)w * SLOT + p]);
+    if (p < SLOT)
+#pragma unroll 4
+        for (int w = wv; w < nslots; w += RED_WAVES) a = __fadd_rn(a, partial[(size_t)w * SLOT + p]);
+    sums[wv][lane] = a;
+    __syncthreads();
+    if (wv != 0 || p >= SLOT) return;
+#pragma unroll
+    for (int w = 1; w < RED_WAVES; ++w) a = __fadd_rn(a, sums[w][lane]);
     out[p] = a;
 }
 
@@ -1346,22 +1366,20 @@ static fr_status mlp_backward(fr_mlp *m, const float *feat_dev, const float *tar
     fr_ctx *ctx = m->ctx;
     FR_CHECK(ctx, B > 0 && feat_dev && targ_dev, FR_ERR_INVALID, "empty training batch");
     const int64_t groups = (B + 15) / 16;
-    const int64_t maxw = (int64_t)std::max(ctx->cu_count, 1) * 4;
-    const int64_t blocks = std::max<int64_t>(1, std::min<int64_t>((groups + TB_WAVES - 1) / TB_WAVES, maxw));
-    const int64_t nwaves = blocks * TB_WAVES;
-    const int iters = (int)((groups + nwaves - 1) / nwaves);
-    if (nwaves > m->partial_slots) {
+    const int64_t blocks = std::min<int64_t>((groups + TB_WAVES - 1) / TB_WAVES, std::max(ctx->cu_count, 1));
+    if (blocks > m->partial_slots) {
         FR_HIP(ctx, hipStreamSynchronize(ctx->stream));
         hipFree(m->partial);
         m->partial = nullptr;
         m->partial_slots = 0;
-        fr_status st = fr_alloc(ctx, (void **)&m->partial, (size_t)nwaves * SLOT * 4);
+        fr_status st = fr_alloc(ctx, (void **)&m->partial, (size_t)blocks * SLOT * 4);
         if (st) return st;
-        m->partial_slots = nwaves;
+        m->partial_slots = blocks;
     }
     hipLaunchKernelGGL(k_mlp_backward, dim3((unsigned)blocks), dim3(64 * TB_WAVES), 0, ctx->stream, view(m), feat_dev,
-                       targ_dev, idx_dev, B, iters, m->partial);
-    hipLaunchKernelGGL(k_reduce_slots, dim3(nblk(SLOT, 256)), dim3(256), 0, ctx->stream, m->partial, nwaves, m->grad);
+                       targ_dev, idx_dev, B, m->partial);
+    hipLaunchKernelGGL(k_reduce_slots, dim3(nblk(SLOT, 64)), dim3(64 * RED_WAVES), 0, ctx->stream, m->partial,
+                       (int)blocks, m->grad);
     FR_HIP(ctx, hipGetLastError());
     return FR_OK;
 }

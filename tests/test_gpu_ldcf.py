@@ -157,6 +157,26 @@ def test_gradient_matches_oracle_and_is_deterministic(ctx):
     assert np.array_equal(gi, gs) and li == ls
 
 
+@pytest.mark.parametrize("B", [1, 15, 16, 17, 64, 65, 4 * 16 * 256, 4 * 16 * 256 + 33, 50001])
+def test_gradient_at_group_and_workgroup_edges(ctx, B):
+    """Batches below, at and past one 16-sample group, one workgroup's four
+    waves and one group per wave of the whole launch, through an index array
+    of half the table's rows.  Bar: the BF16-rounded hidden layer, as in
+    test_gradient_matches_oracle_and_is_deterministic."""
+    rng = np.random.default_rng(B)
+    X = rng.uniform(-1.5, 1.5, (2 * B, 8)).astype(np.float32)
+    t = rng.standard_normal(2 * B).astype(np.float32)
+    idx = rng.permutation(2 * B)[:B].astype(np.int64)
+    p = random_net(B)
+    net = hip.MLP(ctx)
+    net.set_params(p, 0.0, 1.0)
+    got, loss = net.grad(upload(ctx, X), upload(ctx, t), B, idx=upload(ctx, idx))
+    Lr, gr = lo.loss_grad(p, X[idx], t[idx], emulate=True)
+    e = np.linalg.norm(got - gr) / np.linalg.norm(gr)
+    print(f"[mlp grad B={B}] loss {loss:.6f} vs {Lr:.6f}, grad rel-L2 {e:.2e}", flush=True)
+    assert abs(loss - Lr) <= 1e-4 * abs(Lr) and e <= 1e-3
+
+
 def test_training_reduces_loss(ctx):
     """A smooth target of the features is learned on the device."""
     rng = np.random.default_rng(5)

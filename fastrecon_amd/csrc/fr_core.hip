@@ -279,6 +279,7 @@ extern "C" fr_status fr_samples_set_traj(fr_samples *s, const float *traj, int s
     hipFree(tmp);
     FR_CHECK(ctx, e == hipSuccess, FR_ERR_HIP, "set_traj: %s", hipGetErrorString(e));
     s->has_traj = true;
+    ++s->traj_version;
     return FR_OK;
 }
 
@@ -322,6 +323,7 @@ extern "C" fr_status fr_samples_set_traj_device(fr_samples *s, const float *traj
                        traj, stride, s->dim, s->M, s->traj);
     FR_HIP(ctx, hipGetLastError());
     s->has_traj = true;
+    ++s->traj_version;
     return FR_OK;
 }
 

@@ -316,6 +316,11 @@ __global__ void k_scale_by_pos(float *__restrict__ w, float4 *__restrict__ pos, 
     pos[i].w = v;
 }
 
+// Sample-coils from which a plan's first degridding pays for the tile order:
+// acquisition order costs about 0.16 ns (2D: 0.07) each, building the order
+// 0.7 ms at 1.6M samples and 0.3 ms at 0.2M, mostly allocations.
+constexpr int64_t DEGRID_TILES = int64_t(1) << 23;
+
 }  // namespace
 
 fr_status fr_degrid_raw(fr_plan *p, const fr_samples *s, const float2 *grid, int C, float2 *out)
@@ -344,6 +349,22 @@ extern "C" fr_status fr_degrid_execute(fr_plan *p, const fr_samples *s, const fr
     FR_CHECK(ctx, g->dim == p->dim && g->N == p->N && g->frames == p->frames && s->frames == p->frames,
              FR_ERR_INVALID, "grids do not match the plan");
     FR_EXTENT(ctx, out_dev, sizeof(float2) * (size_t)s->M * g->C, "fr_degrid_execute output");
+    // The samples' tile order, once the plan has it; it is built where one
+    // call in acquisition order would cost more than that (a few launches
+    // and allocations), and not while the stream is being captured.
+    if (fr_tiles_fit(p, s)) {
+        bool build = !p->tord && s->M * g->C >= DEGRID_TILES;
+        if (build) {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            FR_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
+            build = cs == hipStreamCaptureStatusNone;
+        }
+        if (build) {
+            fr_status e = fr_tiles_build(p);
+            if (e) return e;
+        }
+        if (p->tord) return fr_tile_degrid(p, g->data, g->C, (float2 *)out_dev);
+    }
     return fr_degrid_raw(p, s, g->data, g->C, (float2 *)out_dev);
 }
 
@@ -413,7 +434,17 @@ extern "C" fr_status fr_dcf_pipe_menon(fr_plan *p, fr_samples *s, int iters, int
     FR_CHECK(ctx, iters >= 0, FR_ERR_INVALID, "iters must be >= 0");
     FR_CHECK(ctx, s->frames == p->frames, FR_ERR_INVALID, "samples and plan differ in frames");
     const int64_t M = s->M;
-    fr_status st = dcf_workspace(p, s);
+    fr_status st = FR_OK;
+    if (fr_tiles_fit(p, s)) {
+        st = fr_tile_density(p, s, iters, init_ones || !s->has_dcf);
+        if (st) return st;
+        s->has_dcf = true;
+        fr_dcf_changed(s);
+        hipError_t e = hipStreamSynchronize(ctx->stream);
+        FR_CHECK(ctx, e == hipSuccess, FR_ERR_HIP, "pipe-menon: %s", hipGetErrorString(e));
+        return FR_OK;
+    }
+    st = dcf_workspace(p, s);
     if (st) return st;
     fr_samples *u = p->dcf_u;
     if (init_ones || !s->has_dcf)

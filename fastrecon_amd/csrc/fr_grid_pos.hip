@@ -44,6 +44,7 @@
 // of a group, and holds component slice l % 16: with NCB component blocks,
 // components [NCB j, NCB j + NCB) of a chunk of 8 NCB coils.
 #include "fr_internal.h"
+#include "fr_taps.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -135,12 +136,7 @@ __device__ __forceinline__ float tap_weight(const float4 &p, const float4 *stbl,
     const float dz = __fsub_rn(fz, p.z);
     const float dy = __fsub_rn(fy, p.y);
     const float dx = __fsub_rn(fx, p.x);
-    const float d2 = __fadd_rn(__fadd_rn(__fmul_rn(dz, dz), __fmul_rn(dy, dy)), __fmul_rn(dx, dx));
-    // index estimate from the 1-ulp square root, then the exact selection
-    const float est = fminf(__builtin_fmaf(__builtin_amdgcn_sqrtf(d2), cidx, 0.49f), lmax);
-    const float4 e = stbl[(int)est];
-    const float wsel = d2 >= e.x ? e.z : e.y;
-    return d2 < dacc ? wsel : 0.f;                    // tap test sqrtf(d2) < hw (GridLut.cpp:133)
+    return fr_tap_weight(fr_tap_dk2(__fmul_rn(dz, dz), __fmul_rn(dy, dy), dx), stbl, dacc, cidx, lmax);
 }
 
 // B = dcf * sample (GridLut.cpp:109); padding coil columns get 0

@@ -42,6 +42,7 @@ struct fr_samples {
     // its positions and refreshes it only when these differ from its copy's
     uint64_t uid = 0;
     uint64_t dcf_version = 0;
+    uint64_t traj_version = 0;     // bumped on every change of traj
 };
 
 uint64_t fr_next_uid();
@@ -142,8 +143,31 @@ struct fr_heavy {
     uint32_t pad;
 };
 
+// A slice of a tile's samples in tile order (fr_tile.hip): samples [s0, s0 +
+// n); tile = the tile count for samples that reach no cell.
+struct fr_titem {
+    uint32_t tile, s0, n, pad;
+};
+
+// A plan's samples in tile order, and the density iterations' buffers (made
+// on their first call; kept until the plan is destroyed).
+struct fr_tiles {
+    float4 *tpos = nullptr;        // M: x, y, z (or frame), the sample's index
+    fr_titem *items = nullptr;     // nitems, by tile
+    uint32_t nitems = 0;
+    uint32_t *first = nullptr;     // first item of each tile
+    uint32_t *many = nullptr;      // tiles with several items
+    uint32_t nmany = 0;
+    float *w = nullptr;            // M densities in tile order
+    float *part = nullptr;         // one region of sums per item
+    float *grid = nullptr;         // the real grid
+};
+
 struct fr_plan {
     fr_ctx *ctx = nullptr;
+    // the trajectory the plan was built on (fr_samples uid and version)
+    uint64_t traj_uid = 0, traj_version = 0;
+    fr_tiles *tord = nullptr;       // position-weight plans: built on first use
     // single-channel workspace of Pipe-Menon and the identity scale (unit
     // data on the plan's trajectory, a one-channel grid, degridded
     // densities): created on first use, kept until the plan is destroyed
@@ -294,6 +318,14 @@ fr_status fr_launch_grid_pos(fr_plan *p, const fr_samples *s, float2 *out, float
 // bytes of heavy-unit slice partials a pass of C coils needs
 size_t fr_grid_scratch_bytes(const fr_plan *p, int C);
 fr_status fr_grid_check(const fr_plan *p, const fr_samples *s, const fr_grids *out);
+// samples in tile order (fr_tile.hip): whether the plan has such an order for
+// the handle's trajectory; the order itself; degridding and the density
+// iterations on it
+bool fr_tiles_fit(const fr_plan *p, const fr_samples *s);
+fr_status fr_tiles_build(fr_plan *p);
+void fr_tiles_free(fr_tiles *t);
+fr_status fr_tile_degrid(const fr_plan *p, const float2 *grid, int C, float2 *out);
+fr_status fr_tile_density(fr_plan *p, fr_samples *s, int iters, bool ones);
 // the no-allocation entry point's static scratch (fr_noalloc.hip): its
 // address on the context's device, looked up once per device
 fr_status fr_scratch_init(fr_ctx *ctx);

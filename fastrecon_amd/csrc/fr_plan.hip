@@ -919,6 +919,7 @@ extern "C" fr_status fr_plan_create(fr_ctx *ctx, const fr_samples *s, unsigned N
     if (!p) return FR_ERR_NOMEM;
     p->ctx = ctx; p->dim = s->dim; p->N = N; p->M = s->M; p->frames = s->frames;
     p->kWidth = kWidth; p->kHW = kWidth / 2.0f; p->L = L;     // GridLut.cpp:86
+    p->traj_uid = s->uid; p->traj_version = s->traj_version;
     p->host_lut.assign(lut, lut + L);
     fr_status e = fr_alloc(ctx, (void **)&p->lut, sizeof(float) * L);
     if (!e) {
@@ -940,6 +941,7 @@ extern "C" fr_status fr_plan_destroy(fr_plan *p)
     hipFree(p->recs); hipFree(p->pos); hipFree(p->tsel); hipFree(p->tiles);
     hipFree(p->dcf_den);
     hipFree(p->dcf_scr);
+    fr_tiles_free(p->tord);
     fr_grids_destroy(p->dcf_g);
     fr_samples_destroy(p->dcf_u);
     delete p;

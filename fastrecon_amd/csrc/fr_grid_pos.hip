@@ -56,9 +56,9 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 constexpr int RB = 16;               // records per batch: four groups of four
 constexpr int PW = FR_POS_WAVES;     // waves per workgroup
 constexpr int CS = 17;               // LDS row stride of the write-out transpose (16 cells + 1)
-// the pipeline reads record indices up to 3 RB - 1 past a live record; the
-// plan pads the record array by 64 entries
-static_assert(3 * RB - 1 < 64, "record padding");
+constexpr int PS = 68;               // and of a pair's (32 cells of a coil, + 16 bytes)
+// the pipeline reads record indices up to 191 past a batch's first
+static_assert(3 * 64 <= FR_POS_PAD, "record padding");
 
 __device__ __forceinline__ void wave_sync()
 {
@@ -89,40 +89,44 @@ __device__ __forceinline__ E ld_off(const E *__restrict__ base, uint32_t byte_of
     return *reinterpret_cast<const E *>(reinterpret_cast<const char *>(base) + byte_off);
 }
 
-// One batch of RB records in flight: lane (j, k) holds group q's record
-// 4 q + k: its position, DCF and the lane's component slice of its row.
-struct batch_st {
-    float4 p[4];
-    float w[4];
+// The rows of one batch of RB records in flight: lane (j, k) holds its
+// component slice of group q's record 4 q + k.
+struct batch_rows {
     float2 a[4], b[4];
 };
 
-__device__ __forceinline__ void load_ids(uint32_t (&id)[4], const uint32_t *__restrict__ recs, uint32_t rb, int k)
-{
-#pragma unroll
-    for (int q = 0; q < 4; ++q) id[q] = ld_off(recs, (rb + 4 * q + k) * (uint32_t)sizeof(uint32_t));
-}
-
-// The position entry carries the sample's DCF in .w (refreshed from the
-// samples before every pass), so a record costs one 16-byte gather for
-// position and weight.
-template <int NCB, bool PAIR, typename TS>
-__device__ __forceinline__ void issue_batch(batch_st &S, const uint32_t (&id)[4], const float4 *__restrict__ pos,
-                                            const TS *__restrict__ data, uint32_t C, int ca, int cbb)
+// Rows of the batch whose samples lanes 16 s .. 16 s + 15 hold: in `at`, the
+// byte offset of a sample's row (SMALL: the data is below 4 GiB; one 32-bit
+// addition per load in place of a 64-bit product and sum) or its index.
+template <int NCB, bool PAIR, bool SMALL, typename TS>
+__device__ __forceinline__ void issue_rows(batch_rows &S, uint32_t at, int s, const TS *__restrict__ data, uint32_t C,
+                                           int ca, int cbb, int k)
 {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const uint32_t s = id[q];
-        S.p[q] = ld_off(pos, s * (uint32_t)sizeof(float4));
-        S.w[q] = S.p[q].w;
-        const TS *row = data + (uint64_t)s * C;
-        if constexpr (NCB == 4 && PAIR) {
-            const float4 v = ld_pair(row, ca);
-            S.a[q] = make_float2(v.x, v.y);
-            S.b[q] = make_float2(v.z, v.w);
+        const uint32_t m = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (16 * s + 4 * q + k), (int)at);
+        if constexpr (SMALL) {
+            const uint32_t o = m + (uint32_t)(ca * (int)sizeof(TS));
+            if constexpr (NCB == 4 && PAIR) {
+                const float4 v = ld_pair(reinterpret_cast<const TS *>(reinterpret_cast<const char *>(data) + o), 0);
+                S.a[q] = make_float2(v.x, v.y);
+                S.b[q] = make_float2(v.z, v.w);
+            } else {
+                S.a[q] = ld_coil(reinterpret_cast<const TS *>(reinterpret_cast<const char *>(data) + o), 0);
+                if constexpr (NCB == 4)
+                    S.b[q] = ld_coil(reinterpret_cast<const TS *>(reinterpret_cast<const char *>(data) +
+                                                                  (m + (uint32_t)(cbb * (int)sizeof(TS)))), 0);
+            }
         } else {
-            S.a[q] = ld_coil(row, ca);
-            if constexpr (NCB == 4) S.b[q] = ld_coil(row, cbb);
+            const TS *row = data + (uint64_t)m * C;
+            if constexpr (NCB == 4 && PAIR) {
+                const float4 v = ld_pair(row, ca);
+                S.a[q] = make_float2(v.x, v.y);
+                S.b[q] = make_float2(v.z, v.w);
+            } else {
+                S.a[q] = ld_coil(row, ca);
+                if constexpr (NCB == 4) S.b[q] = ld_coil(row, cbb);
+            }
         }
     }
 }
@@ -130,48 +134,50 @@ __device__ __forceinline__ void issue_batch(batch_st &S, const uint32_t (&id)[4]
 // Weight of the lane's cell for a sample at p: the reference tap test and
 // LUT index through the selection table (file comment).
 __device__ __forceinline__ float tap_weight(const float4 &p, const float4 *stbl, float fx, float fy, float fz,
-                                            float dacc, float cidx, float lmax)
+                                            float cidx, float lmax)
 {
     // d2 with the reference's operations and order (GridLut.cpp:120-131)
     const float dz = __fsub_rn(fz, p.z);
     const float dy = __fsub_rn(fy, p.y);
     const float dx = __fsub_rn(fx, p.x);
-    return fr_tap_weight(fr_tap_dk2(__fmul_rn(dz, dz), __fmul_rn(dy, dy), dx), stbl, dacc, cidx, lmax);
+    return fr_tap_weight(fr_tap_dk2(__fmul_rn(dz, dz), __fmul_rn(dy, dy), dx), stbl, cidx, lmax);
 }
 
-// B = dcf * sample (GridLut.cpp:109); padding coil columns get 0
-template <int NCB, bool FULL>
-__device__ __forceinline__ void b_values(float (&bv)[NCB], float w, float2 a, float2 b, bool v0ok, bool v1ok, int j)
+// B = dcf * sample (GridLut.cpp:109).  Columns past the chunk's coils repeat
+// its last coil; their sums are not written.
+template <int NCB>
+__device__ __forceinline__ void b_values(float (&bv)[NCB], float w, float2 a, float2 b, int j)
 {
-    const float w0 = FULL || v0ok ? w : 0.f;
     if constexpr (NCB == 4) {
-        const float w1 = FULL || v1ok ? w : 0.f;
-        bv[0] = __fmul_rn(w0, a.x); bv[1] = __fmul_rn(w0, a.y);
-        bv[2] = __fmul_rn(w1, b.x); bv[3] = __fmul_rn(w1, b.y);
+        bv[0] = __fmul_rn(w, a.x); bv[1] = __fmul_rn(w, a.y);
+        bv[2] = __fmul_rn(w, b.x); bv[3] = __fmul_rn(w, b.y);
     } else if constexpr (NCB == 2) {
-        bv[0] = __fmul_rn(w0, a.x); bv[1] = __fmul_rn(w0, a.y);
+        bv[0] = __fmul_rn(w, a.x); bv[1] = __fmul_rn(w, a.y);
     } else {
-        bv[0] = __fmul_rn(w0, (j & 1) ? a.y : a.x);
+        bv[0] = __fmul_rn(w, (j & 1) ? a.y : a.x);
     }
 }
 
-// Apply the four groups of one batch.  The null sample (index M) sits
-// far outside the grid with DCF 0 and a zero row, so padding records add
-// exact zeros.  The four weight computations are independent (their table
-// reads overlap); the matrix instructions then cycle through the NCB
-// accumulators.
-template <int NCB, bool FULL>
-__device__ __forceinline__ void apply_batch(f4 (&acc)[NCB], const batch_st &S, const float4 *stbl, float fx,
-                                            float fy, float fz, float dacc, float cidx, float lmax, bool v0ok,
-                                            bool v1ok, int j)
+// Apply the four groups of one batch, its positions and DCFs in pb[0 .. 15].
+// The null sample (index M) sits far outside the grid with DCF 0 and a zero
+// row, so padding records add exact zeros.  The four weight computations are
+// independent (their table reads overlap); the matrix instructions then cycle
+// through the NCB accumulators.
+template <int NCB>
+__device__ __forceinline__ void apply_batch(f4 (&acc)[NCB], const batch_rows &S, const float4 *pb, const float4 *stbl,
+                                            float fx, float fy, float fz, float cidx, float lmax, int j, int k)
 {
-    float aw[4];
+    float aw[4], w[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) aw[q] = tap_weight(S.p[q], stbl, fx, fy, fz, dacc, cidx, lmax);
+    for (int q = 0; q < 4; ++q) {
+        const float4 p = pb[4 * q + k];
+        w[q] = p.w;
+        aw[q] = tap_weight(p, stbl, fx, fy, fz, cidx, lmax);
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         float bv[NCB];
-        b_values<NCB, FULL>(bv, S.w[q], S.a[q], S.b[q], v0ok, v1ok, j);
+        b_values<NCB>(bv, w[q], S.a[q], S.b[q], j);
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(aw[q], bv[cb], acc[cb], 0, 0, 0);
     }
@@ -207,75 +213,95 @@ __device__ __forceinline__ void lane_cell(const item_box &b, int j, float &fx, f
     }
 }
 
-// Grid the records [r, r1) of one item into acc: software pipeline over
-// batches of RB records -- while batch b is applied, batch b+1's positions,
-// DCFs and rows and batch b+2's sample indices are in flight (past r1 they
-// read the next records or the 64 padding records at the end).
-template <int NCB, bool PAIR, bool FULL, typename TS>
+// Grid the records [r, ..) into acc, batch by batch, until after_batch(r),
+// called with the position past the batch just applied, returns false.
+//
+// Records come in blocks of 64, one per lane: one load brings a block's
+// sample indices and one its positions and DCFs, which go through LDS (pbuf,
+// two blocks) to the 16 lanes that need each; the indices reach the lanes
+// that load a record's row by a lane exchange.  (Loaded where they are used,
+// each by 16 lanes, positions and indices took 16 times the load
+// instructions and return traffic of these.)  Software pipeline: while batch
+// b is applied, batch b + 1's rows, the next block's positions and the block
+// after's indices are in flight (past the last record they read the next
+// records or the FR_POS_PAD padding records at the end).  Bound by VALU issue
+// (about 27 instructions per four records beside the matrix ones: VALU busy
+// 60% and matrix cores 31% at 16 FP16 coils on 384^3) and, at 32 coils, by
+// the traffic of the rows past L2 as well.  32 coils at 256^3: 4.71 -> 4.13 ms
+// in all; 16 FP16 coils at 384^3: 7.75 -> 7.12.  Rows fetched two or three
+// batches ahead were slower (the extra ones past an item's end cost as much
+// as useful ones): 8.1 and 8.5 ms there.
+template <int NCB, bool PAIR, bool SMALL, typename TS, typename After>
+__device__ __forceinline__ void grid_stream(f4 (&acc)[NCB], uint32_t r, const uint32_t *__restrict__ recs,
+                                            const float4 *__restrict__ pos, const TS *__restrict__ data, uint32_t C,
+                                            int ca, int cbb, const float4 *stbl, float4 *pbuf, float &fx, float &fy,
+                                            float &fz, float cidx, float lmax, int j,
+                                            int k, After after_batch)
+{
+    const uint32_t lane = (uint32_t)(16 * k + j);
+    const uint32_t id = ld_off(recs, (r + lane) * 4u);
+    uint32_t id1 = ld_off(recs, (r + 64 + lane) * 4u);
+    float4 P = ld_off(pos, id * 16u);
+    batch_rows S0, S1;
+    auto row_at = [&](uint32_t m) __attribute__((always_inline)) { return SMALL ? m * (C * (uint32_t)sizeof(TS)) : m; };
+    uint32_t at = row_at(id);
+    issue_rows<NCB, PAIR, SMALL>(S0, at, 0, data, C, ca, cbb, k);
+    auto apply = [&](const batch_rows &S, int s) __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        apply_batch<NCB>(acc, S, pbuf + 16 * s, stbl, fx, fy, fz, cidx, lmax, j, k);
+        r += RB;
+    };
+    while (true) {
+        wave_sync();                       // the block before is no longer read
+        pbuf[lane] = P;
+        P = ld_off(pos, id1 * 16u);
+        const uint32_t at1 = row_at(id1);
+        const uint32_t id2 = ld_off(recs, (r + 128 + lane) * 4u);
+        wave_sync();
+#pragma unroll 1
+        for (int q = 0; q < 4; q += 2) {
+            issue_rows<NCB, PAIR, SMALL>(S1, at, q + 1, data, C, ca, cbb, k);
+            apply(S0, q);
+            if (!after_batch(r)) return;
+            issue_rows<NCB, PAIR, SMALL>(S0, q == 0 ? at : at1, (q + 2) & 3, data, C, ca, cbb, k);
+            apply(S1, q + 1);
+            if (!after_batch(r)) return;
+        }
+        at = at1;
+        id1 = id2;
+    }
+}
+
+template <int NCB, bool PAIR, bool SMALL, typename TS>
 __device__ __forceinline__ void grid_records(f4 (&acc)[NCB], uint32_t r, uint32_t r1,
                                              const uint32_t *__restrict__ recs, const float4 *__restrict__ pos,
-                                             const TS *__restrict__ data, uint32_t C,
-                                             int ca, int cbb, const float4 *stbl, float fx, float fy, float fz,
-                                             float dacc, float cidx, float lmax, bool v0ok, bool v1ok, int j, int k)
+                                             const TS *__restrict__ data, uint32_t C, int ca, int cbb,
+                                             const float4 *stbl, float4 *pbuf, float fx, float fy, float fz,
+                                             float cidx, float lmax, int j, int k)
 {
-    uint32_t id0[4], id1[4];
-    batch_st S0, S1;
-    load_ids(id0, recs, r, k);
-    load_ids(id1, recs, r + RB, k);
-    issue_batch<NCB, PAIR>(S0, id0, pos, data, C, ca, cbb);
-    while (true) {
-        load_ids(id0, recs, r + 2 * RB, k);
-        issue_batch<NCB, PAIR>(S1, id1, pos, data, C, ca, cbb);
-        __builtin_amdgcn_sched_barrier(0);
-        apply_batch<NCB, FULL>(acc, S0, stbl, fx, fy, fz, dacc, cidx, lmax, v0ok, v1ok, j);
-        r += RB;
-        if (r >= r1) break;
-        load_ids(id1, recs, r + 2 * RB, k);
-        issue_batch<NCB, PAIR>(S0, id0, pos, data, C, ca, cbb);
-        __builtin_amdgcn_sched_barrier(0);
-        apply_batch<NCB, FULL>(acc, S1, stbl, fx, fy, fz, dacc, cidx, lmax, v0ok, v1ok, j);
-        r += RB;
-        if (r >= r1) break;
-    }
+    grid_stream<NCB, PAIR, SMALL>(acc, r, recs, pos, data, C, ca, cbb, stbl, pbuf, fx, fy, fz, cidx, lmax, j, k, [&](uint32_t q) __attribute__((always_inline)) { return q < r1; });
 }
 
 // grid_records over [r, r1) with a switch at rmid (a multiple of RB): the
 // records up to rmid belong to one unit, the rest to the next; at rmid the
 // pipeline keeps running and on_mid() moves the lane to the next unit's
 // cell (fx, fy, fz) and accumulators.
-template <int NCB, bool PAIR, bool FULL, typename TS, typename Mid>
+template <int NCB, bool PAIR, bool SMALL, typename TS, typename Mid>
 __device__ __forceinline__ void grid_records_mid(f4 (&acc)[NCB], uint32_t r, uint32_t rmid, uint32_t r1,
                                                  const uint32_t *__restrict__ recs, const float4 *__restrict__ pos,
                                                  const TS *__restrict__ data, uint32_t C, int ca, int cbb,
-                                                 const float4 *stbl, float &fx, float &fy, float &fz, float dacc,
-                                                 float cidx, float lmax, bool v0ok, bool v1ok, int j, int k, Mid on_mid)
+                                                 const float4 *stbl, float4 *pbuf, float &fx, float &fy, float &fz,
+                                                 float cidx, float lmax, int j, int k, Mid on_mid)
 {
-    uint32_t id0[4], id1[4];
-    batch_st S0, S1;
-    load_ids(id0, recs, r, k);
-    load_ids(id1, recs, r + RB, k);
-    issue_batch<NCB, PAIR>(S0, id0, pos, data, C, ca, cbb);
-    while (true) {
-        load_ids(id0, recs, r + 2 * RB, k);
-        issue_batch<NCB, PAIR>(S1, id1, pos, data, C, ca, cbb);
-        __builtin_amdgcn_sched_barrier(0);
-        apply_batch<NCB, FULL>(acc, S0, stbl, fx, fy, fz, dacc, cidx, lmax, v0ok, v1ok, j);
-        r += RB;
-        if (r == rmid) on_mid();
-        if (r >= r1) break;
-        load_ids(id1, recs, r + 2 * RB, k);
-        issue_batch<NCB, PAIR>(S0, id0, pos, data, C, ca, cbb);
-        __builtin_amdgcn_sched_barrier(0);
-        apply_batch<NCB, FULL>(acc, S1, stbl, fx, fy, fz, dacc, cidx, lmax, v0ok, v1ok, j);
-        r += RB;
-        if (r == rmid) on_mid();
-        if (r >= r1) break;
-    }
+    grid_stream<NCB, PAIR, SMALL>(acc, r, recs, pos, data, C, ca, cbb, stbl, pbuf, fx, fy, fz, cidx, lmax, j, k, [&](uint32_t q) __attribute__((always_inline)) {
+                                     if (q == rmid) on_mid();
+                                     return q < r1;
+                                 });
 }
 
 // NCB component blocks (chunks of 8 NCB coils).  PAIR: C even, so lane j's
 // two coils (2j, 2j+1 of a 32-coil chunk) are one aligned 16-byte (8-byte
-// for FP16) load.  FULL: every chunk holds 8 NCB coils.
+// for FP16) load.
 //
 // Three kinds of workgroup:
 //  * front: one heavy-unit item per wave (a whole unit, or a slice written
@@ -285,11 +311,11 @@ __device__ __forceinline__ void grid_records_mid(f4 (&acc)[NCB], uint32_t r, uin
 //    rows of PW * bx cells (128 bytes for 4-cell-wide units);
 //  * otherwise a run of ipw consecutive light items per wave, as one
 //    record stream, each unit written out by its wave.
-template <int NCB, bool PAIR, bool FULL, typename TS, int OCC>
+template <int NCB, bool PAIR, bool SMALL, typename TS, int OCC>
 __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OCC, 8))) k_grid_pos(
     const fr_item *__restrict__ items, int64_t nitems, const fr_tile *__restrict__ tiles, int64_t ntiles,
     int lbx, int lby, int lbz, const uint32_t *__restrict__ recs, const float4 *__restrict__ pos,
-    const float4 *__restrict__ tbl, int L, float dacc, float cidx, const TS *__restrict__ data,
+    const float4 *__restrict__ tbl, int L, float cidx, const TS *__restrict__ data,
     int C, int N, size_t cells, float2 *__restrict__ out, float2 *__restrict__ partial,
     int64_t nslots, int cells_max, int64_t nfront, int64_t front_wg, int ipw, int64_t xr, int nt, int tw,
     int osm_floats, int64_t tstride, int fsub)
@@ -298,7 +324,8 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
     float4 *stbl = smem_pos;                                         // L entries
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    float *osm = reinterpret_cast<float *>(smem_pos + L) + wv * osm_floats;
+    float4 *pbuf = smem_pos + L + wv * 64;                           // the wave's block of positions
+    float *osm = reinterpret_cast<float *>(smem_pos + L + PW * 64) + wv * osm_floats;
     for (int q = threadIdx.x; q < L; q += 64 * PW) stbl[q] = tbl[q];
     __syncthreads();
 
@@ -308,7 +335,6 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
     const int c0 = blockIdx.y * chunk;
     const int nc = min(chunk, C - c0);
     const int cl0 = NCB == 4 ? 2 * j : (NCB == 2 ? j : j >> 1);
-    const bool v0ok = cl0 < nc, v1ok = NCB == 4 && cl0 + 1 < nc;
     const int ca = PAIR ? c0 + min(cl0, nc - 2) : c0 + min(cl0, nc - 1), cbb = c0 + min(cl0 + 1, nc - 1);
     const float lmax = (float)(L - 1);
 
@@ -332,15 +358,15 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
         const int32_t myitem = wv == 0 ? T.item[0] : wv == 1 ? T.item[1] : wv == 2 ? T.item[2] : T.item[3];
         const int bx = 1 << lbx, by = 1 << lby;
         const int W = PW * bx, rows = by << lbz;    // tile row length, rows per coil
-        float *tb = reinterpret_cast<float *>(smem_pos + L);
+        float *tb = reinterpret_cast<float *>(smem_pos + L + PW * 64);
         const int cstride = rows * W * 2 + 4;       // floats per coil (+4: fewer bank conflicts)
         if (myitem >= 0) {
             const fr_item it = items[myitem];
             float fx, fy, fz;
             lane_cell(unpack_box(it.t0, it.pad), j, fx, fy, fz);
             if (it.r0 < it.r1)
-                grid_records<NCB, PAIR, FULL>(acc, it.r0, it.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, fx,
-                                              fy, fz, dacc, cidx, lmax, v0ok, v1ok, j, k);
+                grid_records<NCB, PAIR, SMALL>(acc, it.r0, it.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx,
+                                              fy, fz, cidx, lmax, j, k);
             // register r holds cell q = 4 k + r of the unit, component NCB j + cb
 #pragma unroll
             for (int cb = 0; cb < NCB; ++cb)
@@ -383,14 +409,14 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
     // transpose: register r holds cell 4 k + r, component NCB j + cb (coil
     // c: re 2c, im 2c + 1); consecutive lanes then store consecutive cells
     // of one coil.
-    auto write_out = [&](const fr_item &it, const item_box &b) {
+    auto write_out = [&](const fr_item &it, const item_box &b) __attribute__((always_inline)) {
         wave_sync();
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb)
 #pragma unroll
             for (int r = 0; r < 4; ++r) osm[(NCB * j + cb) * CS + 4 * k + r] = acc[cb][r];
         wave_sync();
-        auto put = [&](int cl, int q, size_t go) {
+        auto put = [&](int cl, int q, size_t go) __attribute__((always_inline)) {
             const float2 v = make_float2(osm[(2 * cl) * CS + q], osm[(2 * cl + 1) * CS + q]);
             const int c = c0 + cl;
             if (it.slot < 0) {
@@ -426,12 +452,13 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
     };
 
     // ----------------------------------------------------------- pairs
-    // One wave grids the two x-adjacent units of a pair one after the other
-    // (the first unit's sums held in registers) and writes them out
-    // together: rows of 2 bx cells (64 bytes for 4-cell-wide units) instead
-    // of bx.  Components go through the LDS transpose in steps of 16 coils
-    // (8 when a chunk has 8): region cell x + 2 bx (y + by z) of the pair's
-    // 2 bx x by x bz box, unit A at x < bx, unit B at x >= bx.
+    // One wave grids the two x-adjacent units of a pair (boxes at least 4
+    // cells wide) one after the other, the first unit's sums held in
+    // registers, and writes them out together: rows of 2 bx cells (64 bytes
+    // for 4-cell-wide units) instead of bx.  (Stored straight from the
+    // accumulators, 16 bytes of a row at a time, 32 coils at 256^3 took 4.87
+    // ms against 4.31 with an LDS transpose by 4-byte words and 4.13 with this
+    // one by 16-byte words.)
     if (bid >= front_wg && ntiles > 0) {
         const int64_t pidx = fr_sampled_tile(grp * PW + wv, tstride);   // (tstride 1: every pair)
         if (pidx >= ntiles) return;
@@ -445,76 +472,73 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
             float fx, fy, fz;
             lane_cell(b, j, fx, fy, fz);
             if (it.r0 < it.r1)
-                grid_records<NCB, PAIR, FULL>(acc, it.r0, it.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, fx, fy,
-                                              fz, dacc, cidx, lmax, v0ok, v1ok, j, k);
+                grid_records<NCB, PAIR, SMALL>(acc, it.r0, it.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx, fy,
+                                              fz, cidx, lmax, j, k);
             write_out(it, b);
             return;
         }
-        constexpr int RS = 33;                        // LDS row: 32 region cells + 1
-        const int bxs = 1 << lbx, lb2 = lbx + 1;
-        constexpr int steps = NCB == 4 ? 2 : 1;
-        constexpr int ncs = NCB == 1 ? 8 : 16;        // coils per step
-        // lane (j, k): register r holds cell q = 4 k + r of a unit; unit A's
-        // cells go to region x < bx, B's to x >= bx
-        auto stage = [&](f4 a, int cb, int xoff) {
-            const int comp = NCB == 1 ? j : 2 * j + (cb & 1);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int q = 4 * k + r;
-                osm[comp * RS + (q & (bxs - 1)) + ((q >> lbx) << lb2) + xoff] = a[r];
-            }
-        };
         const fr_item ita = items[ia], itb = items[ib];
         const item_box ba = unpack_box(ita.t0, ita.pad), bb = unpack_box(itb.t0, itb.pad);
         float fx, fy, fz;
         lane_cell(ba, j, fx, fy, fz);
-        // at the end of A: all its component slices into the transpose
-        // buffer (step h at offset h 32 RS); then B's cell and fresh
-        // accumulators
-        auto to_b = [&]() {
-            wave_sync();
+        // at the end of A: its sums aside, B's cell and fresh accumulators
+        f4 acc_a[NCB];
+        auto to_b = [&]() __attribute__((always_inline)) {
 #pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) stage(acc[cb], cb, (cb >> 1) * 32 * RS);
-#pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) acc[cb] = f4{0.f, 0.f, 0.f, 0.f};
+            for (int cb = 0; cb < NCB; ++cb) {
+                acc_a[cb] = acc[cb];
+                acc[cb] = f4{0.f, 0.f, 0.f, 0.f};
+            }
             lane_cell(bb, j, fx, fy, fz);
         };
         if (ita.r0 < ita.r1 && itb.r0 < itb.r1 && itb.r0 == ita.r1) {
             // A's and B's records are consecutive: one pipelined stream
-            grid_records_mid<NCB, PAIR, FULL>(acc, ita.r0, ita.r1, itb.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl,
-                                              fx, fy, fz, dacc, cidx, lmax, v0ok, v1ok, j, k, to_b);
+            grid_records_mid<NCB, PAIR, SMALL>(acc, ita.r0, ita.r1, itb.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf,
+                                              fx, fy, fz, cidx, lmax, j, k, to_b);
         } else {
             if (ita.r0 < ita.r1)
-                grid_records<NCB, PAIR, FULL>(acc, ita.r0, ita.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, fx,
-                                              fy, fz, dacc, cidx, lmax, v0ok, v1ok, j, k);
+                grid_records<NCB, PAIR, SMALL>(acc, ita.r0, ita.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx,
+                                              fy, fz, cidx, lmax, j, k);
             to_b();
             if (itb.r0 < itb.r1)
-                grid_records<NCB, PAIR, FULL>(acc, itb.r0, itb.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, fx,
-                                              fy, fz, dacc, cidx, lmax, v0ok, v1ok, j, k);
+                grid_records<NCB, PAIR, SMALL>(acc, itb.r0, itb.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx,
+                                              fy, fz, cidx, lmax, j, k);
         }
-        const int cell = lane & 31;
-        const int x = cell & ((2 << lbx) - 1), row = cell >> lb2;
+        // Lane (j, k) holds cells 4 k .. 4 k + 3 of both units, neighbours
+        // along x.  By way of LDS, [coil][cell of the pair's 2 bx x by x bz
+        // box][re, im], 16 coils a step, each lane then stores two
+        // neighbouring cells of a coil and 2 bx cells make one write.
+        const int px = (4 * k) & ((1 << lbx) - 1), prow = (4 * k) >> lbx;
+        const int cell = 2 * (lane & 15), x = cell & ((2 << lbx) - 1), row = cell >> (lbx + 1);
         const size_t go = ((size_t)(ba.oz + (row >> lby)) * N + (ba.oy + (row & ((1 << lby) - 1)))) * N + (ba.ox + x);
-        wave_sync();
-#pragma unroll
-        for (int cb = 0; cb < NCB; ++cb) stage(acc[cb], cb, (cb >> 1) * 32 * RS + bxs);
-        wave_sync();
+        constexpr int steps = NCB == 4 ? 2 : 1, ncs = NCB == 1 ? 8 : 16;
 #pragma unroll
         for (int h = 0; h < steps; ++h) {
-            const float *os = osm + h * 32 * RS;
+            wave_sync();
 #pragma unroll
-            for (int t = 0; t < ncs / 2; ++t) {
-                const int cs = (lane >> 5) + 2 * t;
-                const int cl = NCB == 4 ? 2 * cs + h : cs;
-                if (cl < nc) {
-                    const float2 v = make_float2(os[(2 * cs) * RS + cell], os[(2 * cs + 1) * RS + cell]);
-                    float2 *d = out + (size_t)(c0 + cl) * cells + go;
-                    if (nt)
-                        __builtin_nontemporal_store(__builtin_bit_cast(unsigned long long, v),
-                                                    reinterpret_cast<unsigned long long *>(d));
-                    else
-                        *d = v;
+            for (int u = 0; u < 2; ++u) {
+                float *o = osm + (NCB == 1 ? j >> 1 : j) * PS + 2 * ((prow << (lbx + 1)) + px + (u << lbx));
+                if constexpr (NCB == 1) {
+                    const f4 v = u ? acc[0] : acc_a[0];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) o[2 * r + (j & 1)] = v[r];
+                } else {
+                    const f4 re = u ? acc[2 * h] : acc_a[2 * h], im = u ? acc[2 * h + 1] : acc_a[2 * h + 1];
+                    *reinterpret_cast<f4 *>(o) = f4{re[0], im[0], re[1], im[1]};
+                    *reinterpret_cast<f4 *>(o + 4) = f4{re[2], im[2], re[3], im[3]};
                 }
+            }
+            wave_sync();
+#pragma unroll
+            for (int t = 0; t < ncs / 4; ++t) {
+                const int cs = (lane >> 4) + 4 * t, cl = NCB == 4 ? 2 * cs + h : cs;
+                if (cl >= nc) continue;
+                const f4 v = *reinterpret_cast<const f4 *>(osm + cs * PS + 2 * cell);
+                f4 *d = reinterpret_cast<f4 *>(out + (size_t)(c0 + cl) * cells + go);
+                if (nt)
+                    __builtin_nontemporal_store(v, d);
+                else
+                    *d = v;
             }
         }
         return;
@@ -533,71 +557,32 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
     }
     if (i >= iend) return;
 
-    // current item; empty items (units without records) write zeros
-    fr_item cur = items[i];
-    if (bid < front_wg && fsub > 1) {
-        // only the front units of every tstride-th rank; the sub-slice's
-        // records (a multiple of FR_POS_BATCH, possibly none) go to
-        // virtual slot fw
-        if (cur.unit % (uint32_t)tstride != 0) return;
-        const uint32_t sub = (uint32_t)(fw % fsub), len = cur.r1 - cur.r0;
-        const uint32_t sl = ((len + fsub - 1) / fsub + (FR_POS_BATCH - 1)) & ~(uint32_t)(FR_POS_BATCH - 1);
-        const uint32_t a = min(cur.r0 + sub * sl, cur.r1);
-        cur.r0 = a;
-        cur.r1 = min(a + sl, cur.r1);
-        cur.slot = (int32_t)fw;
-    }
-    item_box box = unpack_box(cur.t0, cur.pad);
-    while (cur.r0 == cur.r1) {
-        write_out(cur, box);
-        if (++i >= iend) return;
-        cur = items[i];
-        box = unpack_box(cur.t0, cur.pad);
-    }
-    float fx, fy, fz;
-    lane_cell(box, j, fx, fy, fz);
-
-    // At the end of the current item: write it out, then move to the next
-    // item with records (writing zeros for empty ones).  False when the run
-    // is done.
-    auto next_item = [&]() -> bool {
-        write_out(cur, box);
-        while (++i < iend) {
-            cur = items[i];
-            box = unpack_box(cur.t0, cur.pad);
-            if (cur.r0 < cur.r1) {
-                lane_cell(box, j, fx, fy, fz);
-                return true;
-            }
-            write_out(cur, box);
+    // item by item; units without records are written as zeros
+    for (; i < iend; ++i) {
+        fr_item it = items[i];
+        if (bid < front_wg && fsub > 1) {
+            // only the front units of every tstride-th rank; the sub-slice's
+            // records (a multiple of FR_POS_BATCH, possibly none) go to
+            // virtual slot fw
+            if (it.unit % (uint32_t)tstride != 0) return;
+            const uint32_t sub = (uint32_t)(fw % fsub), len = it.r1 - it.r0;
+            const uint32_t sl = ((len + fsub - 1) / fsub + (FR_POS_BATCH - 1)) & ~(uint32_t)(FR_POS_BATCH - 1);
+            const uint32_t a = min(it.r0 + sub * sl, it.r1);
+            it.r0 = a;
+            it.r1 = min(a + sl, it.r1);
+            it.slot = (int32_t)fw;
         }
-        return false;
-    };
-
-    // the run's items as one record stream (their records are consecutive)
-    uint32_t r = cur.r0;
-    uint32_t id0[4], id1[4];
-    batch_st S0, S1;
-    load_ids(id0, recs, r, k);
-    load_ids(id1, recs, r + RB, k);
-    issue_batch<NCB, PAIR>(S0, id0, pos, data, (uint32_t)C, ca, cbb);
-    while (true) {
-        load_ids(id0, recs, r + 2 * RB, k);
-        issue_batch<NCB, PAIR>(S1, id1, pos, data, (uint32_t)C, ca, cbb);
-        __builtin_amdgcn_sched_barrier(0);
-        apply_batch<NCB, FULL>(acc, S0, stbl, fx, fy, fz, dacc, cidx, lmax, v0ok, v1ok, j);
-        r += RB;
-        if (r == cur.r1 && !next_item()) break;
-        load_ids(id1, recs, r + 2 * RB, k);
-        issue_batch<NCB, PAIR>(S0, id0, pos, data, (uint32_t)C, ca, cbb);
-        __builtin_amdgcn_sched_barrier(0);
-        apply_batch<NCB, FULL>(acc, S1, stbl, fx, fy, fz, dacc, cidx, lmax, v0ok, v1ok, j);
-        r += RB;
-        if (r == cur.r1 && !next_item()) break;
+        const item_box box = unpack_box(it.t0, it.pad);
+        float fx, fy, fz;
+        lane_cell(box, j, fx, fy, fz);
+        if (it.r0 < it.r1)
+            grid_records<NCB, PAIR, SMALL>(acc, it.r0, it.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx, fy, fz,
+                                          cidx, lmax, j, k);
+        write_out(it, box);
     }
 }
 
-template <int NCB, bool PAIR, bool FULL, typename TS, int OCC>
+template <int NCB, bool PAIR, bool SMALL, typename TS, int OCC>
 fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, int64_t tstride, int fsub)
 {
     fr_ctx *ctx = p->ctx;
@@ -620,15 +605,15 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, 
     const int64_t W = front_wg + span * ((groups + span - 1) / span);
     FR_CHECK(ctx, W < (int64_t(1) << 31), FR_ERR_UNSUPPORTED, "gridding launch of %lld workgroups", (long long)W);
     // per wave: the write-out transpose (16 cells x 16 NCB components, or a
-    // pair's 32 cells x 32 components)
-    const int osm_floats = std::max(16 * NCB * CS, (NCB == 4 ? 64 : 32) * 33);
-    const size_t lds = sizeof(float4) * p->L + sizeof(float) * PW * osm_floats;
-    auto kern = k_grid_pos<NCB, PAIR, FULL, TS, OCC>;
+    // step of a pair; a tile of four needs less from its four waves together)
+    const int osm_floats = std::max(16 * NCB * CS, (NCB == 1 ? 8 : 16) * PS);
+    const size_t lds = sizeof(float4) * (p->L + PW * 64) + sizeof(float) * PW * osm_floats;
+    auto kern = k_grid_pos<NCB, PAIR, SMALL, TS, OCC>;
     FR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int lbx = __builtin_ctz((unsigned)p->geom.bx), lby = __builtin_ctz((unsigned)p->geom.by),
               lbz = __builtin_ctz((unsigned)p->geom.bz);
     hipLaunchKernelGGL(kern, dim3((unsigned)W, chunks), dim3(64 * PW), lds, ctx->stream, p->items, p->nitems,
-                       p->tiles, p->ntiles, lbx, lby, lbz, p->recs, p->pos, p->tsel, p->L, p->mfma_dacc, p->mfma_cidx,
+                       p->tiles, p->ntiles, lbx, lby, lbz, p->recs, p->pos, p->tsel, p->L, p->mfma_cidx,
                        (const TS *)s->data, s->C, (int)p->N, cells, out, partial, p->nslots,
                        p->geom.cells_max, p->nitems_front, front_wg, ipw, xr, p->pos_stores == 1 ? 1 : 0,
                        p->tile_units, osm_floats, tstride, tstride > 1 ? fsub : 1);
@@ -636,14 +621,21 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, 
     return FR_OK;
 }
 
+template <int NCB, bool PAIR, typename TS, int OCC>
+fr_status launch_size(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, int64_t ts, int fs)
+{
+    const uint64_t bytes = (uint64_t)(p->M + 1) * s->C * sizeof(TS);
+    return bytes < (uint64_t(1) << 32) ? launch<NCB, PAIR, true, TS, OCC>(p, s, out, partial, ts, fs)
+                                       : launch<NCB, PAIR, false, TS, OCC>(p, s, out, partial, ts, fs);
+}
+
 template <typename TS, int OCC>
 fr_status launch_ncb(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, int64_t ts, int fs)
 {
-    if (s->C <= 8) return launch<1, false, false, TS, OCC>(p, s, out, partial, ts, fs);
-    if (s->C <= 16) return launch<2, false, false, TS, OCC>(p, s, out, partial, ts, fs);
-    if (s->C % 32 == 0) return launch<4, true, true, TS, OCC>(p, s, out, partial, ts, fs);
-    if (s->C % 2 == 0) return launch<4, true, false, TS, OCC>(p, s, out, partial, ts, fs);
-    return launch<4, false, false, TS, OCC>(p, s, out, partial, ts, fs);
+    if (s->C <= 8) return launch_size<1, false, TS, OCC>(p, s, out, partial, ts, fs);
+    if (s->C <= 16) return launch_size<2, false, TS, OCC>(p, s, out, partial, ts, fs);
+    if (s->C % 2 == 0) return launch_size<4, true, TS, OCC>(p, s, out, partial, ts, fs);
+    return launch_size<4, false, TS, OCC>(p, s, out, partial, ts, fs);
 }
 
 // pos[i].w <- the samples' DCF (the null sample keeps 0)

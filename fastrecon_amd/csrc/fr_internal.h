@@ -76,6 +76,7 @@ struct fr_grids {
 #define FR_ACC_POS 6        // matrix-core products of 16-cell units, weights computed from sample positions
 #define FR_POS_MAX_L 2048   // longest LUT of a position-weight plan (its selection table is staged in LDS)
 #define FR_POS_WAVES 4      // waves per workgroup of the position-weight kernel
+#define FR_POS_PAD 256      // null records past a position-weight plan's last one
 #define FR_POS_BATCH 16     // records per batch of the position-weight kernel; units are padded to it
 #define FR_MFMA_MAX_L 4096  // LUT lengths for which the plan builds exact index thresholds (degridding)
 #define FR_CT_MAX_L 1023    // longest LUT for compact 2-byte taps (10-bit index, index L = zero weight)
@@ -214,7 +215,7 @@ struct fr_plan {
     // position-weight mode (FR_ACC_POS): no taps.  hdrs is unused; recs holds
     // each unit's sample indices in ascending order, padded with the index M
     // to a multiple of FR_POS_BATCH (every unit starts at such a multiple),
-    // then 64 more entries M; pos[M + 1] the samples' grid positions and
+    // then FR_POS_PAD more entries M; pos[M + 1] the samples' grid positions and
     // DCF (x, y, z, w; w copied from the samples before every pass), entry
     // M far outside the grid with w = 0; tsel[L] the LUT-index selection
     // table (B[m+1], LUT[m], LUT[m+1], 0) for the estimate m

@@ -877,6 +877,10 @@ fr_status fr_plan_thresholds(fr_plan *p, bool sel)
         std::vector<float4> t(L);
         for (int m = 0; m < L; ++m)
             t[m] = make_float4(B[m + 1], p->host_lut[m], m + 1 < L ? p->host_lut[m + 1] : 0.f, 0.f);
+        // the last entry carries the tap test: a rejected d2 (>= dacc, whose
+        // estimate is L - 1: its root is hw to 1 ulp or more) selects 0, an
+        // accepted one, whose index is at most L - 1, selects LUT[L - 1]
+        t[L - 1].x = p->mfma_dacc;
         if (!p->tsel && (e = fr_alloc(ctx, (void **)&p->tsel, sizeof(float4) * L))) return e;
         FR_HIP(ctx, hipMemcpyAsync(p->tsel, t.data(), sizeof(float4) * L, hipMemcpyHostToDevice, st));
     }

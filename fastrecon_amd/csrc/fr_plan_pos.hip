@@ -264,14 +264,14 @@ __global__ void k_place(const uint32_t *__restrict__ keys, const uint32_t *__res
     recs[P[u] + ((uint64_t)r - Q[u])] = vals[r];
 }
 
-// padding records (null sample M) after each unit's records, and 64 past the end
+// padding records (null sample M) after each unit's records, and FR_POS_PAD past the end
 __global__ void k_pad(int64_t nu, const uint64_t *__restrict__ P, const uint32_t *__restrict__ c_r,
                       const uint32_t *__restrict__ c4_r, uint64_t R4, uint32_t null_sample, uint32_t *__restrict__ recs)
 {
     const int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (u < nu)
         for (uint32_t i = c_r[u]; i < c4_r[u]; ++i) recs[P[u] + i] = null_sample;
-    if (u < 64) recs[R4 + u] = null_sample;
+    if (u < FR_POS_PAD) recs[R4 + u] = null_sample;
 }
 
 __global__ void k_items(int64_t nu, uint32_t S, const uint64_t *__restrict__ P, const uint64_t *__restrict__ I,
@@ -446,7 +446,7 @@ fr_status fr_plan_build_pos(fr_plan *p, const fr_samples *s, const fr_tune *tune
     FR_HIP(ctx, hipMemcpyAsync(&lastn, nrec.p + M - 1, 4, hipMemcpyDeviceToHost, st));
     FR_HIP(ctx, hipStreamSynchronize(st));
     const uint64_t R = last[0] + lastn;
-    FR_CHECK(ctx, R + 4 * (uint64_t)nbox + 64 < (uint64_t(1) << 31), FR_ERR_UNSUPPORTED,
+    FR_CHECK(ctx, R + 16 * (uint64_t)nbox + FR_POS_PAD < (uint64_t(1) << 31), FR_ERR_UNSUPPORTED,
              "plan has %llu records (max about 2^31)", (unsigned long long)R);
 
     // slice size S (records, a multiple of 16): about 32 slices' worth of
@@ -514,7 +514,7 @@ fr_status fr_plan_build_pos(fr_plan *p, const fr_samples *s, const fr_tune *tune
     p->nheavy = (int64_t)tot.nheavy;
     p->nslots = (int64_t)tot.nslots;
     if ((e = fr_alloc(ctx, (void **)&p->units, sizeof(fr_unit) * nu)) ||
-        (e = fr_alloc(ctx, (void **)&p->recs, sizeof(uint32_t) * (tot.R4 + 64))) ||
+        (e = fr_alloc(ctx, (void **)&p->recs, sizeof(uint32_t) * (tot.R4 + FR_POS_PAD))) ||
         (e = fr_alloc(ctx, (void **)&p->items, sizeof(fr_item) * std::max<uint64_t>(1, tot.nitems))) ||
         (e = fr_alloc(ctx, (void **)&p->heavy, sizeof(fr_heavy) * std::max<uint64_t>(1, tot.nheavy))))
         return e;
@@ -540,7 +540,7 @@ fr_status fr_plan_build_pos(fr_plan *p, const fr_samples *s, const fr_tune *tune
         FR_HIP(ctx, hipGetLastError());
         FR_HIP(ctx, hipStreamSynchronize(st));          // before the sort buffers are freed
     }
-    hipLaunchKernelGGL(k_pad, dim3(nblk(std::max<int64_t>(nu, 64), 256)), dim3(256), 0, st, nu, P.p, c_r.p, c4_r.p,
+    hipLaunchKernelGGL(k_pad, dim3(nblk(std::max<int64_t>(nu, FR_POS_PAD), 256)), dim3(256), 0, st, nu, P.p, c_r.p, c4_r.p,
                        tot.R4, (uint32_t)M, p->recs);
 
     // 5. items and heavy units
@@ -550,14 +550,14 @@ fr_status fr_plan_build_pos(fr_plan *p, const fr_samples *s, const fr_tune *tune
 
     // 6. tiles of TW x-adjacent whole units (unit box of 16 cells with
     // power-of-two sides; the grid divides into whole tiles): pairs by
-    // default (tile_writes 0 or 3), rows of 2 bx cells; fours with
+    // default (tile_writes 0 or 3; boxes at least 4 wide), rows of 2 bx cells; fours with
     // tile_writes 1, rows of 4 bx cells; none with tile_writes 2
     const bool pow2 = (geom.bx & (geom.bx - 1)) == 0 && (geom.by & (geom.by - 1)) == 0 &&
                       (geom.bz & (geom.bz - 1)) == 0;
     const int TW = tile_writes == 1 ? FR_POS_WAVES : (tile_writes == 2 ? 0 : 2);
     p->ntiles = 0;
     p->tile_units = 0;
-    if (TW > 0 && pow2 && geom.cells_max == 16 && N % (TW * geom.bx) == 0 && N % geom.by == 0 &&
+    if (TW > 0 && pow2 && (TW != 2 || geom.bx >= 4) && geom.cells_max == 16 && N % (TW * geom.bx) == 0 && N % geom.by == 0 &&
         (flat || N % geom.bz == 0) && nu - (int64_t)tot.nfront_units > 0) {
         const int ntx = g.nbx / TW;
         const int64_t ntiles = (int64_t)ntx * g.nby * g.nbz;

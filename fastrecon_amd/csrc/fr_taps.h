@@ -81,15 +81,15 @@ __device__ __forceinline__ void fr_box_taps(const fr_box &b, const int lo[3], co
 }
 
 // LUT weight of a squared distance d2 (formed with the reference's operations
-// in its order), 0 where the tap test sqrtf(d2) < hw (GridLut.cpp:133) fails
-// (d2 >= dacc).  The index comes from the hardware's 1-ulp square root: est =
-// floor(sqrt~(d2) (L - 1) / hw + 0.49) is the reference index or one below
-// it, and the comparison with stbl[est].x, the least d2 of the next index,
-// picks LUT[est] or LUT[est + 1] (.y, .z).  stbl: a plan's selection table.
-__device__ __forceinline__ float fr_tap_weight(float d2, const float4 *stbl, float dacc, float cidx, float lmax)
+// in its order), 0 where the tap test sqrtf(d2) < hw (GridLut.cpp:133) fails.
+// The index comes from the hardware's 1-ulp square root: est = floor(sqrt~(d2)
+// (L - 1) / hw + 0.49) is the reference index or one below it, and the
+// comparison with stbl[est].x, the least d2 of the next index, picks LUT[est]
+// or LUT[est + 1] (.y, .z).  stbl: a plan's selection table, whose last entry
+// holds the tap test (.x the least rejected d2, .z 0).
+__device__ __forceinline__ float fr_tap_weight(float d2, const float4 *stbl, float cidx, float lmax)
 {
     const float est = fminf(__builtin_fmaf(__builtin_amdgcn_sqrtf(d2), cidx, 0.49f), lmax);
     const float4 e = stbl[(int)est];
-    const float w = d2 >= e.x ? e.z : e.y;
-    return d2 < dacc ? w : 0.f;
+    return d2 >= e.x ? e.z : e.y;
 }

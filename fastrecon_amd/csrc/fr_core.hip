@@ -24,17 +24,87 @@ fr_status fr_fail(fr_ctx *ctx, fr_status st, const char *fmt, ...)
     return st;
 }
 
+// frees what the pool keeps down to `limit` bytes, oldest first (m is held)
+static void pool_trim(fr_pool &pool, size_t limit)
+{
+    size_t n = 0;
+    for (; n < pool.kept.size() && pool.kept_bytes > limit; ++n) {
+        pool.kept_bytes -= pool.kept[n].bytes;
+        (void)hipFree(pool.kept[n].p);
+    }
+    pool.kept.erase(pool.kept.begin(), pool.kept.begin() + n);
+}
+
 fr_status fr_alloc(fr_ctx *ctx, void **p, size_t bytes)
 {
     *p = nullptr;
     if (bytes == 0) return FR_OK;
     hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {                      // once more without the pool's blocks
+        (void)hipGetLastError();
+        std::lock_guard<std::mutex> lock(ctx->pool.m);
+        if (ctx->pool.kept_bytes > 0) {
+            pool_trim(ctx->pool, 0);
+            e = hipMalloc(p, bytes);
+        }
+    }
     if (e != hipSuccess) {
         *p = nullptr;
         (void)hipGetLastError();
         return fr_fail(ctx, FR_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     }
     return FR_OK;
+}
+
+fr_status fr_pool_alloc(fr_ctx *ctx, void **p, size_t bytes)
+{
+    *p = nullptr;
+    if (bytes == 0) return FR_OK;
+    fr_pool &pool = ctx->pool;
+    // sizes in steps of about a sixteenth, so that blocks of
+    // nearly the same use (the record lists of similar scans) replace each other
+    size_t step = 4096;
+    while (bytes <= FR_POOL_BYTES && step * 16 <= bytes) step *= 2;
+    const size_t size = (bytes + step - 1) / step * step;
+    {
+        std::lock_guard<std::mutex> lock(pool.m);
+        size_t best = pool.kept.size();
+        for (size_t i = 0; i < pool.kept.size(); ++i)
+            if (pool.kept[i].bytes >= size && pool.kept[i].bytes <= size + size / 4 &&
+                (best == pool.kept.size() || pool.kept[i].bytes < pool.kept[best].bytes))
+                best = i;
+        if (best < pool.kept.size()) {
+            const fr_pool::block b = pool.kept[best];
+            pool.out.emplace(b.p, b.bytes);     // before the block leaves the list
+            pool.kept.erase(pool.kept.begin() + best);
+            pool.kept_bytes -= b.bytes;
+            *p = b.p;
+            return FR_OK;
+        }
+    }
+    const fr_status e = fr_alloc(ctx, p, size);
+    if (e) return e;
+    std::lock_guard<std::mutex> lock(pool.m);
+    pool.out.emplace(*p, size);
+    return FR_OK;
+}
+
+void fr_pool_free(fr_ctx *ctx, void *p)
+{
+    if (!p) return;
+    fr_pool &pool = ctx->pool;
+    std::lock_guard<std::mutex> lock(pool.m);
+    const auto it = pool.out.find(p);
+    if (it == pool.out.end() || it->second > FR_POOL_BYTES) {
+        if (it != pool.out.end()) pool.out.erase(it);
+        (void)hipFree(p);
+        return;
+    }
+    const fr_pool::block b{p, it->second};
+    pool.out.erase(it);
+    pool_trim(pool, FR_POOL_BYTES - b.bytes);
+    pool.kept.push_back(b);
+    pool.kept_bytes += b.bytes;
 }
 
 // ------------------------------------------------------------------ context
@@ -71,6 +141,10 @@ extern "C" fr_status fr_ctx_destroy(fr_ctx *ctx)
     if (!ctx) return FR_OK;
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
+    {
+        std::lock_guard<std::mutex> lock(ctx->pool.m);
+        pool_trim(ctx->pool, 0);
+    }
     hipStreamDestroy(ctx->stream);
     delete ctx;
     return FR_OK;

@@ -489,10 +489,10 @@ fr_status fr_launch_grid(fr_plan *p, const fr_samples *s, float2 *out, int force
     } else {
         if (need > p->partial_bytes) {
             FR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            hipFree(p->partial);
+            fr_pool_free(ctx, p->partial);
             p->partial = nullptr;
             p->partial_bytes = 0;
-            fr_status e = fr_alloc(ctx, (void **)&p->partial, need);
+            fr_status e = fr_pool_alloc(ctx, (void **)&p->partial, need);
             if (e) return e;
             p->partial_bytes = need;
         }

@@ -7,10 +7,27 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdarg>
+#include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "fastrecon_hip.h"
+
+// Device memory given back by plans, kept for the next ones: hipMalloc and
+// hipFree of a plan's buffers cost more than the kernels that fill them.  One
+// per context; all its users' work is on the context's stream, so a block may
+// be handed out again as soon as it is given back.  At most FR_POOL_BYTES
+// stay in it (the oldest go first); all of it is freed when an allocation
+// fails and with the context.
+constexpr size_t FR_POOL_BYTES = size_t(2) << 30;
+struct fr_pool {
+    struct block { void *p; size_t bytes; };
+    std::mutex m;
+    std::vector<block> kept;                    // oldest first
+    size_t kept_bytes = 0;
+    std::unordered_map<void *, size_t> out;     // blocks in use
+};
 
 struct fr_ctx {
     int device = 0;
@@ -19,6 +36,7 @@ struct fr_ctx {
     int cu_count = 0;
     std::string arch;          // gcnArchName up to the first ':' (e.g. gfx950)
     void *scratch = nullptr;   // this device's copy of the static scratch (fr_noalloc.hip)
+    fr_pool pool;
 };
 
 struct fr_samples {
@@ -269,6 +287,10 @@ fr_status fr_fail(fr_ctx *ctx, fr_status st, const char *fmt, ...);
     } while (0)
 
 fr_status fr_alloc(fr_ctx *ctx, void **p, size_t bytes);
+// from and to the context's pool: for buffers that only work on the context's
+// stream touches.  fr_pool_free also takes memory of fr_alloc.
+fr_status fr_pool_alloc(fr_ctx *ctx, void **p, size_t bytes);
+void fr_pool_free(fr_ctx *ctx, void *p);
 
 static inline size_t fr_cells(int dim, unsigned N)
 {

@@ -388,16 +388,36 @@ int ref_lut_index(float d2, float hw, int L)
 }
 
 // Least non-negative float x with pred(x), by bisection on the bit pattern
-// (non-negative floats order like their bits); pred is monotone.
+// (non-negative floats order like their bits); pred is monotone and holds at
+// hi_bits.  The search widens from a guess, a few steps from the answer.
 template <typename P>
-float least_float(uint32_t hi_bits, P &&pred)
+float least_float(uint32_t hi_bits, float guess, P &&pred)
 {
-    uint32_t lo = 0, hi = hi_bits;               // pred(hi) holds
+    auto holds = [&](uint32_t bits) {
+        float x;
+        std::memcpy(&x, &bits, 4);
+        return pred(x);
+    };
+    uint32_t at;
+    std::memcpy(&at, &guess, 4);
+    if (at > hi_bits) at = hi_bits;              // also a negative guess or NaN
+    uint32_t lo = 0, hi = hi_bits;               // the answer is in [lo, hi]
+    for (uint32_t step = 4;; step *= 4) {
+        if (holds(at)) {
+            hi = at;
+            if (at == 0) break;
+            at = at > step ? at - step : 0;
+            if (!holds(at)) { lo = at + 1; break; }
+        } else {
+            lo = at + 1;
+            at = hi_bits - at > step ? at + step : hi_bits;
+            if (holds(at)) { hi = at; break; }
+        }
+        if (step > (1u << 28)) break;
+    }
     while (lo < hi) {
         const uint32_t mid = lo + (hi - lo) / 2;
-        float x;
-        std::memcpy(&x, &mid, 4);
-        if (pred(x)) hi = mid; else lo = mid + 1;
+        if (holds(mid)) hi = mid; else lo = mid + 1;
     }
     float x;
     std::memcpy(&x, &lo, 4);
@@ -865,13 +885,15 @@ fr_status fr_plan_thresholds(fr_plan *p, bool sel)
     std::vector<float> B(L + 2, INFINITY);
     for (int m = 0; m < L; ++m) {
         if (ref_lut_index(top, hw, L) < m) break;           // not reached below the search bound
-        B[m] = least_float(top_bits, [&](float d2) { return ref_lut_index(d2, hw, L) >= m; });
+        const double dk = (m - 0.5) * (double)hw / (L - 1);
+        B[m] = least_float(top_bits, m ? (float)(dk * dk) : 0.f,
+                           [&](float d2) { return ref_lut_index(d2, hw, L) >= m; });
     }
-    p->mfma_dacc = least_float(top_bits, [&](float d2) { return sqrtf(d2) >= hw; });
+    p->mfma_dacc = least_float(top_bits, hw * hw, [&](float d2) { return sqrtf(d2) >= hw; });
     p->mfma_cidx = (float)((double)(L - 1) / (double)hw);
     std::vector<float2> pairs(L + 1);
     for (int m = 0; m <= L; ++m) pairs[m] = make_float2(B[m], B[m + 1]);
-    if (!p->mfma_pairs && (e = fr_alloc(ctx, (void **)&p->mfma_pairs, sizeof(float2) * (L + 1)))) return e;
+    if (!p->mfma_pairs && (e = fr_pool_alloc(ctx, (void **)&p->mfma_pairs, sizeof(float2) * (L + 1)))) return e;
     FR_HIP(ctx, hipMemcpyAsync(p->mfma_pairs, pairs.data(), sizeof(float2) * (L + 1), hipMemcpyHostToDevice, st));
     if (sel) {
         std::vector<float4> t(L);
@@ -881,7 +903,7 @@ fr_status fr_plan_thresholds(fr_plan *p, bool sel)
         // estimate is L - 1: its root is hw to 1 ulp or more) selects 0, an
         // accepted one, whose index is at most L - 1, selects LUT[L - 1]
         t[L - 1].x = p->mfma_dacc;
-        if (!p->tsel && (e = fr_alloc(ctx, (void **)&p->tsel, sizeof(float4) * L))) return e;
+        if (!p->tsel && (e = fr_pool_alloc(ctx, (void **)&p->tsel, sizeof(float4) * L))) return e;
         FR_HIP(ctx, hipMemcpyAsync(p->tsel, t.data(), sizeof(float4) * L, hipMemcpyHostToDevice, st));
     }
     FR_HIP(ctx, hipStreamSynchronize(st));
@@ -925,7 +947,7 @@ extern "C" fr_status fr_plan_create(fr_ctx *ctx, const fr_samples *s, unsigned N
     p->kWidth = kWidth; p->kHW = kWidth / 2.0f; p->L = L;     // GridLut.cpp:86
     p->traj_uid = s->uid; p->traj_version = s->traj_version;
     p->host_lut.assign(lut, lut + L);
-    fr_status e = fr_alloc(ctx, (void **)&p->lut, sizeof(float) * L);
+    fr_status e = fr_pool_alloc(ctx, (void **)&p->lut, sizeof(float) * L);
     if (!e) {
         hipError_t he = hipMemcpyAsync(p->lut, lut, sizeof(float) * L, hipMemcpyHostToDevice, ctx->stream);
         if (he != hipSuccess) e = fr_fail(ctx, FR_ERR_HIP, "lut upload: %s", hipGetErrorString(he));
@@ -940,9 +962,10 @@ extern "C" fr_status fr_plan_destroy(fr_plan *p)
 {
     if (!p) return FR_OK;
     hipStreamSynchronize(p->ctx->stream);
-    hipFree(p->lut); hipFree(p->units); hipFree(p->hdrs); hipFree(p->taps); hipFree(p->tstart);
-    hipFree(p->items); hipFree(p->heavy); hipFree(p->partial); hipFree(p->batches); hipFree(p->mfma_pairs);
-    hipFree(p->recs); hipFree(p->pos); hipFree(p->tsel); hipFree(p->tiles);
+    for (void *q : {(void *)p->lut, (void *)p->units, (void *)p->hdrs, (void *)p->taps, (void *)p->tstart,
+                    (void *)p->items, (void *)p->heavy, (void *)p->partial, (void *)p->batches, (void *)p->mfma_pairs,
+                    (void *)p->recs, (void *)p->pos, (void *)p->tsel, (void *)p->tiles})
+        fr_pool_free(p->ctx, q);
     hipFree(p->dcf_den);
     hipFree(p->dcf_scr);
     fr_tiles_free(p->tord);

@@ -26,7 +26,7 @@
 
 namespace {
 
-constexpr int TR = 16;          // rows per workgroup tile of the x and y passes
+constexpr int TR = 16;          // rows per workgroup tile of the x and y passes (8 where those tiles are few)
 constexpr int TS = 8;           // rows (output columns) per workgroup tile of the last pass: twice the
                                 // workgroups of a 16-row tile (the pass has only rc^2 / TS tiles)
 // waves per workgroup, each taking TR / NW rows of the tile (8 waves for
@@ -256,52 +256,52 @@ __device__ __forceinline__ int crop_pos(int k, int N, int rc, int shift)
     return kp < rc ? kp : -1;
 }
 
-// Pass over tiles of TR rows: row t of tile T starts at in + rowA(T) + t *
+// Pass over tiles of R rows: row t of tile T starts at in + rowA(T) + t *
 // rowStride; kept output k' of row t goes to out[outA(T) + k' * outK + t].
-// Layout parameters: tile T = (a, b, c0) over dims (na, nb, nt = rows / TR).
+// Layout parameters: tile T = (a, b, c0) over dims (na, nb, nt = rows / R).
 struct pass_desc {
     int64_t na, nb, nt;                          // tile grid
-    int64_t inA, inB, inT, rowStride;            // in offset = a inA + b inB + (t0 + t) rowStride (t0 = tt * TR)
-    int64_t outA, outB, outT, outK;              // out offset = a outA + b outB + tt*TR*outT + k' outK + t outT
+    int64_t inA, inB, inT, rowStride;            // in offset = a inA + b inB + (t0 + t) rowStride (t0 = tt * R)
+    int64_t outA, outB, outT, outK;              // out offset = a outA + b outB + tt*R*outT + k' outK + t outT
 };
 
-template <int N, int NW = waves<N>(), int WGT = 64 * waves<N>()>
+template <int N, int R = TR, int NW = waves<N>(), int WGT = 64 * waves<N>()>
 __global__ void __launch_bounds__(WGT) k_fft_pass(const float2 *__restrict__ in, float2 *__restrict__ out,
                                                   const float2 *__restrict__ gtw, pass_desc d, int rc, int shift,
                                                   float s)
 {
     __shared__ float2 tw[N];
     __shared__ float2 fbuf[NW][2 * N];
-    extern __shared__ float2 otile[];           // [rc][TR]
+    extern __shared__ float2 otile[];           // [rc][R]
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     for (int i = threadIdx.x; i < N; i += WGT) tw[i] = gtw[i];
     __syncthreads();
     const int64_t T = blockIdx.x;
     const int64_t tt = T % d.nt, b = (T / d.nt) % d.nb, a = T / (d.nt * d.nb);
-    const float2 *base = in + a * d.inA + b * d.inB + tt * TR * d.rowStride;
+    const float2 *base = in + a * d.inA + b * d.inB + tt * R * d.rowStride;
     // rows w, w + NW, .. of the tile, each wave's rows loaded two ahead
     float2 xa[b4<N>()][4], xb[b4<N>()][4], xc[b4<N>()][4];
     load_row<N>(base + (int64_t)w * d.rowStride, xa, lane);
     load_row<N>(base + (int64_t)(w + NW) * d.rowStride, xb, lane);
 #pragma unroll
-    for (int i = 0; i < TR / NW; ++i) {
+    for (int i = 0; i < R / NW; ++i) {
         const int t = w + NW * i;
         float2 (&cur)[b4<N>()][4] = i % 3 == 0 ? xa : (i % 3 == 1 ? xb : xc);
         float2 (&nxt)[b4<N>()][4] = (i + 2) % 3 == 0 ? xa : ((i + 2) % 3 == 1 ? xb : xc);
-        if (i + 2 < TR / NW) load_row<N>(base + (int64_t)(t + 2 * NW) * d.rowStride, nxt, lane);
+        if (i + 2 < R / NW) load_row<N>(base + (int64_t)(t + 2 * NW) * d.rowStride, nxt, lane);
         float2 v[nv<N>()];
         fft_row<N>(cur, v, fbuf[w], tw, lane, s);
 #pragma unroll
         for (int q = 0; q < nv<N>(); ++q) {
             const int k = out_k<N>(lane, q);
             const int kp = k < 0 ? -1 : crop_pos(k, N, rc, shift);
-            if (kp >= 0) otile[kp * TR + t] = v[q];
+            if (kp >= 0) otile[kp * R + t] = v[q];
         }
     }
     __syncthreads();
-    float2 *ob = out + a * d.outA + b * d.outB + tt * TR * d.outT;
-    for (int i = threadIdx.x; i < rc * TR; i += WGT) {
-        const int kp = i / TR, t = i % TR;
+    float2 *ob = out + a * d.outA + b * d.outB + tt * R * d.outT;
+    for (int i = threadIdx.x; i < rc * R; i += WGT) {
+        const int kp = i / R, t = i % R;
         ob[(int64_t)kp * d.outK + (int64_t)t * d.outT] = otile[i];
     }
 }
@@ -365,7 +365,90 @@ __global__ void __launch_bounds__(WGT) k_fft_sos(const float2 *__restrict__ in, 
     }
 }
 
+// The last pass where k_fft_sos has too few tiles to fill the chip (one 2D
+// image): 8 waves take TC columns x 8 / TC coils at a time, one row each, and
+// the squares go through LDS to be summed in coil order -- the same sums.
+// A coil takes about 1.7 us of a wave (latency of the row's chain of LDS
+// exchanges) whatever the chip does besides, so the coils in turn are what
+// costs.  8 coils on 512^2: 27.9 us in 32 workgroups -> 6.4 in 256.
+constexpr int SW = 8;
+template <int N, int TC>
+__global__ void __launch_bounds__(64 * SW) k_fft_sos_coils(const float2 *__restrict__ in, float *__restrict__ img,
+                                                           const float2 *__restrict__ gtw, int64_t nt, int C,
+                                                           int64_t inC, int64_t inA, int64_t rowStride, int64_t outA,
+                                                           int64_t outK, int rc, int shift, float s,
+                                                           const float *__restrict__ deapod, int64_t dmod)
+{
+    constexpr int G = SW / TC;                   // coils at a time
+    extern __shared__ float2 sm[];               // tw[N], a row's buffers per wave, squares [SW][rc], sums [rc][TC]
+    float2 *tw = sm;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    float2 *fbuf = sm + N + w * 2 * N;
+    float *sq = reinterpret_cast<float *>(sm + N + SW * 2 * N), *acc = sq + SW * rc;
+    for (int i = threadIdx.x; i < N; i += 64 * SW) tw[i] = gtw[i];
+    for (int i = threadIdx.x; i < rc * TC; i += 64 * SW) acc[i] = 0.f;
+    const int64_t T = blockIdx.x;
+    const int64_t tt = T % nt, a = T / nt;
+    const float2 *row = in + a * inA + (tt * TC + w % TC) * rowStride;
+    float2 x[b4<N>()][4];
+    load_row<N>(row + min(w / TC, C - 1) * inC, x, lane);
+    __syncthreads();
+#pragma unroll 1
+    for (int c0 = 0; c0 < C; c0 += G) {
+        float2 v[nv<N>()];
+        fft_row<N>(x, v, fbuf, tw, lane, s);
+        if (c0 + G < C) load_row<N>(row + min(c0 + G + w / TC, C - 1) * inC, x, lane);
+#pragma unroll
+        for (int q = 0; q < nv<N>(); ++q) {
+            const int k = out_k<N>(lane, q);
+            const int kp = k < 0 ? -1 : crop_pos(k, N, rc, shift);
+            if (kp >= 0) sq[w * rc + kp] = __fadd_rn(__fmul_rn(v[q].x, v[q].x), __fmul_rn(v[q].y, v[q].y));
+        }
+        __syncthreads();
+        const int n = min(G, C - c0);
+        for (int i = threadIdx.x; i < rc * TC; i += 64 * SW) {
+            const int kp = i / TC, t = i % TC;
+            float m = acc[i];
+            for (int g = 0; g < n; ++g) m = __fadd_rn(m, sq[(g * TC + t) * rc + kp]);
+            acc[i] = m;
+        }
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < rc * TC; i += 64 * SW) {
+        const int kp = i / TC, t = i % TC;
+        const int64_t o = a * outA + (int64_t)kp * outK + tt * TC + t;
+        float m = sqrtf(acc[i]);
+        if (deapod) m = __fdiv_rn(m, deapod[o % dmod]);
+        img[o] = m;
+    }
+}
+
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
+
+// Last pass over na slices of rcx columns: tiles of TS columns with the coils
+// in turn, or the coils side by side where those tiles would leave more than
+// half of the chip without a workgroup.
+template <int N>
+fr_status run_sos(fr_fft *f, const float2 *in, float *out, int64_t na, int rcx, int C, int64_t inC, int64_t inA,
+                  int64_t rowStride, int64_t outA, int64_t outK, int rc, int shift, float s, const float *deapod,
+                  int64_t dmod)
+{
+    fr_ctx *ctx = f->ctx;
+    if (C > 1 && na * (rcx / TS) <= ctx->cu_count / 2) {
+        const int tc = C > 4 ? 1 : C > 2 ? 2 : 4;
+        auto kern = tc == 1 ? k_fft_sos_coils<N, 1> : tc == 2 ? k_fft_sos_coils<N, 2> : k_fft_sos_coils<N, 4>;
+        const size_t lds = sizeof(float2) * N * (1 + 2 * SW) + sizeof(float) * rc * (SW + tc);
+        FR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kern, dim3((unsigned)(na * (rcx / tc))), dim3(64 * SW), lds, ctx->stream, in, out, f->tw,
+                           (int64_t)(rcx / tc), C, inC, inA, rowStride, outA, outK, rc, shift, s, deapod, dmod);
+    } else {
+        hipLaunchKernelGGL(k_fft_sos<N>, dim3((unsigned)(na * (rcx / TS))), dim3(64 * waves<N>()),
+                           sizeof(float) * TS * rc, ctx->stream, in, out, f->tw, na, (int64_t)(rcx / TS), C, inC, inA,
+                           rowStride, outA, outK, rc, shift, s, deapod, dmod);
+    }
+    FR_HIP(ctx, hipGetLastError());
+    return FR_OK;
+}
 
 template <int N>
 fr_status run_passes(fr_fft *f, const fr_grids *g, int rcx, int rcy, int rcz, int shift, const float *deapod,
@@ -393,30 +476,27 @@ fr_status run_passes(fr_fft *f, const fr_grids *g, int rcx, int rcy, int rcz, in
         hipLaunchKernelGGL(k_fft_pass<N>, dim3((unsigned)(C * rcx * (N / TR))), dim3(WGT), lds_row * rcy,
                            ctx->stream, B1, B2, f->tw, d2, rcy, shift, s);
         // z + coil sum: tiles (ky, kx-block); row (c, ky, kx) of B2; img[kz][ky][kx]
-        hipLaunchKernelGGL(k_fft_sos<N>, dim3((unsigned)(rcy * (rcx / TS))), dim3(WGT), sizeof(float) * TS * rcz,
-                           ctx->stream, B2, out, f->tw, (int64_t)rcy, (int64_t)(rcx / TS), C,
-                           (int64_t)rcy * rcx * N, (int64_t)rcx * N, (int64_t)N, (int64_t)rcx,
-                           (int64_t)rcy * rcx, rcz, shift, s, deapod, (int64_t)rcz * rcy * rcx);
+        return run_sos<N>(f, B2, out, rcy, rcx, C, (int64_t)rcy * rcx * N, (int64_t)rcx * N, (int64_t)N, (int64_t)rcx,
+                          (int64_t)rcy * rcx, rcz, shift, s, deapod, (int64_t)rcz * rcy * rcx);
     } else {
         const int F = std::max(g->frames, 1);
         const int64_t n1 = (int64_t)C * F * rcx * N;
         fr_status e = fr_fft_workspace(f, sizeof(float2) * (size_t)n1);
         if (e) return e;
         float2 *B1 = (float2 *)f->crop_ws;
-        // x: tiles (c, f, y-block); out B1[c][f][kx][y]
-        pass_desc d1{C, F, N / TR, (int64_t)F * N * N, (int64_t)N * N, 0, N,
+        // x: tiles (c, f, y-block); out B1[c][f][kx][y].  Tiles of 8 rows, two
+        // a wave, where those of 16 are at most two for every CU: 8 coils on
+        // 512^2 11.3 -> 9.7 us
+        const int R = (int64_t)C * F * (N / TR) <= 2 * ctx->cu_count ? 8 : TR;
+        pass_desc d1{C, F, N / R, (int64_t)F * N * N, (int64_t)N * N, 0, N,
                      (int64_t)F * rcx * N, (int64_t)rcx * N, 1, N};
-        hipLaunchKernelGGL(k_fft_pass<N>, dim3((unsigned)(C * F * (N / TR))), dim3(WGT), lds_row * rcx, ctx->stream,
-                           g->data, B1, f->tw, d1, rcx, shift, s);
+        hipLaunchKernelGGL((R == 8 ? k_fft_pass<N, 8> : k_fft_pass<N>), dim3((unsigned)(C * F * (N / R))), dim3(WGT),
+                           sizeof(float2) * R * rcx, ctx->stream, g->data, B1, f->tw, d1, rcx, shift, s);
         // y + coil sum: tiles (f, kx-block); row (c, f, kx) of B1; img[f][ky][kx]
         // (the deapodisation map is one rcy x rcx image shared by the frames)
-        hipLaunchKernelGGL(k_fft_sos<N>, dim3((unsigned)(F * (rcx / TS))), dim3(WGT), sizeof(float) * TS * rcy,
-                           ctx->stream, B1, out, f->tw, (int64_t)F, (int64_t)(rcx / TS), C, (int64_t)F * rcx * N,
-                           (int64_t)rcx * N, (int64_t)N, (int64_t)rcy * rcx, (int64_t)rcx, rcy, shift, s, deapod,
-                           (int64_t)rcy * rcx);
+        return run_sos<N>(f, B1, out, F, rcx, C, (int64_t)F * rcx * N, (int64_t)rcx * N, (int64_t)N,
+                          (int64_t)rcy * rcx, (int64_t)rcx, rcy, shift, s, deapod, (int64_t)rcy * rcx);
     }
-    FR_HIP(ctx, hipGetLastError());
-    return FR_OK;
 }
 
 }  // namespace

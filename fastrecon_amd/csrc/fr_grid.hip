@@ -404,6 +404,10 @@ __global__ void __launch_bounds__(64) k_grid_gather(const fr_item *__restrict__ 
 }
 
 // Heavy units: sum their slices' partial boxes in slice order, write the grid.
+// Bound by the latency of a unit's slices one after the other: AHEAD of them
+// are loaded before they are added (8 coils, 402 spokes on 512^2: 10.5 ->
+// 5.0 us).
+constexpr uint32_t AHEAD = 8;
 __global__ void k_combine(const fr_heavy *__restrict__ heavy, const fr_unit *__restrict__ units,
                           const float2 *__restrict__ partial, int64_t nslots, int cells_max, int C, int N, size_t cells,
                           float2 *__restrict__ out)
@@ -420,11 +424,27 @@ __global__ void k_combine(const fr_heavy *__restrict__ heavy, const fr_unit *__r
         const int c = q / ncell;
         const int cell = q - c * ncell;
         float2 a = make_float2(0.f, 0.f);
-        for (uint32_t k = 0; k < h.nitems; ++k) {
-            const float2 v = base[k * slot_stride + (size_t)c * cells_max + cell];
-            a.x = __fadd_rn(a.x, v.x);
-            a.y = __fadd_rn(a.y, v.y);
+        const float2 *p = base + (size_t)c * cells_max + cell;
+        uint32_t k = 0;
+        for (; k + AHEAD <= h.nitems; k += AHEAD) {
+            float2 v[AHEAD];
+#pragma unroll
+            for (uint32_t i = 0; i < AHEAD; ++i) v[i] = p[(k + i) * slot_stride];
+#pragma unroll
+            for (uint32_t i = 0; i < AHEAD; ++i) {
+                a.x = __fadd_rn(a.x, v[i].x);
+                a.y = __fadd_rn(a.y, v[i].y);
+            }
         }
+        float2 v[AHEAD];                // the last fewer than AHEAD: slot 0 in place of those past the end
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; ++i) v[i] = p[(k + i < h.nitems ? k + i : 0u) * slot_stride];
+#pragma unroll
+        for (uint32_t i = 0; i < AHEAD; ++i)
+            if (k + i < h.nitems) {
+                a.x = __fadd_rn(a.x, v[i].x);
+                a.y = __fadd_rn(a.y, v[i].y);
+            }
         const int lx = cell % ux;
         const int ly = (cell / ux) % uy;
         const int lz = cell / (ux * uy);

@@ -1,0 +1,431 @@
+// Batched in-place FFTs of the grids along each axis in turn (unnormalised,
+// exp(sign 2 pi i / N)), for the sizes that fr_fft_radices takes: the
+// transform of ImageFilter/FFT.cpp:40-51,82-84.
+//
+// One pass per axis over the whole array, so what bounds it is memory: each
+// pass reads and writes the array once.  A workgroup transforms a tile of TC
+// rows (along x: whole rows; along y and z: TC neighbouring columns, so that
+// reads and writes are runs of 8 TC bytes) in mixed-radix Stockham stages.
+// The first stage's inputs come from memory straight into registers and the
+// last stage's outputs go straight back, so a length of three stages makes
+// two exchanges through LDS, in place: every thread holds its one or two
+// butterflies of a stage in registers, and a barrier parts all reads from all
+// writes.  Twiddles come from a table evaluated in FP64.
+//
+// Measured against rocFFT, whose plans of these sizes take strided passes and
+// transposes besides: 5 x 180^3 653 -> 315 us, 8 x 192^3 782 -> 709, 8 x 256^3
+// 1821 -> 1491, 8 x 96^3 94 -> 77, 8 x 512^2 31 -> 23 (about 4 TB/s where the
+// array is larger than the caches).  Relative L2 error 1.3e-7 .. 2.0e-7, up to
+// 17% below rocFFT's at each of 31 sizes from 96^2 to 288^3.
+#include "fr_internal.h"
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+
+namespace {
+
+constexpr int MAX_STAGES = FR_FFT_STAGES, MAX_THREADS = 512;
+using stage_desc = fr_fft_desc::stage;
+using fft_desc = fr_fft_desc;
+
+// t / d by the high word of t m, m = ceil(2^32 / d) (0: d = 1), for the t
+// below 2^16 that occur
+__device__ __forceinline__ uint32_t quot(uint32_t t, uint32_t m) { return m ? __umulhi(t, m) : t; }
+
+__device__ __forceinline__ float2 operator+(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ float2 operator-(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ float2 cmul(float2 a, float2 b)
+{
+    return make_float2(__builtin_fmaf(a.x, b.x, -(a.y * b.y)), __builtin_fmaf(a.x, b.y, a.y * b.x));
+}
+// a + b c, c real
+__device__ __forceinline__ float2 axpy(float2 a, float2 b, float c)
+{
+    return make_float2(__builtin_fmaf(b.x, c, a.x), __builtin_fmaf(b.y, c, a.y));
+}
+// a + s i b
+__device__ __forceinline__ float2 add_i(float2 a, float2 b, float s)
+{
+    return make_float2(__builtin_fmaf(-s, b.y, a.x), __builtin_fmaf(s, b.x, a.y));
+}
+
+// R-point DFTs with w = exp(s 2 pi i / R), in place, natural order
+template <int R>
+__device__ __forceinline__ void dft(float2 (&x)[R], float s)
+{
+    if constexpr (R == 2) {
+        const float2 a = x[0], b = x[1];
+        x[0] = a + b;
+        x[1] = a - b;
+    } else if constexpr (R == 3) {
+        const float2 p = x[1] + x[2], d = x[1] - x[2], m = axpy(x[0], p, -0.5f);
+        const float h = s * 0.866025403784438647f;
+        x[0] = x[0] + p;
+        x[1] = add_i(m, d, h);
+        x[2] = add_i(m, d, -h);
+    } else if constexpr (R == 4) {
+        const float2 a = x[0] + x[2], b = x[0] - x[2], c = x[1] + x[3], d = x[1] - x[3];
+        x[0] = a + c;
+        x[1] = add_i(b, d, s);
+        x[2] = a - c;
+        x[3] = add_i(b, d, -s);
+    } else if constexpr (R == 5) {
+        constexpr float c1 = 0.309016994374947424f, c2 = -0.809016994374947424f;
+        constexpr float s1 = 0.951056516295153572f, s2 = 0.587785252292473129f;
+        const float2 p1 = x[1] + x[4], d1 = x[1] - x[4], p2 = x[2] + x[3], d2 = x[2] - x[3];
+        const float2 a = axpy(axpy(x[0], p1, c1), p2, c2), b = axpy(axpy(x[0], p1, c2), p2, c1);
+        const float2 u = axpy(make_float2(d1.x * s1, d1.y * s1), d2, s2);
+        const float2 v = axpy(make_float2(d1.x * s2, d1.y * s2), d2, -s1);
+        x[0] = x[0] + (p1 + p2);
+        x[1] = add_i(a, u, s);
+        x[4] = add_i(a, u, -s);
+        x[2] = add_i(b, v, s);
+        x[3] = add_i(b, v, -s);
+    } else if constexpr (R == 7) {
+        constexpr float c1 = 0.623489801858733531f, c2 = -0.222520933956314404f, c3 = -0.900968867902419126f;
+        constexpr float s1 = 0.781831482468029809f, s2 = 0.974927912181823607f, s3 = 0.433883739117558120f;
+        const float2 p1 = x[1] + x[6], d1 = x[1] - x[6], p2 = x[2] + x[5], d2 = x[2] - x[5], p3 = x[3] + x[4],
+                     d3 = x[3] - x[4];
+        auto even = [&](float a, float b, float c) __attribute__((always_inline)) {
+            return axpy(axpy(axpy(x[0], p1, a), p2, b), p3, c);
+        };
+        auto odd = [&](float a, float b, float c) __attribute__((always_inline)) {
+            return axpy(axpy(make_float2(d1.x * a, d1.y * a), d2, b), d3, c);
+        };
+        const float2 e1 = even(c1, c2, c3), e2 = even(c2, c3, c1), e3 = even(c3, c1, c2);
+        const float2 o1 = odd(s1, s2, s3), o2 = odd(s2, -s3, -s1), o3 = odd(s3, -s1, s2);
+        x[0] = x[0] + ((p1 + p2) + p3);
+        x[1] = add_i(e1, o1, s);
+        x[6] = add_i(e1, o1, -s);
+        x[2] = add_i(e2, o2, s);
+        x[5] = add_i(e2, o2, -s);
+        x[3] = add_i(e3, o3, s);
+        x[4] = add_i(e3, o3, -s);
+    } else {
+        // R = 2 H: halves of even and odd inputs, X[k] = E[k] + w^k O[k], X[k + H] = E[k] - w^k O[k]
+        constexpr int H = R / 2;
+        static_assert(R == 6 || R == 8 || R == 10, "radix");
+        float2 e[H], o[H];
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            e[i] = x[2 * i];
+            o[i] = x[2 * i + 1];
+        }
+        dft<H>(e, s);
+        dft<H>(o, s);
+        constexpr float r2 = 0.707106781186547524f, r3 = 0.866025403784438647f;
+        constexpr float wc[5] = {1.f, R == 6 ? 0.5f : R == 8 ? r2 : 0.809016994374947424f,
+                                 R == 6 ? -0.5f : R == 8 ? 0.f : 0.309016994374947424f,
+                                 R == 8 ? -r2 : -0.309016994374947424f, -0.809016994374947424f};
+        constexpr float ws[5] = {0.f, R == 6 ? r3 : R == 8 ? r2 : 0.587785252292473129f,
+                                 R == 6 ? r3 : R == 8 ? 1.f : 0.951056516295153572f,
+                                 R == 8 ? r2 : 0.951056516295153572f, 0.587785252292473129f};
+#pragma unroll
+        for (int i = 0; i < H; ++i) {
+            const float2 t = i == 0               ? o[0]
+                             : (R == 8 && i == 2) ? make_float2(-s * o[2].y, s * o[2].x)
+                                                  : cmul(o[i], make_float2(wc[i], s * ws[i]));
+            x[i] = e[i] + t;
+            x[i + H] = e[i] - t;
+        }
+    }
+}
+
+// A tile's place in memory: element n of row q at base + n step + q pitch.
+struct tile_at {
+    char *base;
+    int64_t step;                               // bytes, as pitch
+    uint32_t pitch;
+    int rows;                                   // rows of the tile that exist
+};
+
+// crop position of output k (fftshifted if asked) or -1
+__device__ __forceinline__ int crop_pos(int k, int N, int rc, int shift)
+{
+    const int kp = (shift ? (k < N / 2 ? k + N / 2 : k - N / 2) : k) - (N - rc) / 2;
+    return kp >= 0 && kp < rc ? kp : -1;
+}
+
+// Where the last pass leaves the sum of squares of its coils: rc kept outputs
+// of its axis at out + k' outK, one element a kept column.  The arithmetic
+// and the order of k_sos (fr_image.hip).
+struct sos_out {
+    float *acc;                                 // LDS [rc][TC]
+    float *out;
+    const float *deapod;
+    int64_t coil, outK;
+    int C, rc, shift;
+    int rcx, rcy;                               // columns kept: x and, in 3D, y
+};
+
+// An element of a row in LDS.  Rows: one after the
+// other, an element of padding after every eighth (the first stage writes at
+// a stride of its radix); columns: side by side.
+template <bool ROWS>
+__device__ __forceinline__ int lds_at(const fft_desc &d, int n, int row)
+{
+    return ROWS ? row * d.pitch + n + (n >> 3) : (n << d.ltc) + row;
+}
+
+// Stage i for the whole tile, NB butterflies a thread.  ROWS: rows lie one
+// after the other (step 1) and lanes run along a row; otherwise they lie side
+// by side (pitch 1) and lanes run across them.  Memory addresses are a
+// uniform base for each input (output) of the butterflies and one offset a
+// butterfly, below 2^32 bytes.
+template <int R, bool ROWS, int NB, bool SOS>
+__device__ __forceinline__ void stage(const fft_desc &d, int i, const tile_at &t, float2 *buf, float2 *tw,
+                                      const float2 *__restrict__ gtw, float s, const sos_out &o)
+{
+    const stage_desc &g = d.st[i];
+    const bool first = i == 0, last = i == d.stages - 1;
+    const int total = g.nb << d.ltc;
+    float2 x[NB][R];
+    int row[NB], j[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int q = threadIdx.x + b * blockDim.x;
+        if (ROWS) {
+            row[b] = (int)quot(q, g.m_nb);
+            j[b] = q - row[b] * g.nb;
+        } else {
+            row[b] = q & ((1 << d.ltc) - 1);
+            j[b] = q >> d.ltc;
+        }
+        if (q >= total || row[b] >= t.rows) row[b] = -1;
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (row[b] < 0) continue;
+        if (first) {
+            const uint32_t off = (uint32_t)j[b] * (uint32_t)t.step + (uint32_t)row[b] * t.pitch;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                x[b][r] = *reinterpret_cast<const float2 *>(t.base + r * (g.nb * t.step) + off);
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[b][r] = buf[lds_at<ROWS>(d, j[b] + r * g.nb, row[b])];
+        }
+    }
+    // the table on its way behind the first inputs; otherwise all reads before the writes below
+    if (first)
+        for (int q = threadIdx.x; q < d.N; q += blockDim.x) tw[q] = gtw[q];
+    else
+        __syncthreads();
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        if (row[b] < 0) continue;
+        const int jq = (int)quot(j[b], g.m_ns), jm = j[b] - jq * g.Ns;
+        if (!first) {
+#pragma unroll
+            for (int r = 1; r < R; ++r) x[b][r] = cmul(x[b][r], tw[r * jm * g.step]);
+        }
+        dft<R>(x[b], s);
+        const int n = jq * g.Ns * R + jm;
+        if (last) {
+            const uint32_t off = (uint32_t)n * (uint32_t)t.step + (uint32_t)row[b] * t.pitch;
+#pragma unroll
+            for (int r = 0; r < R; ++r) *reinterpret_cast<float2 *>(t.base + r * (g.Ns * t.step) + off) = x[b][r];
+            if constexpr (SOS) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int kp = crop_pos(n + r * g.Ns, d.N, o.rc, o.shift);
+                    if (kp >= 0) {              // the same thread for every coil
+                        float &a = o.acc[(kp << d.ltc) + row[b]];
+                        a = __fadd_rn(a, __fadd_rn(__fmul_rn(x[b][r].x, x[b][r].x), __fmul_rn(x[b][r].y, x[b][r].y)));
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) buf[lds_at<ROWS>(d, n + r * g.Ns, row[b])] = x[b][r];
+        }
+    }
+    if (!last) __syncthreads();
+}
+
+template <bool ROWS, int NB, bool SOS>
+__device__ __forceinline__ void transform(const fft_desc &d, const tile_at &t, float2 *buf, float2 *tw,
+                                          const float2 *__restrict__ gtw, float s, const sos_out &o)
+{
+    for (int i = 0; i < d.stages; ++i)
+        switch (d.st[i].R) {                    // the barrier after stage 0 also covers the twiddles
+        case 2: stage<2, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        case 3: stage<3, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        case 4: stage<4, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        case 5: stage<5, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        case 6: stage<6, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        case 7: stage<7, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        case 8: stage<8, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        default: stage<10, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        }
+}
+
+// Rows (ROWS): `count` rows of N, tile T the rows from T TC.  Columns: planes
+// of count columns, N apart by `step`; tile T the columns from (T mod tiles)
+// TC of plane T / tiles, planes `plane` elements apart.  SOS: the one plane of
+// each coil in turn, then the image.
+template <bool ROWS, int NB, bool SOS>
+__global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 6 : 4))) k_fft(
+    float2 *data, const float2 *__restrict__ gtw, fft_desc d, int64_t count, uint32_t tiles, uint32_t all, int64_t step,
+    int64_t plane, float s, sos_out o)
+{
+    extern __shared__ float2 sm[];              // twiddles [N], tile, sums
+    float2 *buf = sm + d.N;
+    // a compact eighth of the tiles for each XCD (workgroups go to them in
+    // turn): what fits an XCD's L2 is still there for the next axis (8 x
+    // 512^2: x and y pass together 31 -> 23 us, 8 x 320^2 24 -> 15)
+    const uint32_t T = (blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (T >= all) return;
+    const uint32_t P = ROWS ? 0u : T / tiles;
+    const int64_t q0 = (int64_t)(T - P * tiles) << d.ltc;
+    tile_at t;
+    t.base = reinterpret_cast<char *>(ROWS ? data + q0 * d.N : data + P * plane + q0);
+    t.step = 8 * (ROWS ? 1 : step);
+    t.pitch = 8u * (ROWS ? (uint32_t)d.N : 1u);
+    t.rows = (int)min((int64_t)1 << d.ltc, count - q0);
+    if constexpr (!SOS) {
+        transform<ROWS, NB, false>(d, t, buf, sm, gtw, s, o);
+    } else {
+        o.acc = reinterpret_cast<float *>(buf + ((size_t)d.N << d.ltc));
+        for (int i = threadIdx.x; i < o.rc << d.ltc; i += blockDim.x) o.acc[i] = 0.f;
+        for (int c = 0; c < o.C; ++c) {         // (two stages or more: a barrier before the first use of acc)
+            transform<ROWS, NB, true>(d, t, buf, sm, gtw, s, o);
+            t.base += 8 * o.coil;
+            __syncthreads();
+        }
+        for (int i = threadIdx.x; i < o.rc << d.ltc; i += blockDim.x) {
+            const int kp = i >> d.ltc, row = i & ((1 << d.ltc) - 1);
+            if (row >= t.rows) continue;
+            const uint32_t col = (uint32_t)q0 + row, y = col / (uint32_t)d.N;       // (2D: y = 0)
+            const int xp = crop_pos((int)(col - y * d.N), d.N, o.rcx, o.shift);
+            const int yp = count > d.N ? crop_pos((int)y, d.N, o.rcy, o.shift) : 0;
+            if (xp < 0 || yp < 0) continue;
+            const int64_t at = kp * o.outK + (int64_t)yp * o.rcx + xp;
+            float m = sqrtf(o.acc[i]);
+            if (o.deapod) m = __fdiv_rn(m, o.deapod[at]);
+            o.out[at] = m;
+        }
+    }
+}
+
+// The fewest stages, then the largest least radix; odd radices first (the
+// first stage's LDS writes go at a stride of the radix along a row).
+void search(int n, int least, int *cur, int depth, int *best, int &best_depth, int &best_min)
+{
+    if (n == 1) {
+        const int mn = depth ? cur[0] : 0;      // radices ascend
+        if (depth > 0 && (best_depth == 0 || depth < best_depth || (depth == best_depth && mn > best_min))) {
+            best_depth = depth;
+            best_min = mn;
+            std::copy(cur, cur + depth, best);
+        }
+        return;
+    }
+    if (depth == MAX_STAGES) return;
+    for (int r : {2, 3, 4, 5, 6, 7, 8, 10})
+        if (r >= least && n % r == 0) {
+            cur[depth] = r;
+            search(n / r, r, cur, depth + 1, best, best_depth, best_min);
+        }
+}
+
+constexpr uint32_t magic(uint32_t d) { return d > 1 ? (uint32_t)(((uint64_t(1) << 32) + d - 1) / d) : 0u; }
+
+// radices of N: false if it has other factors, a single stage (whose inputs
+// and outputs would share no barrier) or rows too long for a tile of 8
+bool plan(int N, fft_desc &d)
+{
+    if (N < 8 || N > 1024) return false;
+    int cur[MAX_STAGES], best[MAX_STAGES], n = 0, mn = 0;
+    search(N, 2, cur, 0, best, n, mn);
+    if (n < 2) return false;
+    std::stable_sort(best, best + n, [](int a, int b) { return (a & 1) > (b & 1); });
+    d.N = N;
+    d.stages = n;
+    d.pitch = N + N / 8 + 1;
+    d.nbmax = 0;
+    int Ns = 1;
+    for (int i = 0; i < n; ++i) {
+        const int R = best[i], nb = N / R;
+        d.st[i] = stage_desc{R, nb, Ns, N / (R * Ns), magic(nb), magic(Ns)};
+        d.nbmax = std::max(d.nbmax, nb);
+        Ns *= R;
+    }
+    return d.nbmax * 8 <= 2 * MAX_THREADS;
+}
+
+template <bool ROWS>
+fr_status pass(fr_fft *f, float2 *data, int64_t planes, int64_t count, int64_t step,
+               int64_t plane, const sos_out *sos = nullptr)
+{
+    fr_ctx *ctx = f->ctx;
+    fft_desc d = f->desc;
+    // rows a tile: at most 16 (128-byte runs) and two butterflies a thread;
+    // fewer, down to 4, for one tile a CU, and along x, where that breaks no
+    // runs, for four.  At 8 x 512^2 and 16, 8, 4 rows: x 13.1, 13.3, 11.1 us,
+    // y 14.2, 17.1, 20.2; 4 x 240^2 at 4 against 2 rows: y 7.6, 9.0.
+    d.ltc = 4;
+    while (d.nbmax << d.ltc > 2 * MAX_THREADS) --d.ltc;
+    auto tiles = [&] { return (count + (1 << d.ltc) - 1) >> d.ltc; };
+    while (d.ltc > 2 && planes * tiles() < (ROWS ? 4 : 1) * ctx->cu_count) --d.ltc;
+    const int work = d.nbmax << d.ltc, each = work > MAX_THREADS ? 2 : 1, threads = ((work + each - 1) / each + 63) & ~63;
+    const size_t lds = sizeof(float2) * (d.N + ((size_t)(ROWS ? d.pitch : d.N) << d.ltc)) +
+                       (sos ? sizeof(float) * ((size_t)sos->rc << d.ltc) : 0);
+    const int64_t W = planes * tiles();
+    FR_CHECK(ctx, W < (int64_t(1) << 31), FR_ERR_UNSUPPORTED, "FFT launch of %lld workgroups", (long long)W);
+    auto kern = each == 1 ? k_fft<ROWS, 1, false> : k_fft<ROWS, 2, false>;
+    if constexpr (!ROWS)
+        if (sos) kern = each == 1 ? k_fft<ROWS, 1, true> : k_fft<ROWS, 2, true>;
+    if (lds > 65536)
+        FR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(kern, dim3((unsigned)((W + 7) / 8 * 8)), dim3(threads), lds, ctx->stream, data, f->tw, d, count,
+                       (uint32_t)tiles(), (uint32_t)W, step, plane, (float)f->sign, sos ? *sos : sos_out{});
+    FR_HIP(ctx, hipGetLastError());
+    return FR_OK;
+}
+
+}  // namespace
+
+// Whether f's size is transformed here; lays out its stages.
+bool fr_fft_radices(fr_fft *f)
+{
+    // (a grid below 2^32 bytes: 32-bit offsets)
+    return f->N <= (f->dim == 3 ? 800u : 1024u) && plan((int)f->N, f->desc);
+}
+
+// The grids of f's batch, in place; f->tw is set.  With an image (sum of
+// squares over the C coils of one grid each, kept outputs rcx x rcy x rcz),
+// the last pass takes a tile's coils in turn and forms it.
+static fr_status passes(fr_fft *f, float2 *data, const sos_out *sos)
+{
+    const int64_t N = f->N, B = f->batch, last = sos ? 1 : B;
+    fr_status e = pass<true>(f, data, 1, B * N * (f->dim == 3 ? N : 1), 1, 0);
+    if (!e && f->dim == 3) e = pass<false>(f, data, B * N, N, N, N * N);
+    if (!e) e = f->dim == 3 ? pass<false>(f, data, last, N * N, N * N, N * N * N, sos)
+                            : pass<false>(f, data, last, N, N, N * N, sos);
+    return e;
+}
+
+fr_status fr_fft_passes(fr_fft *f, float2 *data) { return passes(f, data, nullptr); }
+
+// Whether the image comes out of the last pass: for one coil (96^2: 6.1 us
+// against 4.9 and 2.6 for k_sos and a launch).  Several coils would go one
+// after the other, nothing loaded ahead: 5 x 180^3 145 us against 96 and 12.
+bool fr_fft_sos_last(const fr_fft *f, const fr_grids *g) { return f->own && g->frames == 0 && g->C == 1; }
+
+fr_status fr_fft_passes_sos(fr_fft *f, const fr_grids *g, int rcx, int rcy, int rcz, int shift, const float *deapod,
+                            float *out)
+{
+    sos_out o{};
+    o.out = out;
+    o.deapod = deapod;
+    o.C = g->C;
+    o.coil = (int64_t)g->cells;
+    o.rc = g->dim == 3 ? rcz : rcy;
+    o.outK = g->dim == 3 ? (int64_t)rcy * rcx : rcx;
+    o.rcx = rcx;
+    o.rcy = rcy;
+    o.shift = shift;
+    return passes(f, g->data, &o);
+}

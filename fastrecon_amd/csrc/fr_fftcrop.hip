@@ -559,7 +559,10 @@ extern "C" fr_status fr_fft_sos(fr_fft *f, fr_grids *g, unsigned rcx, unsigned r
     FR_EXTENT(ctx, out_dev, sizeof(float) * rcx * rcy * rcz, "fr_fft_sos image");
     FR_EXTENT(ctx, deapod_dev, sizeof(float) * rcx * rcy * (g->dim == 3 ? rcz : 1u), "fr_fft_sos deapodisation map");
     if (!fr_fft_sos_fused(f, g, rcx, rcy, rcz)) {
-        // other sizes: the full batched FFT in place, then the fused epilogue
+        // other sizes: the full batched FFT in place, the image from its last
+        // pass or by the fused epilogue
+        if (fr_fft_sos_last(f, g))
+            return fr_fft_passes_sos(f, g, (int)rcx, (int)rcy, (int)rcz, apply_shift, deapod_dev, out_dev);
         fr_status e = fr_fft_execute(f, g);
         if (!e) e = fr_sos(ctx, g, rcx, rcy, rcz, apply_shift, deapod_dev, out_dev);
         return e;

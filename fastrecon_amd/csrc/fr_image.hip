@@ -1,4 +1,5 @@
-// Image stage: batched rocFFT over all coils, in-place fftshift, and the
+// Image stage: batched FFT over all coils (fr_fft.hip; rocFFT for the sizes it
+// does not take), in-place fftshift, and the
 // fused shift + crop + sum-of-squares (+ deapodisation) epilogue.
 #include "fr_internal.h"
 
@@ -83,11 +84,18 @@ extern "C" fr_status fr_fft_create(fr_ctx *ctx, int dim, unsigned N, int batch, 
     FR_CHECK(ctx, dim == 2 || dim == 3, FR_ERR_INVALID, "dim must be 2 or 3");
     FR_CHECK(ctx, batch >= 1, FR_ERR_INVALID, "batch must be >= 1");
     FR_CHECK(ctx, sign == 1 || sign == -1, FR_ERR_INVALID, "sign must be +1 or -1");
-    std::call_once(g_rocfft_once, [] { g_rocfft_setup = rocfft_setup(); });
-    FR_CHECK(ctx, g_rocfft_setup == rocfft_status_success, FR_ERR_LIBRARY, "rocfft_setup failed");
     fr_fft *f = new (std::nothrow) fr_fft;
     if (!f) return FR_ERR_NOMEM;
     f->ctx = ctx; f->dim = dim; f->N = N; f->batch = batch; f->sign = sign;
+    if (fr_fft_radices(f)) {
+        f->own = true;
+        const fr_status st = fr_fft_tw(f);
+        if (st) { fr_fft_destroy(f); return st; }
+        *out = f;
+        return FR_OK;
+    }
+    std::call_once(g_rocfft_once, [] { g_rocfft_setup = rocfft_setup(); });
+    if (g_rocfft_setup != rocfft_status_success) { delete f; return fr_fail(ctx, FR_ERR_LIBRARY, "rocfft_setup failed"); }
     size_t lengths[3] = {N, N, N};
     rocfft_plan plan = nullptr;
     rocfft_status rs = rocfft_plan_create(&plan, rocfft_placement_inplace,
@@ -131,6 +139,7 @@ extern "C" fr_status fr_fft_execute(fr_fft *f, fr_grids *g)
              FR_ERR_INVALID,
              "grids (dim %d, N %u, C %d) do not match the FFT plan (dim %d, N %u, batch %d)", g->dim, g->N, g->C,
              f->dim, f->N, f->batch);
+    if (f->own) return fr_fft_passes(f, g->data);
     void *bufs[1] = {g->data};
     rocfft_status rs = rocfft_execute((rocfft_plan)f->plan, bufs, nullptr, (rocfft_execution_info)f->info);
     FR_CHECK(ctx, rs == rocfft_status_success, FR_ERR_LIBRARY, "rocfft_execute: %d", (int)rs);

@@ -254,17 +254,35 @@ struct fr_plan {
     double build_ms = 0.0;
 };
 
+// Stages of an N-point transform (fr_fft.hip): radix R, nb = N / R butterflies
+// a row, Ns the product of the radices before it, step = N / (R Ns) twiddle
+// exponents per unit of j mod Ns; m_nb, m_ns for divisions by nb and Ns.
+constexpr int FR_FFT_STAGES = 6;
+struct fr_fft_desc {
+    struct stage {
+        int R, nb, Ns, step;
+        uint32_t m_nb, m_ns;
+    };
+    int N, stages, nbmax;           // nbmax: the largest nb
+    int ltc;                        // 1 << ltc rows a tile (set for a pass)
+    int pitch;                      // of a row in LDS (rows along x)
+    stage st[FR_FFT_STAGES];
+};
+
 struct fr_fft {
     fr_ctx *ctx = nullptr;
     int dim = 0;
     unsigned N = 0;
     int batch = 0;
     int sign = 1;
+    bool own = false;                  // transformed by fr_fft.hip; the others by rocFFT:
+    fr_fft_desc desc{};
     void *plan = nullptr;              // rocfft_plan
     void *info = nullptr;              // rocfft_execution_info
     void *work = nullptr;
     size_t work_bytes = 0;
-    // cropped FFT + SOS path (fr_fftcrop.hip): twiddles and pass buffers
+    // twiddles (fr_fft.hip and the cropped FFT + SOS path, fr_fftcrop.hip)
+    // and that path's pass buffers
     float2 *tw = nullptr;
     void *crop_ws = nullptr;
     size_t crop_ws_bytes = 0;
@@ -352,6 +370,13 @@ fr_status fr_tile_density(fr_plan *p, fr_samples *s, int iters, bool ones);
 // the no-allocation entry point's static scratch (fr_noalloc.hip): its
 // address on the context's device, looked up once per device
 fr_status fr_scratch_init(fr_ctx *ctx);
+// sizes that fr_fft.hip transforms, and its transform of f's batch of grids
+bool fr_fft_radices(fr_fft *f);
+fr_status fr_fft_passes(fr_fft *f, float2 *data);
+// the same, the last pass forming the sum-of-squares image as well
+bool fr_fft_sos_last(const fr_fft *f, const fr_grids *g);
+fr_status fr_fft_passes_sos(fr_fft *f, const fr_grids *g, int rcx, int rcy, int rcz, int shift, const float *deapod,
+                            float *out);
 // cropped FFT + SOS helpers (fr_fftcrop.hip)
 fr_status fr_fft_workspace(fr_fft *f, size_t bytes);
 // FR_ERR_INVALID unless [p, p + bytes) lies inside the device allocation of p

@@ -37,6 +37,8 @@ struct fr_ctx {
     std::string arch;          // gcnArchName up to the first ':' (e.g. gfx950)
     void *scratch = nullptr;   // this device's copy of the static scratch (fr_noalloc.hip)
     fr_pool pool;
+    std::mutex low_m;
+    float *low = nullptr;      // the low filter's coefficients (fr_image.hip), made on first use
 };
 
 struct fr_samples {

@@ -224,13 +224,18 @@ __device__ __forceinline__ void lane_cell(const item_box &b, int j, float &fx, f
 // instructions and return traffic of these.)  Software pipeline: while batch
 // b is applied, batch b + 1's rows, the next block's positions and the block
 // after's indices are in flight (past the last record they read the next
-// records or the FR_POS_PAD padding records at the end).  Bound by VALU issue
-// (about 27 instructions per four records beside the matrix ones: VALU busy
-// 60% and matrix cores 31% at 16 FP16 coils on 384^3) and, at 32 coils, by
-// the traffic of the rows past L2 as well.  32 coils at 256^3: 4.71 -> 4.13 ms
-// in all; 16 FP16 coils at 384^3: 7.75 -> 7.12.  Rows fetched two or three
-// batches ahead were slower (the extra ones past an item's end cost as much
-// as useful ones): 8.1 and 8.5 ms there.
+// records or the FR_POS_PAD padding records at the end).  Bound by the
+// latency of a batch's chain (row loads, table reads, matrix products) over
+// the waves that fit a SIMD, and at 32 coils by the traffic of the rows past
+// L2 as well: up to 16 coils, where six waves fit instead of five (a wave's
+// records and its write-out share their LDS, 80 VGPRs), 16 FP16 coils at
+// 384^3 went from 7.00 to 6.69 ms and 12 coils of 64 frames on 384^2 from
+// 1.19 to 1.13, while a third fewer VALU instructions a weight (squared
+// distances along each axis formed once a record) gained nothing: 7.01.  By
+// blocks at all: 32 coils at 256^3 4.71 -> 4.13 ms (now 4.06), 16 FP16 coils
+// at 384^3 7.75 -> 7.12.  Rows fetched two or three batches ahead were slower
+// (the extra ones past an item's end cost as much as useful ones): 8.1 and
+// 8.5 ms there.
 template <int NCB, bool PAIR, bool SMALL, typename TS, typename After>
 __device__ __forceinline__ void grid_stream(f4 (&acc)[NCB], uint32_t r, const uint32_t *__restrict__ recs,
                                             const float4 *__restrict__ pos, const TS *__restrict__ data, uint32_t C,
@@ -312,20 +317,22 @@ __device__ __forceinline__ void grid_records_mid(f4 (&acc)[NCB], uint32_t r, uin
 //  * otherwise a run of ipw consecutive light items per wave, as one
 //    record stream, each unit written out by its wave.
 template <int NCB, bool PAIR, bool SMALL, typename TS, int OCC>
-__global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OCC, 8))) k_grid_pos(
+__global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OCC == 4 && NCB <= 2 ? 6 : OCC, 8))) k_grid_pos(
     const fr_item *__restrict__ items, int64_t nitems, const fr_tile *__restrict__ tiles, int64_t ntiles,
     int lbx, int lby, int lbz, const uint32_t *__restrict__ recs, const float4 *__restrict__ pos,
     const float4 *__restrict__ tbl, int L, float cidx, const TS *__restrict__ data,
     int C, int N, size_t cells, float2 *__restrict__ out, float2 *__restrict__ partial,
     int64_t nslots, int cells_max, int64_t nfront, int64_t front_wg, int ipw, int64_t xr, int nt, int tw,
-    int osm_floats, int64_t tstride, int fsub)
+    int wave_floats, int64_t tstride, int fsub)
 {
     extern __shared__ float4 smem_pos[];
     float4 *stbl = smem_pos;                                         // L entries
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    float4 *pbuf = smem_pos + L + wv * 64;                           // the wave's block of positions
-    float *osm = reinterpret_cast<float *>(smem_pos + L + PW * 64) + wv * osm_floats;
+    // the wave's block of positions and, after them (its LDS instructions stay
+    // in order), its write-out transpose in the same place
+    float4 *pbuf = smem_pos + L + wv * (wave_floats / 4);
+    float *osm = reinterpret_cast<float *>(pbuf);
     for (int q = threadIdx.x; q < L; q += 64 * PW) stbl[q] = tbl[q];
     __syncthreads();
 
@@ -358,7 +365,7 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
         const int32_t myitem = wv == 0 ? T.item[0] : wv == 1 ? T.item[1] : wv == 2 ? T.item[2] : T.item[3];
         const int bx = 1 << lbx, by = 1 << lby;
         const int W = PW * bx, rows = by << lbz;    // tile row length, rows per coil
-        float *tb = reinterpret_cast<float *>(smem_pos + L + PW * 64);
+        float *tb = reinterpret_cast<float *>(smem_pos + L) + PW * wave_floats;
         const int cstride = rows * W * 2 + 4;       // floats per coil (+4: fewer bank conflicts)
         if (myitem >= 0) {
             const fr_item it = items[myitem];
@@ -607,7 +614,10 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, 
     // per wave: the write-out transpose (16 cells x 16 NCB components, or a
     // step of a pair; a tile of four needs less from its four waves together)
     const int osm_floats = std::max(16 * NCB * CS, (NCB == 1 ? 8 : 16) * PS);
-    const size_t lds = sizeof(float4) * (p->L + PW * 64) + sizeof(float) * PW * osm_floats;
+    // in the place of the block of positions before it; a tile of four, whose
+    // waves write each other's cells, has its own
+    const int wave_floats = std::max(64 * 4, osm_floats);
+    const size_t lds = sizeof(float4) * p->L + sizeof(float) * PW * (wave_floats + (fours ? osm_floats : 0));
     auto kern = k_grid_pos<NCB, PAIR, SMALL, TS, OCC>;
     FR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int lbx = __builtin_ctz((unsigned)p->geom.bx), lby = __builtin_ctz((unsigned)p->geom.by),
@@ -616,7 +626,7 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, 
                        p->tiles, p->ntiles, lbx, lby, lbz, p->recs, p->pos, p->tsel, p->L, p->mfma_cidx,
                        (const TS *)s->data, s->C, (int)p->N, cells, out, partial, p->nslots,
                        p->geom.cells_max, p->nitems_front, front_wg, ipw, xr, p->pos_stores == 1 ? 1 : 0,
-                       p->tile_units, osm_floats, tstride, tstride > 1 ? fsub : 1);
+                       p->tile_units, wave_floats, tstride, tstride > 1 ? fsub : 1);
     FR_HIP(ctx, hipGetLastError());
     return FR_OK;
 }

@@ -145,7 +145,6 @@ extern "C" fr_status fr_ctx_destroy(fr_ctx *ctx)
         std::lock_guard<std::mutex> lock(ctx->pool.m);
         pool_trim(ctx->pool, 0);
     }
-    hipFree(ctx->low);
     hipStreamDestroy(ctx->stream);
     delete ctx;
     return FR_OK;

@@ -333,29 +333,6 @@ __global__ void k_sos_map(const float2 *__restrict__ g, const float2 *__restrict
     out[i] = make_float2(ar, ai);
 }
 
-// The filter's coefficients, the same for every call, exactly as the
-// reference's host loop has them: expf(-r / 100.0).  Uploaded once a context.
-fr_status lowfilter_table(fr_ctx *ctx, const float **out)
-{
-    std::lock_guard<std::mutex> lock(ctx->low_m);
-    if (!ctx->low) {
-        float coeff[2000];
-        for (int r = 0; r < 2000; ++r) coeff[r] = expf((float)(-r / 100.0));
-        float *d = nullptr;
-        const fr_status st = fr_alloc(ctx, (void **)&d, sizeof coeff);
-        if (st) return st;
-        hipError_t e = hipMemcpyAsync(d, coeff, sizeof coeff, hipMemcpyHostToDevice, ctx->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-        if (e != hipSuccess) {
-            (void)hipFree(d);
-            return fr_fail(ctx, FR_ERR_HIP, "lowFilter: %s", hipGetErrorString(e));
-        }
-        ctx->low = d;
-    }
-    *out = ctx->low;
-    return FR_OK;
-}
-
 }  // namespace
 
 extern "C" fr_status fr_lowfilter(fr_ctx *ctx, fr_grids *g, int res)
@@ -363,13 +340,21 @@ extern "C" fr_status fr_lowfilter(fr_ctx *ctx, fr_grids *g, int res)
     if (!ctx || !g) return FR_ERR_INVALID;
     FR_CHECK(ctx, g->frames == 0, FR_ERR_UNSUPPORTED, "not available for batched frames");
     FR_CHECK(ctx, res > 0, FR_ERR_INVALID, "lowFilter resolution must be positive");
+    // coefficients exactly as the reference's host loop: expf(-r / 100.0)
+    float coeff[2000];
+    for (int r = 0; r < 2000; ++r) coeff[r] = expf((float)(-r / 100.0));
     const float att = (float)(2.0 * res * res / 4.0);
-    const float *coeff = nullptr;
-    const fr_status st = lowfilter_table(ctx, &coeff);
+    float *dc = nullptr;
+    fr_status st = fr_alloc(ctx, (void **)&dc, sizeof coeff);
     if (st) return st;
-    hipLaunchKernelGGL(k_lowfilter, dim3(nblk(g->cells, 256)), dim3(256), 0, ctx->stream, g->data, g->dim, (int)g->N,
-                       g->C, g->cells, att, coeff);
-    FR_HIP(ctx, hipGetLastError());
+    hipError_t e = hipMemcpyAsync(dc, coeff, sizeof coeff, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_lowfilter, dim3(nblk(g->cells, 256)), dim3(256), 0, ctx->stream, g->data, g->dim, (int)g->N,
+                           g->C, g->cells, att, dc);
+        e = hipStreamSynchronize(ctx->stream);
+    }
+    hipFree(dc);
+    FR_CHECK(ctx, e == hipSuccess, FR_ERR_HIP, "lowFilter: %s", hipGetErrorString(e));
     return FR_OK;
 }
 

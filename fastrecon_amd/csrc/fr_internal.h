@@ -18,9 +18,10 @@
 // hipFree of a plan's buffers cost more than the kernels that fill them.  One
 // per context; all its users' work is on the context's stream, so a block may
 // be handed out again as soon as it is given back.  At most FR_POOL_BYTES
-// stay in it (the oldest go first); all of it is freed when an allocation
-// fails and with the context.
-constexpr size_t FR_POOL_BYTES = size_t(2) << 30;
+// stay in it (the oldest go first; a plan of 13.1M samples on 256^3 takes 2.7
+// GB while it is built); all of it is freed when an allocation fails and with
+// the context.
+constexpr size_t FR_POOL_BYTES = size_t(4) << 30;
 struct fr_pool {
     struct block { void *p; size_t bytes; };
     std::mutex m;
@@ -37,8 +38,6 @@ struct fr_ctx {
     std::string arch;          // gcnArchName up to the first ':' (e.g. gfx950)
     void *scratch = nullptr;   // this device's copy of the static scratch (fr_noalloc.hip)
     fr_pool pool;
-    std::mutex low_m;
-    float *low = nullptr;      // the low filter's coefficients (fr_image.hip), made on first use
 };
 
 struct fr_samples {

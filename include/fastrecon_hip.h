@@ -213,12 +213,17 @@ fr_status fr_grid_execute_noalloc(fr_plan *p, const fr_samples *s, fr_grids *out
 /* Degridding (grid -> samples), the adjoint of fr_grid_execute with the
  * same taps, no DCF.  Net-new (the reference has none).  s supplies the
  * trajectory the plan was built on; out: device complex64, sample-major
- * [M][g->C]. */
+ * [M][g->C].  A position-weight plan whose kernel is at most 4 cells wide
+ * orders its samples by grid tile on the first large call (not during a
+ * capture; or on the first fr_dcf_pipe_menon) and keeps that order, about 16
+ * bytes a sample, until fr_plan_destroy. */
 fr_status fr_degrid_execute(fr_plan *p, const fr_samples *s, const fr_grids *g, void *out_dev);
 
 /* -------------------------------------------------------------------- FFT */
 /* Replaces cuFFT (ImageFilter/cuFFT.cpp:15-37) and FFT (FFT.cpp:30-91):
- * one batched in-place C2C rocFFT plan over all coils, unnormalised.
+ * one batched in-place C2C transform over all coils, unnormalised: sizes of
+ * factors 2, 3, 5 and 7 up to 1024 (3D 800) by kernels of this library, the
+ * others by rocFFT.
  * sign +1 is FFTW_BACKWARD / CUFFT_INVERSE, the reference default. */
 fr_status fr_fft_create(fr_ctx *ctx, int dim, unsigned N, int batch, int sign, fr_fft **out);
 fr_status fr_fft_destroy(fr_fft *f);
@@ -270,10 +275,12 @@ fr_status fr_deapod_map(fr_ctx *ctx, int dim, unsigned N, float kWidth, const fl
 /* --------------------------------------------------- density compensation */
 /* Pipe-Menon iterative DCF (net-new): w <- w / G^H G w, `iters` times,
  * starting from the samples' current DCF (or 1 if init_ones), written back
- * to the samples' DCF.  Uses this plan's gridding and degridding kernels.
- * The first call (of this or fr_dcf_identity_scale) gives the plan a
- * single-channel workspace (the trajectory, unit data, one grid, M complex
- * densities) that it keeps until fr_plan_destroy. */
+ * to the samples' DCF.  The first call gives the plan a workspace that it keeps
+ * until fr_plan_destroy: on a position-weight plan with a kernel of at most 4
+ * cells, and samples still on the plan's trajectory, the samples in tile order
+ * with a density each, a real grid and a box of sums per work item; otherwise
+ * (and for fr_dcf_identity_scale) the trajectory, unit data, one grid and M
+ * complex densities, with this plan's gridding and degridding kernels. */
 fr_status fr_dcf_pipe_menon(fr_plan *p, fr_samples *s, int iters, int init_ones);
 
 /* Global scale of the samples' DCF (net-new) from the Pipe-Menon fixed-point

@@ -81,8 +81,9 @@ __device__ __forceinline__ float4 ld_pair(const __half2 *__restrict__ row, int c
     return make_float4(a.x, a.y, b.x, b.y);
 }
 
-// element at a 32-bit byte offset from a uniform base (the record, position
-// and DCF arrays stay below 4 GiB: at most 2^27 samples)
+// element at a 32-bit byte offset from a uniform base: positions (at most 2^27
+// samples, 2 GiB), or the records of a stream, from its first one on (a plan's
+// records take up to 16 GiB)
 template <typename E>
 __device__ __forceinline__ E ld_off(const E *__restrict__ base, uint32_t byte_off)
 {
@@ -213,8 +214,9 @@ __device__ __forceinline__ void lane_cell(const item_box &b, int j, float &fx, f
     }
 }
 
-// Grid the records [r, ..) into acc, batch by batch, until after_batch(r),
-// called with the position past the batch just applied, returns false.
+// Grid the records from recs[0] on into acc, batch by batch, until
+// after_batch(r), called with the number of records applied so far (below
+// 2^30), returns false.
 //
 // Records come in blocks of 64, one per lane: one load brings a block's
 // sample indices and one its positions and DCFs, which go through LDS (pbuf,
@@ -237,13 +239,14 @@ __device__ __forceinline__ void lane_cell(const item_box &b, int j, float &fx, f
 // (the extra ones past an item's end cost as much as useful ones): 8.1 and
 // 8.5 ms there.
 template <int NCB, bool PAIR, bool SMALL, typename TS, typename After>
-__device__ __forceinline__ void grid_stream(f4 (&acc)[NCB], uint32_t r, const uint32_t *__restrict__ recs,
+__device__ __forceinline__ void grid_stream(f4 (&acc)[NCB], const uint32_t *__restrict__ recs,
                                             const float4 *__restrict__ pos, const TS *__restrict__ data, uint32_t C,
                                             int ca, int cbb, const float4 *stbl, float4 *pbuf, float &fx, float &fy,
                                             float &fz, float cidx, float lmax, int j,
                                             int k, After after_batch)
 {
     const uint32_t lane = (uint32_t)(16 * k + j);
+    uint32_t r = 0;
     const uint32_t id = ld_off(recs, (r + lane) * 4u);
     uint32_t id1 = ld_off(recs, (r + 64 + lane) * 4u);
     float4 P = ld_off(pos, id * 16u);
@@ -284,7 +287,9 @@ __device__ __forceinline__ void grid_records(f4 (&acc)[NCB], uint32_t r, uint32_
                                              const float4 *stbl, float4 *pbuf, float fx, float fy, float fz,
                                              float cidx, float lmax, int j, int k)
 {
-    grid_stream<NCB, PAIR, SMALL>(acc, r, recs, pos, data, C, ca, cbb, stbl, pbuf, fx, fy, fz, cidx, lmax, j, k, [&](uint32_t q) __attribute__((always_inline)) { return q < r1; });
+    const uint32_t n = r1 - r;
+    grid_stream<NCB, PAIR, SMALL>(acc, recs + r, pos, data, C, ca, cbb, stbl, pbuf, fx, fy, fz, cidx, lmax, j, k,
+                                  [&](uint32_t q) __attribute__((always_inline)) { return q < n; });
 }
 
 // grid_records over [r, r1) with a switch at rmid (a multiple of RB): the
@@ -298,10 +303,12 @@ __device__ __forceinline__ void grid_records_mid(f4 (&acc)[NCB], uint32_t r, uin
                                                  const float4 *stbl, float4 *pbuf, float &fx, float &fy, float &fz,
                                                  float cidx, float lmax, int j, int k, Mid on_mid)
 {
-    grid_stream<NCB, PAIR, SMALL>(acc, r, recs, pos, data, C, ca, cbb, stbl, pbuf, fx, fy, fz, cidx, lmax, j, k, [&](uint32_t q) __attribute__((always_inline)) {
-                                     if (q == rmid) on_mid();
-                                     return q < r1;
-                                 });
+    const uint32_t mid = rmid - r, n = r1 - r;
+    grid_stream<NCB, PAIR, SMALL>(acc, recs + r, pos, data, C, ca, cbb, stbl, pbuf, fx, fy, fz, cidx, lmax, j, k,
+                                  [&](uint32_t q) __attribute__((always_inline)) {
+                                      if (q == mid) on_mid();
+                                      return q < n;
+                                  });
 }
 
 // NCB component blocks (chunks of 8 NCB coils).  PAIR: C even, so lane j's

@@ -433,7 +433,9 @@ fr_status fr_plan_build_pos(fr_plan *p, const fr_samples *s, const fr_tune *tune
     const int cus = std::max(1, ctx->cu_count);
     uint64_t S = std::min<uint64_t>(16384, std::max<uint64_t>(64, R / ((uint64_t)cus * 32)));
     if (tune && tune->split_taps > 0) S = (uint64_t)tune->split_taps;
-    S = std::min<uint64_t>((S + 15) / 16 * 16, uint64_t(1) << 30);
+    // (at most 2^25: the gridding kernel counts a wave's records in 32-bit
+    // byte offsets, of a slice or of up to 64 units below the heavy cut)
+    S = std::min<uint64_t>((S + 15) / 16 * 16, uint64_t(1) << 25);
     const uint32_t heavy_cut = (uint32_t)std::max<uint64_t>(4, S / 4);
 
     // 2. records by box, in sample order

@@ -39,69 +39,110 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b)
 {
     return make_float2(__builtin_fmaf(a.x, b.x, -(a.y * b.y)), __builtin_fmaf(a.x, b.y, a.y * b.x));
 }
-// a + b c, c real
-__device__ __forceinline__ float2 axpy(float2 a, float2 b, float c)
+// A butterfly's constant: its FP32 rounding and the rest.  The rounding alone
+// is the same relative error (1.8e-8 for sqrt(3) / 2) at every element of
+// every stage, which an image of several coils does not average out as it
+// does the elements' own roundings.  By the transform alone, 5 coils on 180^3
+// are 4.3e-8 from FP64 with both parts and 5.2e-8 with the first one (rocFFT
+// 5.5e-8); 5 x 250^2 5.0e-8 and 8.2e-8.  It costs nothing there that can be
+// seen (up to 4% at sizes of radix 10).
+struct real2 {
+    float hi, lo;
+};
+__host__ __device__ constexpr real2 two(double c) { return {(float)c, (float)(c - (double)(float)c)}; }
+// a + b c
+__device__ __forceinline__ float fma2(float b, real2 c, float a)
 {
-    return make_float2(__builtin_fmaf(b.x, c, a.x), __builtin_fmaf(b.y, c, a.y));
+    if (__builtin_constant_p(c.lo) && c.lo == 0.f) return __builtin_fmaf(b, c.hi, a);
+    return __builtin_fmaf(b, c.hi, __builtin_fmaf(b, c.lo, a));
 }
-// a + s i b
-__device__ __forceinline__ float2 add_i(float2 a, float2 b, float s)
+__device__ __forceinline__ float mul2(float b, real2 c)
 {
-    return make_float2(__builtin_fmaf(-s, b.y, a.x), __builtin_fmaf(s, b.x, a.y));
+    if (__builtin_constant_p(c.lo) && c.lo == 0.f) return b * c.hi;
+    return __builtin_fmaf(b, c.hi, b * c.lo);
 }
+__device__ __forceinline__ float2 axpy(float2 a, float2 b, real2 c)
+{
+    return make_float2(fma2(b.x, c, a.x), fma2(b.y, c, a.y));
+}
+__device__ __forceinline__ float2 scale(float2 b, real2 c) { return make_float2(mul2(b.x, c), mul2(b.y, c)); }
+// a + i b c and a - i b c
+__device__ __forceinline__ float2 add_i(float2 a, float2 b, real2 c)
+{
+    return make_float2(fma2(-b.y, c, a.x), fma2(b.x, c, a.y));
+}
+__device__ __forceinline__ float2 sub_i(float2 a, float2 b, real2 c)
+{
+    return make_float2(fma2(b.y, c, a.x), fma2(-b.x, c, a.y));
+}
+// a (c + i d)
+__device__ __forceinline__ float2 cmul(float2 a, real2 c, real2 d)
+{
+    return make_float2(fma2(a.x, c, mul2(-a.y, d)), fma2(a.x, d, mul2(a.y, c)));
+}
+// a + i b, a - i b
+__device__ __forceinline__ float2 add_i(float2 a, float2 b) { return make_float2(a.x - b.y, a.y + b.x); }
+__device__ __forceinline__ float2 sub_i(float2 a, float2 b) { return make_float2(a.x + b.y, a.y - b.x); }
 
-// R-point DFTs with w = exp(s 2 pi i / R), in place, natural order
-template <int R>
-__device__ __forceinline__ void dft(float2 (&x)[R], float s)
+// R-point DFTs with w = exp(S 2 pi i / R), S = 1 or -1, in place, natural order
+template <int R, int S>
+__device__ __forceinline__ void dft(float2 (&x)[R])
 {
     if constexpr (R == 2) {
         const float2 a = x[0], b = x[1];
         x[0] = a + b;
         x[1] = a - b;
     } else if constexpr (R == 3) {
-        const float2 p = x[1] + x[2], d = x[1] - x[2], m = axpy(x[0], p, -0.5f);
-        const float h = s * 0.866025403784438647f;
+        constexpr real2 r3 = two(0.86602540378443864676);
+        const float2 p = x[1] + x[2], d = S > 0 ? x[1] - x[2] : x[2] - x[1];
+        const float2 m = make_float2(__builtin_fmaf(p.x, -0.5f, x[0].x), __builtin_fmaf(p.y, -0.5f, x[0].y));
         x[0] = x[0] + p;
-        x[1] = add_i(m, d, h);
-        x[2] = add_i(m, d, -h);
+        x[1] = add_i(m, d, r3);
+        x[2] = sub_i(m, d, r3);
     } else if constexpr (R == 4) {
-        const float2 a = x[0] + x[2], b = x[0] - x[2], c = x[1] + x[3], d = x[1] - x[3];
+        const float2 a = x[0] + x[2], b = x[0] - x[2], c = x[1] + x[3], d = S > 0 ? x[1] - x[3] : x[3] - x[1];
         x[0] = a + c;
-        x[1] = add_i(b, d, s);
+        x[1] = add_i(b, d);
         x[2] = a - c;
-        x[3] = add_i(b, d, -s);
+        x[3] = sub_i(b, d);
     } else if constexpr (R == 5) {
-        constexpr float c1 = 0.309016994374947424f, c2 = -0.809016994374947424f;
-        constexpr float s1 = 0.951056516295153572f, s2 = 0.587785252292473129f;
-        const float2 p1 = x[1] + x[4], d1 = x[1] - x[4], p2 = x[2] + x[3], d2 = x[2] - x[3];
-        const float2 a = axpy(axpy(x[0], p1, c1), p2, c2), b = axpy(axpy(x[0], p1, c2), p2, c1);
-        const float2 u = axpy(make_float2(d1.x * s1, d1.y * s1), d2, s2);
-        const float2 v = axpy(make_float2(d1.x * s2, d1.y * s2), d2, -s1);
-        x[0] = x[0] + (p1 + p2);
-        x[1] = add_i(a, u, s);
-        x[4] = add_i(a, u, -s);
-        x[2] = add_i(b, v, s);
-        x[3] = add_i(b, v, -s);
+        // cos(2 pi / 5), cos(4 pi / 5) = -1/4 +- sqrt(5) / 4
+        constexpr real2 k = two(0.55901699437494742410), s1 = two(0.95105651629515357212), s2 = two(0.58778525229247312917);
+        constexpr real2 m1 = two(-0.95105651629515357212);
+        const float2 p1 = x[1] + x[4], p2 = x[2] + x[3], p = p1 + p2, t = scale(p1 - p2, k);
+        const float2 d1 = S > 0 ? x[1] - x[4] : x[4] - x[1], d2 = S > 0 ? x[2] - x[3] : x[3] - x[2];
+        const float2 m = make_float2(__builtin_fmaf(p.x, -0.25f, x[0].x), __builtin_fmaf(p.y, -0.25f, x[0].y));
+        const float2 a = m + t, b = m - t;
+        const float2 u = axpy(scale(d1, s1), d2, s2), v = axpy(scale(d1, s2), d2, m1);
+        x[0] = x[0] + p;
+        x[1] = add_i(a, u);
+        x[4] = sub_i(a, u);
+        x[2] = add_i(b, v);
+        x[3] = sub_i(b, v);
     } else if constexpr (R == 7) {
-        constexpr float c1 = 0.623489801858733531f, c2 = -0.222520933956314404f, c3 = -0.900968867902419126f;
-        constexpr float s1 = 0.781831482468029809f, s2 = 0.974927912181823607f, s3 = 0.433883739117558120f;
-        const float2 p1 = x[1] + x[6], d1 = x[1] - x[6], p2 = x[2] + x[5], d2 = x[2] - x[5], p3 = x[3] + x[4],
-                     d3 = x[3] - x[4];
-        auto even = [&](float a, float b, float c) __attribute__((always_inline)) {
+        constexpr real2 c1 = two(0.62348980185873353053), c2 = two(-0.22252093395631440429),
+                        c3 = two(-0.90096886790241912624);
+        constexpr real2 s1 = two(0.78183148246802980871), s2 = two(0.97492791218182360702),
+                        s3 = two(0.43388373911755812048);
+        constexpr real2 m1 = two(-0.78183148246802980871), m3 = two(-0.43388373911755812048);
+        const float2 p1 = x[1] + x[6], p2 = x[2] + x[5], p3 = x[3] + x[4];
+        const float2 d1 = S > 0 ? x[1] - x[6] : x[6] - x[1], d2 = S > 0 ? x[2] - x[5] : x[5] - x[2],
+                     d3 = S > 0 ? x[3] - x[4] : x[4] - x[3];
+        auto even = [&](real2 a, real2 b, real2 c) __attribute__((always_inline)) {
             return axpy(axpy(axpy(x[0], p1, a), p2, b), p3, c);
         };
-        auto odd = [&](float a, float b, float c) __attribute__((always_inline)) {
-            return axpy(axpy(make_float2(d1.x * a, d1.y * a), d2, b), d3, c);
+        auto odd = [&](real2 a, real2 b, real2 c) __attribute__((always_inline)) {
+            return axpy(axpy(scale(d1, a), d2, b), d3, c);
         };
         const float2 e1 = even(c1, c2, c3), e2 = even(c2, c3, c1), e3 = even(c3, c1, c2);
-        const float2 o1 = odd(s1, s2, s3), o2 = odd(s2, -s3, -s1), o3 = odd(s3, -s1, s2);
+        const float2 o1 = odd(s1, s2, s3), o2 = odd(s2, m3, m1), o3 = odd(s3, m1, s2);
         x[0] = x[0] + ((p1 + p2) + p3);
-        x[1] = add_i(e1, o1, s);
-        x[6] = add_i(e1, o1, -s);
-        x[2] = add_i(e2, o2, s);
-        x[5] = add_i(e2, o2, -s);
-        x[3] = add_i(e3, o3, s);
-        x[4] = add_i(e3, o3, -s);
+        x[1] = add_i(e1, o1);
+        x[6] = sub_i(e1, o1);
+        x[2] = add_i(e2, o2);
+        x[5] = sub_i(e2, o2);
+        x[3] = add_i(e3, o3);
+        x[4] = sub_i(e3, o3);
     } else {
         // R = 2 H: halves of even and odd inputs, X[k] = E[k] + w^k O[k], X[k + H] = E[k] - w^k O[k]
         constexpr int H = R / 2;
@@ -112,20 +153,21 @@ __device__ __forceinline__ void dft(float2 (&x)[R], float s)
             e[i] = x[2 * i];
             o[i] = x[2 * i + 1];
         }
-        dft<H>(e, s);
-        dft<H>(o, s);
-        constexpr float r2 = 0.707106781186547524f, r3 = 0.866025403784438647f;
-        constexpr float wc[5] = {1.f, R == 6 ? 0.5f : R == 8 ? r2 : 0.809016994374947424f,
-                                 R == 6 ? -0.5f : R == 8 ? 0.f : 0.309016994374947424f,
-                                 R == 8 ? -r2 : -0.309016994374947424f, -0.809016994374947424f};
-        constexpr float ws[5] = {0.f, R == 6 ? r3 : R == 8 ? r2 : 0.587785252292473129f,
-                                 R == 6 ? r3 : R == 8 ? 1.f : 0.951056516295153572f,
-                                 R == 8 ? r2 : 0.951056516295153572f, 0.587785252292473129f};
+        dft<H, S>(e);
+        dft<H, S>(o);
+        constexpr double r3 = 0.86602540378443864676, C1 = 0.80901699437494742410, C2 = 0.30901699437494742410;
+        constexpr double S1 = 0.58778525229247312917, S2 = 0.95105651629515357212;
+        constexpr real2 wc[5] = {two(1.), two(R == 6 ? 0.5 : C1), two(R == 6 ? -0.5 : C2), two(-C2), two(-C1)};
+        constexpr real2 ws[5] = {two(0.), two(S * (R == 6 ? r3 : S1)), two(S * (R == 6 ? r3 : S2)), two(S * S2), two(S * S1)};
+        constexpr real2 r2 = two(0.70710678118654752440);
 #pragma unroll
         for (int i = 0; i < H; ++i) {
-            const float2 t = i == 0               ? o[0]
-                             : (R == 8 && i == 2) ? make_float2(-s * o[2].y, s * o[2].x)
-                                                  : cmul(o[i], make_float2(wc[i], s * ws[i]));
+            const float2 si = S > 0 ? make_float2(-o[i].y, o[i].x) : make_float2(o[i].y, -o[i].x);
+            const float2 t = i == 0    ? o[0]
+                             : R != 8  ? cmul(o[i], wc[i], ws[i])
+                             : i == 1  ? scale(o[i] + si, r2)
+                             : i == 2  ? si
+                                       : scale(si - o[i], r2);
             x[i] = e[i] + t;
             x[i + H] = e[i] - t;
         }
@@ -173,9 +215,9 @@ __device__ __forceinline__ int lds_at(const fft_desc &d, int n, int row)
 // by side (pitch 1) and lanes run across them.  Memory addresses are a
 // uniform base for each input (output) of the butterflies and one offset a
 // butterfly, below 2^32 bytes.
-template <int R, bool ROWS, int NB, bool SOS>
+template <int R, bool ROWS, int NB, int S, bool SOS>
 __device__ __forceinline__ void stage(const fft_desc &d, int i, const tile_at &t, float2 *buf, float2 *tw,
-                                      const float2 *__restrict__ gtw, float s, const sos_out &o)
+                                      const float2 *__restrict__ gtw, const sos_out &o)
 {
     const stage_desc &g = d.st[i];
     const bool first = i == 0, last = i == d.stages - 1;
@@ -220,7 +262,7 @@ __device__ __forceinline__ void stage(const fft_desc &d, int i, const tile_at &t
 #pragma unroll
             for (int r = 1; r < R; ++r) x[b][r] = cmul(x[b][r], tw[r * jm * g.step]);
         }
-        dft<R>(x[b], s);
+        dft<R, S>(x[b]);
         const int n = jq * g.Ns * R + jm;
         if (last) {
             const uint32_t off = (uint32_t)n * (uint32_t)t.step + (uint32_t)row[b] * t.pitch;
@@ -244,20 +286,20 @@ __device__ __forceinline__ void stage(const fft_desc &d, int i, const tile_at &t
     if (!last) __syncthreads();
 }
 
-template <bool ROWS, int NB, bool SOS>
+template <bool ROWS, int NB, int S, bool SOS>
 __device__ __forceinline__ void transform(const fft_desc &d, const tile_at &t, float2 *buf, float2 *tw,
-                                          const float2 *__restrict__ gtw, float s, const sos_out &o)
+                                          const float2 *__restrict__ gtw, const sos_out &o)
 {
     for (int i = 0; i < d.stages; ++i)
         switch (d.st[i].R) {                    // the barrier after stage 0 also covers the twiddles
-        case 2: stage<2, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
-        case 3: stage<3, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
-        case 4: stage<4, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
-        case 5: stage<5, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
-        case 6: stage<6, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
-        case 7: stage<7, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
-        case 8: stage<8, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
-        default: stage<10, ROWS, NB, SOS>(d, i, t, buf, tw, gtw, s, o); break;
+        case 2: stage<2, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
+        case 3: stage<3, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
+        case 4: stage<4, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
+        case 5: stage<5, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
+        case 6: stage<6, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
+        case 7: stage<7, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
+        case 8: stage<8, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
+        default: stage<10, ROWS, NB, S, SOS>(d, i, t, buf, tw, gtw, o); break;
         }
 }
 
@@ -265,10 +307,10 @@ __device__ __forceinline__ void transform(const fft_desc &d, const tile_at &t, f
 // of count columns, N apart by `step`; tile T the columns from (T mod tiles)
 // TC of plane T / tiles, planes `plane` elements apart.  SOS: the one plane of
 // each coil in turn, then the image.
-template <bool ROWS, int NB, bool SOS>
+template <bool ROWS, int NB, int S, bool SOS>
 __global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 6 : 4))) k_fft(
     float2 *data, const float2 *__restrict__ gtw, fft_desc d, int64_t count, uint32_t tiles, uint32_t all, int64_t step,
-    int64_t plane, float s, sos_out o)
+    int64_t plane, sos_out o)
 {
     extern __shared__ float2 sm[];              // twiddles [N], tile, sums
     float2 *buf = sm + d.N;
@@ -285,12 +327,12 @@ __global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_e
     t.pitch = 8u * (ROWS ? (uint32_t)d.N : 1u);
     t.rows = (int)min((int64_t)1 << d.ltc, count - q0);
     if constexpr (!SOS) {
-        transform<ROWS, NB, false>(d, t, buf, sm, gtw, s, o);
+        transform<ROWS, NB, S, false>(d, t, buf, sm, gtw, o);
     } else {
         o.acc = reinterpret_cast<float *>(buf + ((size_t)d.N << d.ltc));
         for (int i = threadIdx.x; i < o.rc << d.ltc; i += blockDim.x) o.acc[i] = 0.f;
         for (int c = 0; c < o.C; ++c) {         // (two stages or more: a barrier before the first use of acc)
-            transform<ROWS, NB, true>(d, t, buf, sm, gtw, s, o);
+            transform<ROWS, NB, S, true>(d, t, buf, sm, gtw, o);
             t.base += 8 * o.coil;
             __syncthreads();
         }
@@ -374,13 +416,17 @@ fr_status pass(fr_fft *f, float2 *data, int64_t planes, int64_t count, int64_t s
                        (sos ? sizeof(float) * ((size_t)sos->rc << d.ltc) : 0);
     const int64_t W = planes * tiles();
     FR_CHECK(ctx, W < (int64_t(1) << 31), FR_ERR_UNSUPPORTED, "FFT launch of %lld workgroups", (long long)W);
-    auto kern = each == 1 ? k_fft<ROWS, 1, false> : k_fft<ROWS, 2, false>;
+    const bool pos = f->sign > 0;
+    auto kern = each == 1 ? (pos ? k_fft<ROWS, 1, 1, false> : k_fft<ROWS, 1, -1, false>)
+                          : (pos ? k_fft<ROWS, 2, 1, false> : k_fft<ROWS, 2, -1, false>);
     if constexpr (!ROWS)
-        if (sos) kern = each == 1 ? k_fft<ROWS, 1, true> : k_fft<ROWS, 2, true>;
+        if (sos)
+            kern = each == 1 ? (pos ? k_fft<ROWS, 1, 1, true> : k_fft<ROWS, 1, -1, true>)
+                             : (pos ? k_fft<ROWS, 2, 1, true> : k_fft<ROWS, 2, -1, true>);
     if (lds > 65536)
         FR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(kern, dim3((unsigned)((W + 7) / 8 * 8)), dim3(threads), lds, ctx->stream, data, f->tw, d, count,
-                       (uint32_t)tiles(), (uint32_t)W, step, plane, (float)f->sign, sos ? *sos : sos_out{});
+                       (uint32_t)tiles(), (uint32_t)W, step, plane, sos ? *sos : sos_out{});
     FR_HIP(ctx, hipGetLastError());
     return FR_OK;
 }

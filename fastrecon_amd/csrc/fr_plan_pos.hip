@@ -195,7 +195,7 @@ __global__ void k_box_keys(const uint32_t *__restrict__ first, const uint32_t *_
 }
 
 // What a unit takes, and (scanned) where it starts.  The sums stay below
-// 2^31: checked on the padded record count before.
+// 2^32: checked on the padded record count before.
 struct ustat {
     uint32_t recs;              // records, padded to FR_POS_BATCH
     uint32_t items, slots;      // items; slots of partial sums (units with several items)
@@ -262,8 +262,8 @@ __global__ void k_units(const uint32_t *__restrict__ order, int64_t nu, pgeom g,
     const uint32_t box0 = (uint32_t)ox | ((uint32_t)oy << 16);
     const uint32_t box1 = (uint32_t)oz | (((uint32_t)ux | ((uint32_t)uy << 5) | ((uint32_t)uz << 10)) << 16);
     for (uint32_t q = 0; q < nit; ++q) {
-        const uint32_t r0 = p.recs + q * S;
-        const uint32_t r1 = min(r0 + S, p.recs + c4);
+        const uint32_t r0 = p.recs + q * S, end = p.recs + c4;
+        const uint32_t r1 = r0 + min(S, end - r0);
         items[p.items + q] = fr_item{(uint32_t)u, nit > 1 ? (int32_t)(p.slots + q) : -1, r0, r1, box0, box1};
     }
     if (nit > 1) heavy[p.heavy] = fr_heavy{(uint32_t)u, nit, p.slots, 0u};
@@ -423,7 +423,10 @@ fr_status fr_plan_build_pos(fr_plan *p, const fr_samples *s, const fr_tune *tune
     uint64_t R = 0;
     FR_HIP(ctx, hipMemcpyAsync(&R, spos + M, 8, hipMemcpyDeviceToHost, st));
     FR_HIP(ctx, hipStreamSynchronize(st));
-    FR_CHECK(ctx, R + 16 * (uint64_t)nbox + FR_POS_PAD < (uint64_t(1) << 31), FR_ERR_UNSUPPORTED,
+    // Sorts take below 2^31 records, and the padded ones (a box without any
+    // takes none) are counted in 32 bits.
+    const uint64_t padded = R + (FR_POS_BATCH - 1) * std::min<uint64_t>(R, nbox) + FR_POS_PAD;
+    FR_CHECK(ctx, R + 4 * (uint64_t)nbox + 64 < (uint64_t(1) << 31) && padded < (uint64_t(1) << 32), FR_ERR_UNSUPPORTED,
              "plan has %llu records (max about 2^31)", (unsigned long long)R);
 
     // slice size S (records, a multiple of 16): about 32 slices' worth of

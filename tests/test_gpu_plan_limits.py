@@ -43,3 +43,32 @@ def test_more_than_2_30_records(ctx):
             h.close()
     assert grids[0].real.max() < 1 << 24
     np.testing.assert_array_equal(grids[0], grids[1] + grids[2])
+
+
+def corner(ctx, N, shift, M):
+    """Records of a plan, and the gridded and degridded samples, of points within 64^3 cells from `shift` on."""
+    rng = np.random.default_rng(1)
+    t = (rng.integers(4 * 64, 60 * 64, (M, 3)) / 64).astype(np.float32)
+    s = hip.Samples(ctx, 3, M, 1)
+    s.set_traj(t + np.float32(shift))
+    s.set_dcf(np.ones(M, np.float32))
+    s.set_coil(0, rng.standard_normal((M, 2)).astype(np.float32).view(np.complex64)[:, 0])
+    p = hip.Plan(ctx, s, N, 4.0, hip.kb_lut(4.0, 2.0, 512)[0])
+    g = hip.Grids(ctx, 3, N, 1)
+    out = hip.DeviceBuffer(ctx, 8 * M)
+    hip.grid_execute(p, s, g)
+    hip.degrid_execute(p, s, g, out)
+    got = p.info()["records"], out.to_host(np.int32)
+    for h in (out, g, p, s):
+        h.close()
+    return got
+
+
+def test_more_boxes_than_records(ctx):
+    """The records are refused by what they take when padded, and boxes without any take nothing.  Weights and sums
+    are those of the same samples on a small grid, bit for bit (shifts are multiples of the unit boxes' sides)."""
+    N, M = 1288, 1_700_000
+    small, large = corner(ctx, 64, 0, M), corner(ctx, N, 1220, M)
+    assert small[0] == large[0]
+    assert small[0] + 16 * (N // 4) * (N // 2) ** 2 >= 1 << 31
+    np.testing.assert_array_equal(small[1], large[1])

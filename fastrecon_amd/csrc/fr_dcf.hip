@@ -351,7 +351,8 @@ extern "C" fr_status fr_degrid_execute(fr_plan *p, const fr_samples *s, const fr
     FR_EXTENT(ctx, out_dev, sizeof(float2) * (size_t)s->M * g->C, "fr_degrid_execute output");
     // The samples' tile order, once the plan has it; it is built where one
     // call in acquisition order would cost more than that (a few launches
-    // and allocations), and not while the stream is being captured.
+    // and allocations), and not while the stream is being captured.  The
+    // general kernel, which allocates nothing, where there is no memory for it.
     if (fr_tiles_fit(p, s)) {
         bool build = !p->tord && s->M * g->C >= DEGRID_TILES;
         if (build) {
@@ -361,7 +362,7 @@ extern "C" fr_status fr_degrid_execute(fr_plan *p, const fr_samples *s, const fr
         }
         if (build) {
             fr_status e = fr_tiles_build(p);
-            if (e) return e;
+            if (e && e != FR_ERR_NOMEM) return e;
         }
         if (p->tord) return fr_tile_degrid(p, g->data, g->C, (float2 *)out_dev);
     }
@@ -434,10 +435,10 @@ extern "C" fr_status fr_dcf_pipe_menon(fr_plan *p, fr_samples *s, int iters, int
     FR_CHECK(ctx, iters >= 0, FR_ERR_INVALID, "iters must be >= 0");
     FR_CHECK(ctx, s->frames == p->frames, FR_ERR_INVALID, "samples and plan differ in frames");
     const int64_t M = s->M;
-    fr_status st = FR_OK;
-    if (fr_tiles_fit(p, s)) {
-        st = fr_tile_density(p, s, iters, init_ones || !s->has_dcf);
-        if (st) return st;
+    // (the general path's workspace is smaller where tiles hold few samples)
+    fr_status st = fr_tiles_fit(p, s) ? fr_tile_density(p, s, iters, init_ones || !s->has_dcf) : FR_ERR_NOMEM;
+    if (st && st != FR_ERR_NOMEM) return st;
+    if (!st) {
         s->has_dcf = true;
         fr_dcf_changed(s);
         hipError_t e = hipStreamSynchronize(ctx->stream);

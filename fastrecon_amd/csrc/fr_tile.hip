@@ -734,10 +734,15 @@ fr_status fr_tile_density(fr_plan *p, fr_samples *s, int iters, bool ones)
     if (e) return e;
     fr_tiles *t = p->tord;
     const size_t box = p->dim == 3 ? shape<3>::CELLS : shape<2>::CELLS;
-    if (!t->w && ((e = fr_alloc(ctx, (void **)&t->w, sizeof(float) * p->M)))) return e;
-    if (!t->grid && (e = fr_alloc(ctx, (void **)&t->grid, sizeof(float) * fr_plan_cells(p->dim, p->N, p->frames))))
+    if ((!t->w && (e = fr_alloc(ctx, (void **)&t->w, sizeof(float) * p->M))) ||
+        (!t->grid &&
+         (e = fr_alloc(ctx, (void **)&t->grid, sizeof(float) * fr_plan_cells(p->dim, p->N, p->frames)))) ||
+        (!t->part && (e = fr_alloc(ctx, (void **)&t->part, sizeof(float) * box * t->nitems)))) {
+        hipFree(t->w);                          // all of it for the general path
+        hipFree(t->grid);
+        t->w = t->grid = nullptr;
         return e;
-    if (!t->part && (e = fr_alloc(ctx, (void **)&t->part, sizeof(float) * box * t->nitems))) return e;
+    }
     const tgeom g = geom_of(p);
     return p->dim == 3 ? density<3>(p, g, s, iters, ones) : density<2>(p, g, s, iters, ones);
 }

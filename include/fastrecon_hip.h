@@ -215,8 +215,9 @@ fr_status fr_grid_execute_noalloc(fr_plan *p, const fr_samples *s, fr_grids *out
  * trajectory the plan was built on; out: device complex64, sample-major
  * [M][g->C].  A position-weight plan whose kernel is at most 4 cells wide
  * orders its samples by grid tile on the first large call (not during a
- * capture; or on the first fr_dcf_pipe_menon) and keeps that order, about 16
- * bytes a sample, until fr_plan_destroy. */
+ * capture, nor where there is no memory for it; or on the first
+ * fr_dcf_pipe_menon) and keeps that order, about 16 bytes a sample, until
+ * fr_plan_destroy. */
 fr_status fr_degrid_execute(fr_plan *p, const fr_samples *s, const fr_grids *g, void *out_dev);
 
 /* -------------------------------------------------------------------- FFT */
@@ -278,9 +279,10 @@ fr_status fr_deapod_map(fr_ctx *ctx, int dim, unsigned N, float kWidth, const fl
  * to the samples' DCF.  The first call gives the plan a workspace that it keeps
  * until fr_plan_destroy: on a position-weight plan with a kernel of at most 4
  * cells, and samples still on the plan's trajectory, the samples in tile order
- * with a density each, a real grid and a box of sums per work item; otherwise
- * (and for fr_dcf_identity_scale) the trajectory, unit data, one grid and M
- * complex densities, with this plan's gridding and degridding kernels. */
+ * with a density each, a real grid and a box of sums per work item; otherwise,
+ * or where there is no memory for that (and for fr_dcf_identity_scale), the
+ * trajectory, unit data, one grid and M complex densities, with this plan's
+ * gridding and degridding kernels. */
 fr_status fr_dcf_pipe_menon(fr_plan *p, fr_samples *s, int iters, int init_ones);
 
 /* Global scale of the samples' DCF (net-new) from the Pipe-Menon fixed-point

@@ -227,12 +227,32 @@ __device__ __forceinline__ void box_taps(const float4 &p, const int (&lo)[3], in
     }
 }
 
+// f(cell, w) for a sample's accepted taps alone, in the same order.  For
+// regions with an infinite or NaN value, which a weight of 0 does not leave
+// out of a sum.
+template <int DIM, typename F>
+__device__ __forceinline__ void accepted_taps(const float4 &p, const int (&lo)[3], int ox, int oy, int oz, int N,
+                                              const table &T, F &&f)
+{
+    constexpr int E = shape<DIM>::EDGE;
+#pragma unroll 1
+    for (int t = 0; t < shape<DIM>::TAPS; ++t) {
+        const int x = t & 3, y = t >> 2 & 3, z = t >> 4;
+        const float dz = DIM == 3 ? __fsub_rn((float)(lo[2] + z), p.z) : 0.f;
+        const float dy = __fsub_rn((float)(lo[1] + y), p.y), dx = __fsub_rn((float)(lo[0] + x), p.x);
+        const float d2 = fr_tap_dk2(__fmul_rn(dz, dz), __fmul_rn(dy, dy), dx);
+        // a cell past the grid's edge is no tap (its region value is 0)
+        if (!(d2 < T.dacc) || lo[0] + x >= N || lo[1] + y >= N || (DIM == 3 && lo[2] + z >= N)) continue;
+        f(((DIM == 3 ? lo[2] - oz + z : 0) * E + lo[1] - oy + y) * E + lo[0] - ox + x, lut_weight(T, d2));
+    }
+}
+
 // out[s][c0 + c] for the samples of one item.  The region's coils lie side by
 // side in LDS, a cell's in an odd multiple of 4 words for pairs of coils, of 2
 // words for an odd number (16- or 8-byte reads of random cells then spread
 // over all banks).  A rejected tap adds 0 * v, which leaves a sum unchanged
 // bit for bit unless v is infinite or NaN; a region with such a value takes
-// the second loop, which skips the tap.  Bound by the LDS: per tap two table
+// the second loop, of accepted taps.  Bound by the LDS: per tap two table
 // reads and the cell's coils, all at random addresses.
 template <int NC> constexpr int cell_words() { return NC % 4 == 0 ? 2 * NC + 4 : 2 * NC; }
 
@@ -316,25 +336,14 @@ __global__ void __launch_bounds__(64 * NW) k_tile_degrid(const fr_titem *__restr
                     }
             });
         } else {
-#pragma unroll 1
-            for (int t = 0; t < shape<DIM>::TAPS; ++t) {
-                const int x = t & 3, y = t >> 2 & 3, z = t >> 4;
-                const float dz = DIM == 3 ? __fsub_rn((float)(lo[2] + z), p.z) : 0.f;
-                const float dy = __fsub_rn((float)(lo[1] + y), p.y), dx = __fsub_rn((float)(lo[0] + x), p.x);
-                const float d2 = fr_tap_dk2(__fmul_rn(dz, dz), __fmul_rn(dy, dy), dx);
-                if (!(d2 < dacc)) continue;
-                const float w = lut_weight(T, d2);
-                const int cell = ((DIM == 3 ? lo[2] - oz + z : 0) * shape<DIM>::EDGE + lo[1] - oy + y) *
-                                     shape<DIM>::EDGE + lo[0] - ox + x;
-                // a cell past the grid's edge is no tap (its region value is 0)
-                if (lo[0] + x >= g.N || lo[1] + y >= g.N || (DIM == 3 && lo[2] + z >= g.N)) continue;
+            accepted_taps<DIM>(p, lo, ox, oy, oz, g.N, T, [&](int cell, float w) {
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
                     const float2 v = *reinterpret_cast<const float2 *>(reg + cell * CW + 2 * c);
                     a[c].x = __fadd_rn(a[c].x, __fmul_rn(w, v.x));
                     a[c].y = __fadd_rn(a[c].y, __fmul_rn(w, v.y));
                 }
-            }
+            });
         }
         float2 *o = out + (size_t)__float_as_uint(p.w) * C + c0;
 #pragma unroll
@@ -502,29 +511,41 @@ __global__ void __launch_bounds__(64 * WAVES) k_dens_update(const fr_titem *__re
                                                             float *__restrict__ w)
 {
     extern __shared__ float4 sm[];
+    __shared__ int odd;
     float *reg = reinterpret_cast<float *>(sm) + table_floats(L);
     const fr_titem it = items[blockIdx.x];
     if (it.tile == g.nt) {
         for (uint32_t i = threadIdx.x; i < it.n; i += 64 * WAVES) w[it.s0 + i] = 0.f;
         return;
     }
+    if (threadIdx.x == 0) odd = 0;
     const table T = stage_table(reinterpret_cast<float *>(sm), tbl, L, dacc, cidx);
+    __syncthreads();
     int ox, oy, oz;
     tile_origin<DIM>(it.tile, g, ox, oy, oz);
+    bool fine = true;
     for (int q = threadIdx.x; q < shape<DIM>::CELLS; q += 64 * WAVES) {
         const int64_t at = region_cell<DIM>(q, ox, oy, oz, g.N);
-        reg[q] = at >= 0 ? grid[at] : 0.f;
+        const float v = at >= 0 ? grid[at] : 0.f;
+        reg[q] = v;
+        fine = fine && __fsub_rn(v, v) == 0.f;
     }
+    if (!fine) odd = 1;
     __syncthreads();
+    const bool skip = odd != 0;
     for (uint32_t i = threadIdx.x; i < it.n; i += 64 * WAVES) {
         const float4 p = tpos[it.s0 + i];
         int lo[3];
         box_of<DIM>(p, g, lo);
         float d = 0.f;
-        box_taps<DIM>(p, lo, ox, oy, oz, T, [&](int cell, const float (&t)[4]) {
+        if (!skip)
+            box_taps<DIM>(p, lo, ox, oy, oz, T, [&](int cell, const float (&t)[4]) {
 #pragma unroll
-            for (int x = 0; x < 4; ++x) d = __fadd_rn(d, __fmul_rn(t[x], reg[cell + x]));
-        });
+                for (int x = 0; x < 4; ++x) d = __fadd_rn(d, __fmul_rn(t[x], reg[cell + x]));
+            });
+        else
+            accepted_taps<DIM>(p, lo, ox, oy, oz, g.N, T,
+                               [&](int cell, float t) { d = __fadd_rn(d, __fmul_rn(t, reg[cell])); });
         w[it.s0 + i] = d > 0.f ? __fdiv_rn(w[it.s0 + i], d) : 0.f;
     }
 }

@@ -353,6 +353,15 @@ __global__ void __launch_bounds__(64 * NW) k_tile_degrid(const fr_titem *__restr
 }
 
 // ---------------------------------------------------------------- density
+// A wave's LDS instructions execute in order; this keeps the compiler from
+// moving one lane's read before another lane's write (no instruction).
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 constexpr int STAGED = 16;       // floats per staged sample
 constexpr int AHEAD = 8;         // samples (2D: groups of 4) whose weights are computed before their adds
 
@@ -412,15 +421,13 @@ __global__ void __launch_bounds__(64 * WAVES) k_dens_grid(const fr_titem *__rest
             wo = make_float2(w[it.s0 + i + lane],
                              __int_as_float(((DIM == 3 ? lo[2] - oz : 0) * E + lo[1] - oy) * E + lo[0] - ox));
         }
-        __builtin_amdgcn_wave_barrier();     // the wave's LDS instructions stay in order
+        wave_sync();                         // the samples before are no longer read
         float4 *row = reinterpret_cast<float4 *>(stage + lane * STAGED);
         row[0] = d[0];
         row[1] = d[1];
         row[2] = d[2];
         *reinterpret_cast<float2 *>(row + 3) = wo;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
         // AHEAD samples' values first, then their adds (the compiler cannot
         // tell the boxes from the staged samples, so it would not move a
         // read past an add); rejected taps add 0 to a cell of the lane's own
@@ -437,9 +444,11 @@ __global__ void __launch_bounds__(64 * WAVES) k_dens_grid(const fr_titem *__rest
                 c[u] = d2 < dacc ? box + __float_as_int(q.y) : none;
             }
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) *c[u] = __fadd_rn(*c[u], v[u]);
+            for (int u = 0; u < AHEAD; ++u) {
+                *c[u] = __fadd_rn(*c[u], v[u]);
+                wave_sync();                 // the next sample's lanes may add to the same cells
+            }
         }
-        __builtin_amdgcn_wave_barrier();
     }
     __syncthreads();
     float *o = part + (size_t)blockIdx.x * CELLS;

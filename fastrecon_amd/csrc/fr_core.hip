@@ -107,6 +107,23 @@ void fr_pool_free(fr_ctx *ctx, void *p)
     pool.kept_bytes += b.bytes;
 }
 
+bool fr_keep(fr_kept **list, void *p)
+{
+    fr_kept *k = new (std::nothrow) fr_kept{p, *list};
+    if (k) *list = k;
+    return k != nullptr;
+}
+
+void fr_free_kept(fr_ctx *ctx, fr_kept *list)
+{
+    while (list) {
+        fr_kept *k = list;
+        list = k->next;
+        fr_pool_free(ctx, k->p);
+        delete k;
+    }
+}
+
 // ------------------------------------------------------------------ context
 extern "C" fr_status fr_ctx_create(int device, fr_ctx **out)
 {

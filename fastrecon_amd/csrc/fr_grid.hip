@@ -509,7 +509,12 @@ fr_status fr_launch_grid(fr_plan *p, const fr_samples *s, float2 *out, int force
     } else {
         if (need > p->partial_bytes) {
             FR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-            fr_pool_free(ctx, p->partial);
+            if (p->partial_captured && p->partial) {
+                FR_CHECK(ctx, fr_keep(&p->old_partials, p->partial), FR_ERR_NOMEM, "no host memory");
+                p->partial_captured = false;
+            } else {
+                fr_pool_free(ctx, p->partial);
+            }
             p->partial = nullptr;
             p->partial_bytes = 0;
             fr_status e = fr_pool_alloc(ctx, (void **)&p->partial, need);
@@ -517,6 +522,11 @@ fr_status fr_launch_grid(fr_plan *p, const fr_samples *s, float2 *out, int force
             p->partial_bytes = need;
         }
         partial = (float2 *)p->partial;
+        if (need > 0 && !p->partial_captured) {
+            hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+            FR_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
+            p->partial_captured = cs != hipStreamCaptureStatusNone;
+        }
     }
     if (p->nitems == 0) return FR_OK;
     const int mode = force_mode ? force_mode : p->accumulate;

@@ -183,6 +183,12 @@ struct fr_tiles {
     float *grid = nullptr;         // the real grid
 };
 
+// Blocks that a handle no longer uses itself and frees with the rest.
+struct fr_kept {
+    void *p;
+    fr_kept *next;
+};
+
 struct fr_plan {
     fr_ctx *ctx = nullptr;
     // the trajectory the plan was built on (fr_samples uid and version)
@@ -223,6 +229,11 @@ struct fr_plan {
     int64_t nheavy = 0, nslots = 0;
     float *partial = nullptr;          // scratch for heavy-unit slices
     size_t partial_bytes = 0;
+    // a captured pass writes there: a graph may be replayed as long as the
+    // plan lives, so a larger scratch does not give the block back but sets
+    // it aside
+    bool partial_captured = false;
+    fr_kept *old_partials = nullptr;
     fr_batch *batches = nullptr;       // gather mode: item i owns batches [items[i].t0, ..)
     // matrix-core mode: exact LUT-index thresholds on the squared distance,
     // pairs (B[m], B[m+1]) for m = 0 .. L, B[m] = least d2 whose reference
@@ -310,6 +321,9 @@ fr_status fr_alloc(fr_ctx *ctx, void **p, size_t bytes);
 // stream touches.  fr_pool_free also takes memory of fr_alloc.
 fr_status fr_pool_alloc(fr_ctx *ctx, void **p, size_t bytes);
 void fr_pool_free(fr_ctx *ctx, void *p);
+// p onto the list (false: no host memory for the entry); the list's blocks freed
+bool fr_keep(fr_kept **list, void *p);
+void fr_free_kept(fr_ctx *ctx, fr_kept *list);
 
 static inline size_t fr_cells(int dim, unsigned N)
 {

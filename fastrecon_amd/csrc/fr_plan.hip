@@ -966,6 +966,7 @@ extern "C" fr_status fr_plan_destroy(fr_plan *p)
                     (void *)p->items, (void *)p->heavy, (void *)p->partial, (void *)p->batches, (void *)p->mfma_pairs,
                     (void *)p->recs, (void *)p->pos, (void *)p->tsel, (void *)p->tiles})
         fr_pool_free(p->ctx, q);
+    fr_free_kept(p->ctx, p->old_partials);
     hipFree(p->dcf_den);
     hipFree(p->dcf_scr);
     fr_tiles_free(p->tord);

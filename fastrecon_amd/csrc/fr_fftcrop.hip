@@ -503,14 +503,26 @@ fr_status run_passes(fr_fft *f, const fr_grids *g, int rcx, int rcy, int rcz, in
 
 fr_status fr_fft_workspace(fr_fft *f, size_t bytes)
 {
-    if (bytes <= f->crop_ws_bytes) return FR_OK;
-    FR_HIP(f->ctx, hipStreamSynchronize(f->ctx->stream));
-    (void)hipFree(f->crop_ws);
-    f->crop_ws = nullptr;
-    f->crop_ws_bytes = 0;
-    fr_status e = fr_alloc(f->ctx, &f->crop_ws, bytes);
-    if (e) return e;
-    f->crop_ws_bytes = bytes;
+    fr_ctx *ctx = f->ctx;
+    if (bytes > f->crop_ws_bytes) {
+        FR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (f->crop_captured && f->crop_ws) {
+            FR_CHECK(ctx, fr_keep(&f->old_crop_ws, f->crop_ws), FR_ERR_NOMEM, "no host memory");
+            f->crop_captured = false;
+        } else {
+            (void)hipFree(f->crop_ws);
+        }
+        f->crop_ws = nullptr;
+        f->crop_ws_bytes = 0;
+        fr_status e = fr_alloc(ctx, &f->crop_ws, bytes);
+        if (e) return e;
+        f->crop_ws_bytes = bytes;
+    }
+    if (!f->crop_captured) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        FR_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
+        f->crop_captured = cs != hipStreamCaptureStatusNone;
+    }
     return FR_OK;
 }
 

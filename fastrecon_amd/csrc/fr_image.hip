@@ -140,6 +140,7 @@ extern "C" fr_status fr_fft_destroy(fr_fft *f)
     hipFree(f->work);
     hipFree(f->tw);
     hipFree(f->crop_ws);
+    fr_free_kept(f->ctx, f->old_crop_ws);
     delete f;
     return FR_OK;
 }

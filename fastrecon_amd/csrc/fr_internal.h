@@ -40,6 +40,12 @@ struct fr_ctx {
     fr_pool pool;
 };
 
+// Blocks that a handle no longer uses itself and frees with the rest.
+struct fr_kept {
+    void *p;
+    fr_kept *next;
+};
+
 struct fr_samples {
     fr_ctx *ctx = nullptr;
     int dim = 0;
@@ -183,12 +189,6 @@ struct fr_tiles {
     float *grid = nullptr;         // the real grid
 };
 
-// Blocks that a handle no longer uses itself and frees with the rest.
-struct fr_kept {
-    void *p;
-    fr_kept *next;
-};
-
 struct fr_plan {
     fr_ctx *ctx = nullptr;
     // the trajectory the plan was built on (fr_samples uid and version)
@@ -298,6 +298,8 @@ struct fr_fft {
     float2 *tw = nullptr;
     void *crop_ws = nullptr;
     size_t crop_ws_bytes = 0;
+    bool crop_captured = false;        // a captured pass uses them: as a plan's slice scratch
+    fr_kept *old_crop_ws = nullptr;
 };
 
 // ----------------------------------------------------------------- errors

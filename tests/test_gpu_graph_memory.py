@@ -56,3 +56,36 @@ def test_more_coils_after_the_capture(ctx, tune):
             hip.grid_execute(po, so, go)
             np.testing.assert_array_equal(go.download_all(), before)
     np.testing.assert_array_equal(gm.download(0), ref[0])
+
+
+def test_larger_crop_after_the_capture(ctx):
+    N, C, rc, large = 256, 3, (64, 64, 1), (256, 200, 1)
+    rng = np.random.default_rng(0)
+    y = (rng.standard_normal((C, N * N)) + 1j * rng.standard_normal((C, N * N))).astype(np.complex64)
+    t = rng.uniform(0, N - 1, (2000, 2)).astype(np.float32)
+    s = hip.Samples(ctx, 2, 2000, C)
+    s.set_traj(t)
+    s.set_dcf(np.ones(2000, np.float32))
+    s.set_coils(y[:, :2000])
+    g, f = hip.Grids(ctx, 2, N, C), hip.FFT(ctx, 2, N, C)
+    plan = hip.Plan(ctx, s, N, 4.0, hip.kb_lut(4.0, 2.0, 512)[0])
+    out = hip.DeviceBuffer(ctx, 4 * rc[0] * rc[1])
+    graph = hip.Graph(plan, s, g, f, rc, True, None, out)
+    graph.launch()
+    ref = out.to_host(np.int32)
+    g2 = hip.Grids(ctx, 2, N, C)
+    for c in range(C):
+        g2.upload(c, y[c])
+    wide = hip.fft_sos(f, g2, large).to_host(np.int32)
+    size = 8 * C * rc[0] * N                                         # of the first pass' buffer
+    held = [hip.DeviceBuffer(ctx, size) for _ in range(64)]
+    mark = rng.integers(0, 255, size).astype(np.uint8)
+    for b in held:
+        b.from_host(mark)
+    for turn in range(3):
+        out.from_host(np.zeros(rc[0] * rc[1], np.float32))
+        graph.launch()
+        np.testing.assert_array_equal(out.to_host(np.int32), ref)
+        for b in held:
+            np.testing.assert_array_equal(b.to_host(np.uint8), mark)
+        np.testing.assert_array_equal(hip.fft_sos(f, g2, large).to_host(np.int32), wide)

@@ -56,6 +56,18 @@ fr_status fr_alloc(fr_ctx *ctx, void **p, size_t bytes)
     return FR_OK;
 }
 
+// p among the blocks in use (m is held); false without host memory for it: no
+// exception leaves a C entry point
+static bool pool_note(fr_pool &pool, void *p, size_t bytes)
+{
+    try {
+        pool.out.emplace(p, bytes);
+        return true;
+    } catch (const std::bad_alloc &) {
+        return false;
+    }
+}
+
 fr_status fr_pool_alloc(fr_ctx *ctx, void **p, size_t bytes)
 {
     *p = nullptr;
@@ -75,7 +87,7 @@ fr_status fr_pool_alloc(fr_ctx *ctx, void **p, size_t bytes)
                 best = i;
         if (best < pool.kept.size()) {
             const fr_pool::block b = pool.kept[best];
-            pool.out.emplace(b.p, b.bytes);     // before the block leaves the list
+            if (!pool_note(pool, b.p, b.bytes)) return fr_fail(ctx, FR_ERR_NOMEM, "no host memory");
             pool.kept.erase(pool.kept.begin() + best);
             pool.kept_bytes -= b.bytes;
             *p = b.p;
@@ -85,7 +97,11 @@ fr_status fr_pool_alloc(fr_ctx *ctx, void **p, size_t bytes)
     const fr_status e = fr_alloc(ctx, p, size);
     if (e) return e;
     std::lock_guard<std::mutex> lock(pool.m);
-    pool.out.emplace(*p, size);
+    if (!pool_note(pool, *p, size)) {
+        (void)hipFree(*p);
+        *p = nullptr;
+        return fr_fail(ctx, FR_ERR_NOMEM, "no host memory");
+    }
     return FR_OK;
 }
 
@@ -103,8 +119,12 @@ void fr_pool_free(fr_ctx *ctx, void *p)
     const fr_pool::block b{p, it->second};
     pool.out.erase(it);
     pool_trim(pool, FR_POOL_BYTES - b.bytes);
-    pool.kept.push_back(b);
-    pool.kept_bytes += b.bytes;
+    try {
+        pool.kept.push_back(b);
+        pool.kept_bytes += b.bytes;
+    } catch (const std::bad_alloc &) {
+        (void)hipFree(p);
+    }
 }
 
 bool fr_keep(fr_kept **list, void *p)

@@ -199,6 +199,16 @@ extern "C" fr_status fr_ctx_synchronize(fr_ctx *ctx)
     return FR_OK;
 }
 
+// The blocks' last work is on the context's stream.
+extern "C" fr_status fr_ctx_trim(fr_ctx *ctx)
+{
+    if (!ctx) return FR_ERR_INVALID;
+    FR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    std::lock_guard<std::mutex> lock(ctx->pool.m);
+    pool_trim(ctx->pool, 0);
+    return FR_OK;
+}
+
 extern "C" void *fr_ctx_stream(fr_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }
 
 // ------------------------------------------------------------------ samples

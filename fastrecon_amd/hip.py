@@ -26,7 +26,7 @@ FR_LAYOUT_COIL_MAJOR, FR_LAYOUT_SAMPLE_MAJOR = 0, 1
 # every symbol the header declares (checked by the CPU test suite)
 EXPORTS = [
     "fr_kb_lut", "fr_traj_normalize", "fr_traj_transform",
-    "fr_ctx_create", "fr_ctx_destroy", "fr_last_error", "fr_ctx_synchronize", "fr_ctx_stream",
+    "fr_ctx_create", "fr_ctx_destroy", "fr_last_error", "fr_ctx_synchronize", "fr_ctx_trim", "fr_ctx_stream",
     "fr_samples_create", "fr_samples_destroy", "fr_samples_set_traj", "fr_samples_set_dcf",
     "fr_samples_set_coil", "fr_samples_update", "fr_samples_set_data_device", "fr_samples_set_dcf_device",
     "fr_samples_set_traj_device", "fr_samples_get_dcf",
@@ -91,6 +91,7 @@ def load():
         "fr_ctx_create": [C.c_int, _pp],
         "fr_ctx_destroy": [_vp],
         "fr_ctx_synchronize": [_vp],
+        "fr_ctx_trim": [_vp],
         "fr_samples_create": [_vp, C.c_int, C.c_int64, C.c_int, C.c_int, _pp],
         "fr_samples_destroy": [_vp],
         "fr_samples_set_traj": [_vp, _vp, C.c_int],
@@ -238,6 +239,10 @@ class Context:
 
     def sync(self):
         self.check(self.L.fr_ctx_synchronize(self.h), "fr_ctx_synchronize")
+
+    def trim(self):
+        """Frees the device memory that the context keeps from closed plans (up to 4 GiB)."""
+        self.check(self.L.fr_ctx_trim(self.h), "fr_ctx_trim")
 
     def close(self):
         if self.h:

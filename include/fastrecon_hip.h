@@ -129,11 +129,16 @@ fr_status fr_traj_transform(float *traj, int64_t M, int stride, int dim, float t
 
 /* ---------------------------------------------------------------- context */
 /* No reference counterpart (the reference uses the CUDA default stream and
- * checks no errors, cuGridLut.cu:303). */
+ * checks no errors, cuGridLut.cu:303).
+ * A context keeps up to 4 GiB of device memory that its plans gave back, for
+ * the next ones (allocating and freeing take longer than building a plan). It
+ * frees what it keeps when one of its own allocations fails, in fr_ctx_trim
+ * (for other users of the device's memory) and in fr_ctx_destroy. */
 fr_status fr_ctx_create(int device, fr_ctx **out);
 fr_status fr_ctx_destroy(fr_ctx *ctx);
 const char *fr_last_error(const fr_ctx *ctx);
 fr_status fr_ctx_synchronize(fr_ctx *ctx);
+fr_status fr_ctx_trim(fr_ctx *ctx);
 void *fr_ctx_stream(fr_ctx *ctx);              /* the hipStream_t */
 
 /* ---------------------------------------------------------------- samples */

@@ -466,10 +466,9 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
     };
 
     // ----------------------------------------------------------- pairs
-    // One wave grids the two x-adjacent units of a pair (boxes at least 4
-    // cells wide) one after the other, the first unit's sums held in
-    // registers, and writes them out together: rows of 2 bx cells (64 bytes
-    // for 4-cell-wide units) instead of bx.  (Stored straight from the
+    // One wave grids the two x-adjacent units of a pair one after the other,
+    // the first unit's sums held in registers, and writes them out together:
+    // rows of 2 bx cells (64 bytes for 4-cell-wide units) instead of bx.  (Stored straight from the
     // accumulators, 16 bytes of a row at a time, 32 coils at 256^3 took 4.87
     // ms against 4.31 with an LDS transpose by 4-byte words and 4.13 with this
     // one by 16-byte words.)
@@ -519,12 +518,15 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
                                               fy, fz, cidx, lmax, j, k);
         }
         // Lane (j, k) holds cells 4 k .. 4 k + 3 of both units, neighbours
-        // along x.  By way of LDS, [coil][cell of the pair's 2 bx x by x bz
+        // along x in boxes at least 4 wide.  By way of LDS, [coil][cell of the pair's 2 bx x by x bz
         // box][re, im], 16 coils a step, each lane then stores two
         // neighbouring cells of a coil and 2 bx cells make one write.
         const int px = (4 * k) & ((1 << lbx) - 1), prow = (4 * k) >> lbx;
         const int cell = 2 * (lane & 15), x = cell & ((2 << lbx) - 1), row = cell >> (lbx + 1);
         const size_t go = ((size_t)(ba.oz + (row >> lby)) * N + (ba.oy + (row & ((1 << lby) - 1)))) * N + (ba.ox + x);
+        // floats from the lane's first cell to its second and third: boxes
+        // less than 4 wide hold those in a next row
+        const int d1 = lbx >= 1 ? 2 : 4, d2 = lbx >= 2 ? 4 : 8;
         constexpr int steps = NCB == 4 ? 2 : 1, ncs = NCB == 1 ? 8 : 16;
 #pragma unroll
         for (int h = 0; h < steps; ++h) {
@@ -535,11 +537,17 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
                 if constexpr (NCB == 1) {
                     const f4 v = u ? acc[0] : acc_a[0];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) o[2 * r + (j & 1)] = v[r];
+                    for (int r = 0; r < 4; ++r) o[(r & 1) * d1 + (r >> 1) * d2 + (j & 1)] = v[r];
                 } else {
                     const f4 re = u ? acc[2 * h] : acc_a[2 * h], im = u ? acc[2 * h + 1] : acc_a[2 * h + 1];
-                    *reinterpret_cast<f4 *>(o) = f4{re[0], im[0], re[1], im[1]};
-                    *reinterpret_cast<f4 *>(o + 4) = f4{re[2], im[2], re[3], im[3]};
+                    if (lbx >= 1) {
+                        *reinterpret_cast<f4 *>(o) = f4{re[0], im[0], re[1], im[1]};
+                        *reinterpret_cast<f4 *>(o + d2) = f4{re[2], im[2], re[3], im[3]};
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            *reinterpret_cast<float2 *>(o + 4 * r) = make_float2(re[r], im[r]);
+                    }
                 }
             }
             wave_sync();

@@ -506,14 +506,14 @@ fr_status fr_plan_build_pos(fr_plan *p, const fr_samples *s, const fr_tune *tune
 
     // 7. tiles of TW x-adjacent whole units (unit box of 16 cells with
     // power-of-two sides; the grid divides into whole tiles): pairs by
-    // default (tile_writes 0 or 3; boxes at least 4 wide), rows of 2 bx cells; fours with
+    // default (tile_writes 0 or 3), rows of 2 bx cells; fours with
     // tile_writes 1, rows of 4 bx cells; none with tile_writes 2
     const bool pow2 = (geom.bx & (geom.bx - 1)) == 0 && (geom.by & (geom.by - 1)) == 0 &&
                       (geom.bz & (geom.bz - 1)) == 0;
     const int TW = tile_writes == 1 ? FR_POS_WAVES : (tile_writes == 2 ? 0 : 2);
     p->ntiles = 0;
     p->tile_units = 0;
-    if (TW > 0 && pow2 && (TW != 2 || geom.bx >= 4) && geom.cells_max == 16 && N % (TW * geom.bx) == 0 && N % geom.by == 0 &&
+    if (TW > 0 && pow2 && geom.cells_max == 16 && N % (TW * geom.bx) == 0 && N % geom.by == 0 &&
         (flat || N % geom.bz == 0) && nu > (int64_t)tot.sum.front) {
         const int ntx = g.nbx / TW;
         const int64_t ntiles = (int64_t)ntx * g.nby * g.nbz, nfront = tot.sum.front;

@@ -311,6 +311,14 @@ __device__ __forceinline__ void grid_records_mid(f4 (&acc)[NCB], uint32_t r, uin
                                   });
 }
 
+// Waves a SIMD that the registers have to leave room for: of the variants for
+// 4 (OCC 4) and for 3 (OCC 1), which up to 16 coils need fewer registers.
+template <int NCB, int OCC>
+constexpr int pos_waves()
+{
+    return NCB == 1 ? 6 : NCB == 2 ? (OCC == 4 ? 6 : 5) : OCC;
+}
+
 // NCB component blocks (chunks of 8 NCB coils).  PAIR: C even, so lane j's
 // two coils (2j, 2j+1 of a 32-coil chunk) are one aligned 16-byte (8-byte
 // for FP16) load.
@@ -324,22 +332,23 @@ __device__ __forceinline__ void grid_records_mid(f4 (&acc)[NCB], uint32_t r, uin
 //  * otherwise a run of ipw consecutive light items per wave, as one
 //    record stream, each unit written out by its wave.
 template <int NCB, bool PAIR, bool SMALL, typename TS, int OCC>
-__global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OCC == 4 && NCB <= 2 ? 6 : OCC, 8))) k_grid_pos(
+__global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(pos_waves<NCB, OCC>(), 8))) k_grid_pos(
     const fr_item *__restrict__ items, int64_t nitems, const fr_tile *__restrict__ tiles, int64_t ntiles,
     int lbx, int lby, int lbz, const uint32_t *__restrict__ recs, const float4 *__restrict__ pos,
     const float4 *__restrict__ tbl, int L, float cidx, const TS *__restrict__ data,
     int C, int N, size_t cells, float2 *__restrict__ out, float2 *__restrict__ partial,
     int64_t nslots, int cells_max, int64_t nfront, int64_t front_wg, int ipw, int64_t xr, int nt, int tw,
-    int wave_floats, int64_t tstride, int fsub)
+    int wave_floats, int osm_at, int64_t tstride, int fsub)
 {
     extern __shared__ float4 smem_pos[];
     float4 *stbl = smem_pos;                                         // L entries
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     // the wave's block of positions and, after them (its LDS instructions stay
-    // in order), its write-out transpose in the same place
+    // in order), its write-out transpose in the same place; beside them for
+    // runs of items
     float4 *pbuf = smem_pos + L + wv * (wave_floats / 4);
-    float *osm = reinterpret_cast<float *>(pbuf);
+    float *osm = reinterpret_cast<float *>(pbuf) + osm_at;
     for (int q = threadIdx.x; q < L; q += 64 * PW) stbl[q] = tbl[q];
     __syncthreads();
 
@@ -579,29 +588,53 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(OC
     }
     if (i >= iend) return;
 
-    // item by item; units without records are written as zeros
-    for (; i < iend; ++i) {
-        fr_item it = items[i];
-        if (bid < front_wg && fsub > 1) {
-            // only the front units of every tstride-th rank; the sub-slice's
-            // records (a multiple of FR_POS_BATCH, possibly none) go to
-            // virtual slot fw
-            if (it.unit % (uint32_t)tstride != 0) return;
-            const uint32_t sub = (uint32_t)(fw % fsub), len = it.r1 - it.r0;
-            const uint32_t sl = ((len + fsub - 1) / fsub + (FR_POS_BATCH - 1)) & ~(uint32_t)(FR_POS_BATCH - 1);
-            const uint32_t a = min(it.r0 + sub * sl, it.r1);
-            it.r0 = a;
-            it.r1 = min(a + sl, it.r1);
-            it.slot = (int32_t)fw;
-        }
-        const item_box box = unpack_box(it.t0, it.pad);
-        float fx, fy, fz;
+    fr_item it = items[i];
+    item_box box = unpack_box(it.t0, it.pad);
+    float fx, fy, fz;
+    if (ipw > 1 && bid >= front_wg) {
+        // A run of light items (one each a unit, their records consecutive)
+        // as one record stream: at an item's end the pipeline keeps running
+        // while the unit is written out, from LDS beside the positions.
+        // Units without records are written as zeros.
+        auto next = [&]() __attribute__((always_inline)) {
+            write_out(it, box);
+            while (++i < iend) {
+                it = items[i];
+                box = unpack_box(it.t0, it.pad);
+                if (it.r0 < it.r1) return true;
+                write_out(it, box);
+            }
+            return false;
+        };
+        if (it.r0 == it.r1 && !next()) return;
         lane_cell(box, j, fx, fy, fz);
-        if (it.r0 < it.r1)
-            grid_records<NCB, PAIR, SMALL>(acc, it.r0, it.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx, fy, fz,
-                                          cidx, lmax, j, k);
-        write_out(it, box);
+        const uint32_t first = it.r0;
+        grid_stream<NCB, PAIR, SMALL>(acc, recs + first, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx, fy, fz, cidx,
+                                      lmax, j, k, [&](uint32_t q) __attribute__((always_inline)) {
+                                          if (q != it.r1 - first) return true;
+                                          const bool more = next();
+                                          if (more) lane_cell(box, j, fx, fy, fz);
+                                          return more;
+                                      });
+        return;
     }
+    if (bid < front_wg && fsub > 1) {
+        // only the front units of every tstride-th rank; the sub-slice's
+        // records (a multiple of FR_POS_BATCH, possibly none) go to
+        // virtual slot fw
+        if (it.unit % (uint32_t)tstride != 0) return;
+        const uint32_t sub = (uint32_t)(fw % fsub), len = it.r1 - it.r0;
+        const uint32_t sl = ((len + fsub - 1) / fsub + (FR_POS_BATCH - 1)) & ~(uint32_t)(FR_POS_BATCH - 1);
+        const uint32_t a = min(it.r0 + sub * sl, it.r1);
+        it.r0 = a;
+        it.r1 = min(a + sl, it.r1);
+        it.slot = (int32_t)fw;
+    }
+    lane_cell(box, j, fx, fy, fz);
+    if (it.r0 < it.r1)
+        grid_records<NCB, PAIR, SMALL>(acc, it.r0, it.r1, recs, pos, data, (uint32_t)C, ca, cbb, stbl, pbuf, fx, fy, fz,
+                                      cidx, lmax, j, k);
+    write_out(it, box);
 }
 
 template <int NCB, bool PAIR, bool SMALL, typename TS, int OCC>
@@ -631,7 +664,8 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, 
     const int osm_floats = std::max(16 * NCB * CS, (NCB == 1 ? 8 : 16) * PS);
     // in the place of the block of positions before it; a tile of four, whose
     // waves write each other's cells, has its own
-    const int wave_floats = std::max(64 * 4, osm_floats);
+    const int osm_at = p->ntiles == 0 && ipw > 1 ? 64 * 4 : 0;
+    const int wave_floats = std::max(64 * 4, osm_at + osm_floats);
     const size_t lds = sizeof(float4) * p->L + sizeof(float) * PW * (wave_floats + (fours ? osm_floats : 0));
     auto kern = k_grid_pos<NCB, PAIR, SMALL, TS, OCC>;
     FR_HIP(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -641,7 +675,7 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, 
                        p->tiles, p->ntiles, lbx, lby, lbz, p->recs, p->pos, p->tsel, p->L, p->mfma_cidx,
                        (const TS *)s->data, s->C, (int)p->N, cells, out, partial, p->nslots,
                        p->geom.cells_max, p->nitems_front, front_wg, ipw, xr, p->pos_stores == 1 ? 1 : 0,
-                       p->tile_units, wave_floats, tstride, tstride > 1 ? fsub : 1);
+                       p->tile_units, wave_floats, osm_at, tstride, tstride > 1 ? fsub : 1);
     FR_HIP(ctx, hipGetLastError());
     return FR_OK;
 }

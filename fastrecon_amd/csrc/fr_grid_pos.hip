@@ -643,22 +643,29 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial, 
     fr_ctx *ctx = p->ctx;
     const size_t cells = fr_plan_cells(p->dim, p->N, p->frames);
     const int chunks = (s->C + 8 * NCB - 1) / (8 * NCB);
-    const int ipw = std::max(1, p->pos_ipw);
-    const int64_t per_wg = (int64_t)PW * ipw;
+    const int64_t light = p->nitems - p->nitems_front;
     // tstride > 1 (pair plans only): the sampled pairs (fr_sampled_tile), and
     // the front items cut into fsub sub-slices each (one wave per sub-slice)
     const int64_t front_wg = (p->nitems_front * (tstride > 1 ? fsub : 1) + PW - 1) / PW;
-    const int64_t light = p->nitems - p->nitems_front;
     const int64_t npairs = fr_sampled_tiles(p->ntiles, tstride);
     // light work: tiles of four (one per workgroup), pairs (PW per
-    // workgroup) or runs of ipw items per wave
+    // workgroup) or runs of ipw items per wave; longer runs where one wave an
+    // item would be more work-items than a launch takes (grids above 1024^3
+    // that do not divide into pairs)
     const bool fours = p->ntiles > 0 && p->tile_units == PW;
-    const int64_t groups = p->ntiles > 0 ? (fours ? p->ntiles : (npairs + PW - 1) / PW)
-                                         : (light + per_wg - 1) / per_wg;
-    const int64_t xr = std::max<int64_t>(1, p->xcd_run / (p->ntiles > 0 ? (fours ? PW : 2 * PW) : per_wg));
-    const int64_t span = 8 * xr;
-    const int64_t W = front_wg + span * ((groups + span - 1) / span);
-    FR_CHECK(ctx, W < (int64_t(1) << 31), FR_ERR_UNSUPPORTED, "gridding launch of %lld workgroups", (long long)W);
+    int ipw = std::max(1, p->pos_ipw);
+    int64_t xr = 0, W = 0;
+    for (;; ipw *= 2) {
+        const int64_t per_wg = (int64_t)PW * ipw;
+        const int64_t groups = p->ntiles > 0 ? (fours ? p->ntiles : (npairs + PW - 1) / PW)
+                                             : (light + per_wg - 1) / per_wg;
+        xr = std::max<int64_t>(1, p->xcd_run / (p->ntiles > 0 ? (fours ? PW : 2 * PW) : per_wg));
+        const int64_t span = 8 * xr;
+        W = front_wg + span * ((groups + span - 1) / span);
+        if (W * 64 * PW < (int64_t(1) << 32) || p->ntiles > 0 || ipw > 64) break;
+    }
+    FR_CHECK(ctx, W * 64 * PW < (int64_t(1) << 32), FR_ERR_UNSUPPORTED, "gridding launch of %lld workgroups",
+             (long long)W);
     // per wave: the write-out transpose (16 cells x 16 NCB components, or a
     // step of a pair; a tile of four needs less from its four waves together)
     const int osm_floats = std::max(16 * NCB * CS, (NCB == 1 ? 8 : 16) * PS);

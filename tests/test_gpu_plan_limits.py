@@ -72,3 +72,11 @@ def test_more_boxes_than_records(ctx):
     assert small[0] == large[0]
     assert small[0] + 16 * (N // 4) * (N // 2) ** 2 >= 1 << 31
     np.testing.assert_array_equal(small[1], large[1])
+
+
+def test_more_units_than_a_launch_has_waves(ctx):
+    """1290^3 does not divide into pairs of boxes: 134M units, of which a launch takes 67M at one a wave."""
+    M = 3000
+    small, large = corner(ctx, 64, 0, M), corner(ctx, 1290, 1220, M)
+    assert small[0] == large[0]
+    np.testing.assert_array_equal(small[1], large[1])

@@ -431,13 +431,49 @@ fr_status pass(fr_fft *f, float2 *data, int64_t planes, int64_t count, int64_t s
     return FR_OK;
 }
 
+// Where rocFFT's kernels are the faster ones.  It has kernels that transform
+// these sizes in one pass over a small 2D grid, or in one pass an axis without
+// transposes, and a launch or two less, or more threads at work in each
+// stage, beats these passes on few elements (4 x 240^2: 9.3 us against 11.5;
+// 16^2 to 48^2: half) and, where the radices of a size leave threads idle in
+// some stages (the 7s and 2 of 98), on many (8 x 98^3: 98 against 112).  At
+// the sizes not listed, of all that plan() takes up to 1000^2 and 400^3, these
+// passes were faster, or within 3%, from 1 grid to 2^26 elements (3D 2^27):
+// 0.45 to 0.95 of rocFFT's time.  A listed size is transformed here from
+// `from` to `to` thousand elements in all (measured at 10 to 23 batches each;
+// the lines lie between the two that they part).
+constexpr int64_t ALL = int64_t(1) << 40;
+struct window {
+    int dim, N;
+    int64_t from, to;
+};
+constexpr window windows[] = {
+    {2, 12, ALL, ALL}, {2, 14, 280, ALL}, {2, 15, ALL, ALL}, {2, 16, ALL, ALL}, {2, 18, ALL, ALL}, {2, 20, ALL, ALL},
+    {2, 21, 390, ALL}, {2, 24, ALL, ALL}, {2, 25, ALL, ALL}, {2, 27, ALL, ALL}, {2, 28, 490, ALL}, {2, 30, 100, ALL},
+    {2, 32, ALL, ALL}, {2, 35, ALL, ALL}, {2, 36, 290, ALL}, {2, 40, 250, ALL}, {2, 42, 390, ALL}, {2, 45, 320, ALL},
+    {2, 48, ALL, ALL}, {2, 49, 380, ALL}, {2, 50, 390, 1600}, {2, 54, 320, 1300}, {2, 56, 490, ALL},
+    {2, 60, 280, ALL}, {2, 63, 310, 5700}, {2, 64, 320, 5900}, {2, 70, 270, ALL}, {2, 72, 410, 2300},
+    {2, 75, 220, ALL}, {2, 80, 350, 4000}, {2, 81, 510, 2100}, {2, 84, 280, 2200}, {2, 98, 530, 1100},
+    {2, 100, 0, 780}, {2, 105, 310, 2400}, {2, 108, 460, 3700}, {2, 112, 490, 3900}, {2, 125, 310, ALL},
+    {2, 128, 450, 2600}, {2, 135, 0, 1400}, {2, 144, 230, ALL}, {2, 160, 280, 4000}, {2, 162, 320, 1800},
+    {2, 168, 200, ALL}, {2, 192, 260, ALL}, {2, 200, 280, 35000}, {2, 216, 320, ALL}, {2, 224, 170, ALL},
+    {2, 240, 400, 36000}, {2, 243, 410, ALL}, {2, 256, 450, ALL}, {2, 280, 350, ALL}, {2, 336, 390, ALL},
+    {2, 343, 410, ALL}, {2, 512, 370, ALL}, {3, 16, ALL, ALL}, {3, 25, ALL, ALL}, {3, 27, ALL, ALL},
+    {3, 32, 450, ALL}, {3, 48, 270, ALL}, {3, 60, 310, ALL}, {3, 64, 910, ALL}, {3, 72, 530, 1800},
+    {3, 80, 720, 5000}, {3, 81, 0, 7400}, {3, 84, 0, 2100}, {3, 98, 0, 2200}, {3, 108, 0, 12000}, {3, 112, 0, 2000},
+    {3, 125, 0, 38000}, {3, 162, 15000, 42000}};
+
 }  // namespace
 
-// Whether f's size is transformed here; lays out its stages.
+// Whether f's grids are transformed here; lays out the stages.
 bool fr_fft_radices(fr_fft *f)
 {
     // (a grid below 2^32 bytes: 32-bit offsets)
-    return f->N <= (f->dim == 3 ? 800u : 1024u) && plan((int)f->N, f->desc);
+    if (f->N > (f->dim == 3 ? 800u : 1024u) || !plan((int)f->N, f->desc)) return false;
+    const int64_t thousands = (int64_t)f->batch * f->N * f->N * (f->dim == 3 ? f->N : 1) / 1000;
+    for (const window &w : windows)
+        if (w.dim == f->dim && w.N == (int)f->N) return thousands >= w.from && thousands < w.to;
+    return true;
 }
 
 // The grids of f's batch, in place; f->tw is set.  With an image (sum of

@@ -189,15 +189,15 @@ __device__ __forceinline__ int crop_pos(int k, int N, int rc, int shift)
     return kp >= 0 && kp < rc ? kp : -1;
 }
 
-// Where the last pass leaves the sum of squares of its coils: rc kept outputs
-// of its axis at out + k' outK, one element a kept column.  The arithmetic
-// and the order of k_sos (fr_image.hip).
+// Where the last pass leaves the image of its one coil: rc kept outputs of its
+// axis at out + k' outK, one element a kept column.  The arithmetic of k_sos
+// (fr_image.hip).
 struct sos_out {
     float *acc;                                 // LDS [rc][TC]
     float *out;
     const float *deapod;
-    int64_t coil, outK;
-    int C, rc, shift;
+    int64_t outK;
+    int rc, shift;
     int rcx, rcy;                               // columns kept: x and, in 3D, y
 };
 
@@ -272,10 +272,9 @@ __device__ __forceinline__ void stage(const fft_desc &d, int i, const tile_at &t
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const int kp = crop_pos(n + r * g.Ns, d.N, o.rc, o.shift);
-                    if (kp >= 0) {              // the same thread for every coil
-                        float &a = o.acc[(kp << d.ltc) + row[b]];
-                        a = __fadd_rn(a, __fadd_rn(__fmul_rn(x[b][r].x, x[b][r].x), __fmul_rn(x[b][r].y, x[b][r].y)));
-                    }
+                    if (kp >= 0)
+                        o.acc[(kp << d.ltc) + row[b]] =
+                            __fadd_rn(__fmul_rn(x[b][r].x, x[b][r].x), __fmul_rn(x[b][r].y, x[b][r].y));
                 }
             }
         } else {
@@ -305,8 +304,8 @@ __device__ __forceinline__ void transform(const fft_desc &d, const tile_at &t, f
 
 // Rows (ROWS): `count` rows of N, tile T the rows from T TC.  Columns: planes
 // of count columns, N apart by `step`; tile T the columns from (T mod tiles)
-// TC of plane T / tiles, planes `plane` elements apart.  SOS: the one plane of
-// each coil in turn, then the image.
+// TC of plane T / tiles, planes `plane` elements apart.  SOS: one plane, and
+// the image.
 template <bool ROWS, int NB, int S, bool SOS>
 __global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 6 : 4))) k_fft(
     float2 *data, const float2 *__restrict__ gtw, fft_desc d, int64_t count, uint32_t tiles, uint32_t all, int64_t step,
@@ -330,12 +329,8 @@ __global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_e
         transform<ROWS, NB, S, false>(d, t, buf, sm, gtw, o);
     } else {
         o.acc = reinterpret_cast<float *>(buf + ((size_t)d.N << d.ltc));
-        for (int i = threadIdx.x; i < o.rc << d.ltc; i += blockDim.x) o.acc[i] = 0.f;
-        for (int c = 0; c < o.C; ++c) {         // (two stages or more: a barrier before the first use of acc)
-            transform<ROWS, NB, S, true>(d, t, buf, sm, gtw, o);
-            t.base += 8 * o.coil;
-            __syncthreads();
-        }
+        transform<ROWS, NB, S, true>(d, t, buf, sm, gtw, o);
+        __syncthreads();
         for (int i = threadIdx.x; i < o.rc << d.ltc; i += blockDim.x) {
             const int kp = i >> d.ltc, row = i & ((1 << d.ltc) - 1);
             if (row >= t.rows) continue;
@@ -476,9 +471,8 @@ bool fr_fft_radices(fr_fft *f)
     return true;
 }
 
-// The grids of f's batch, in place; f->tw is set.  With an image (sum of
-// squares over the C coils of one grid each, kept outputs rcx x rcy x rcz),
-// the last pass takes a tile's coils in turn and forms it.
+// The grids of f's batch, in place; f->tw is set.  With an image (of one coil
+// and grid, kept outputs rcx x rcy x rcz), the last pass forms it.
 static fr_status passes(fr_fft *f, float2 *data, const sos_out *sos)
 {
     const int64_t N = f->N, B = f->batch, last = sos ? 1 : B;
@@ -491,10 +485,15 @@ static fr_status passes(fr_fft *f, float2 *data, const sos_out *sos)
 
 fr_status fr_fft_passes(fr_fft *f, float2 *data) { return passes(f, data, nullptr); }
 
-// Whether the image comes out of the last pass: for one coil (96^2: 6.1 us
-// against 4.9 and 2.6 for k_sos and a launch).  Several coils would go one
-// after the other, nothing loaded ahead: 5 x 180^3 145 us against 96 and 12.
-bool fr_fft_sos_last(const fr_fft *f, const fr_grids *g) { return f->own && g->frames == 0 && g->C == 1; }
+// Whether the image comes out of the last pass: of one coil, in 2D and of 3D
+// grids up to 2^20 cells (a launch less: 96^2 9.9 us against 11.8 with k_sos,
+// 40^3 13.6 and 15.0, 96^3 24.6 and 26.4).  Above, the pass with its image is
+// the slower one (144^3 52.9 us and 52.2, 240^3 156.9 and 150.9), and several
+// coils would go one after the other, nothing loaded ahead.
+bool fr_fft_sos_last(const fr_fft *f, const fr_grids *g)
+{
+    return f->own && g->frames == 0 && g->C == 1 && (g->dim == 2 || g->cells <= (size_t(1) << 20));
+}
 
 fr_status fr_fft_passes_sos(fr_fft *f, const fr_grids *g, int rcx, int rcy, int rcz, int shift, const float *deapod,
                             float *out)
@@ -502,8 +501,6 @@ fr_status fr_fft_passes_sos(fr_fft *f, const fr_grids *g, int rcx, int rcy, int 
     sos_out o{};
     o.out = out;
     o.deapod = deapod;
-    o.C = g->C;
-    o.coil = (int64_t)g->cells;
     o.rc = g->dim == 3 ? rcz : rcy;
     o.outK = g->dim == 3 ? (int64_t)rcy * rcx : rcx;
     o.rcx = rcx;

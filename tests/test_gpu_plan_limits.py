@@ -80,3 +80,28 @@ def test_more_units_than_a_launch_has_waves(ctx):
     small, large = corner(ctx, 64, 0, M), corner(ctx, 1290, 1220, M)
     assert small[0] == large[0]
     np.testing.assert_array_equal(small[1], large[1])
+
+
+def test_data_past_4_gib(ctx):
+    """Rows addressed in 64 bits: coils of one data set times powers of two, bit for bit that set's grid times them."""
+    rng = np.random.default_rng(2)
+    N, M, C = 48, 8_400_000, 65
+    t = rng.uniform(0, N - 1, (M, 3)).astype(np.float32)
+    y = rng.standard_normal((M, 2)).astype(np.float32).view(np.complex64)[:, 0]
+    lut, _ = hip.kb_lut(4.0, 2.0, 512)
+    grids = []
+    for coils in (1, C):
+        s = hip.Samples(ctx, 3, M, coils)
+        assert (8 * (M + 1) * coils >= 1 << 32) == (coils == C)
+        s.set_traj(t)
+        s.set_dcf(np.ones(M, np.float32))
+        for c in range(coils):
+            s.set_coil(c, y * np.float32(2.0 ** (c % 7)))
+        g = hip.Grids(ctx, 3, N, coils)
+        p = hip.Plan(ctx, s, N, 4.0, lut)
+        hip.grid_execute(p, s, g)
+        grids.append(g.download_all())
+        for h in (g, p, s):
+            h.close()
+    for c in range(C):
+        np.testing.assert_array_equal(grids[1][c], grids[0][0] * np.float32(2.0 ** (c % 7)))

@@ -40,3 +40,28 @@ def test_density_that_is_not_finite(ctx, dim, N, M, value):
     assert 0 < (got[1] == 0).sum() < M // 2
     np.testing.assert_array_equal(got[0] == 0, got[1] == 0)
     np.testing.assert_allclose(got[0], got[1], rtol=1e-5)
+
+
+@pytest.mark.parametrize("dim,N,M", [(3, 27, 6000), (2, 53, 9000)])
+def test_start_from_a_density(ctx, orc, dim, N, M):
+    """Three iterations and three more from their density are six, bit for bit; from a random density, the FP64
+    oracle's (bar: 1e-6 as for the other Pipe-Menon tests)."""
+    rng = np.random.default_rng(N)
+    t = rng.uniform(-1.0, N, (M, dim))
+    t[: M // 2] = rng.normal(N / 2, N / 12, (M // 2, dim))
+    t = t.astype(np.float32)
+    lut, _ = hip.kb_lut(4.0, 2.0, 512)
+    s = samples(ctx, t, np.ones(M, np.float32))
+    p = hip.Plan(ctx, s, N, 4.0, lut)
+    hip.pipe_menon(p, s, 6, True)
+    six = s.get_dcf()
+    hip.pipe_menon(p, s, 3, True)
+    hip.pipe_menon(p, s, 3, False)
+    np.testing.assert_array_equal(s.get_dcf().view(np.int32), six.view(np.int32))
+    w0 = rng.uniform(0.1, 3.0, M).astype(np.float32)
+    s.set_dcf(w0)
+    hip.pipe_menon(p, s, 4, False)
+    ref = orc.pipe_menon(t, N, 4.0, lut, iters=4, w0=w0)
+    e = np.linalg.norm(s.get_dcf() - ref) / np.linalg.norm(ref)
+    print(f"[pipe-menon from a density dim={dim} N={N}] rel-L2 {e:.2e}", flush=True)
+    assert e <= 1e-6

@@ -373,7 +373,7 @@ __global__ void k_transpose_cm_to_sm(const float2 *__restrict__ in, int64_t M, i
 
 __global__ void k_convert_sm_c16(const float2 *__restrict__ in, int64_t n, __half2 *__restrict__ out)
 {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = fr_element();
     if (i < n) {
         float2 v = in[i];
         out[i] = __halves2half2(__float2half_rn(v.x), __float2half_rn(v.y));
@@ -537,7 +537,7 @@ extern "C" fr_status fr_samples_set_data_device(fr_samples *s, const void *data,
         if (s->type == FR_SAMPLES_C64) {
             FR_HIP(ctx, hipMemcpyAsync(s->data, data, 8 * (size_t)n, hipMemcpyDeviceToDevice, ctx->stream));
         } else {
-            hipLaunchKernelGGL(k_convert_sm_c16, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream,
+            hipLaunchKernelGGL(k_convert_sm_c16, fr_elements(n, 256), dim3(256), 0, ctx->stream,
                                (const float2 *)data, n, (__half2 *)s->data);
         }
     } else {

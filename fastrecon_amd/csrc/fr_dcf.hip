@@ -17,7 +17,7 @@ __global__ void k_degrid(const float *__restrict__ traj, int64_t M, int dim, int
                          const float *__restrict__ lut, const float2 *__restrict__ grid, size_t cells, int C,
                          float2 *__restrict__ out, int frames)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = fr_element();
     if (i >= M * C) return;
     const int64_t s = i / C;
     const int c = (int)(i - s * C);
@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256) k_degrid_thr(const float *__restrict__ tr
     for (int q = threadIdx.x; q <= L; q += blockDim.x) pairs[q] = gpairs[q];
     for (int q = threadIdx.x; q < L; q += blockDim.x) slut[q] = lut[q];
     __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = fr_element();
     if (i >= M * C) return;
     const int64_t s = i / C;
     const int c = (int)(i - s * C);
@@ -328,13 +328,13 @@ fr_status fr_degrid_raw(fr_plan *p, const fr_samples *s, const float2 *grid, int
     fr_ctx *ctx = p->ctx;
     if (p->mfma_pairs) {
         const size_t lds = sizeof(float2) * (p->L + 1) + sizeof(float) * p->L;
-        hipLaunchKernelGGL(k_degrid_thr, dim3(nblk(p->M * C, 256)), dim3(256), lds, ctx->stream, s->traj, p->M,
+        hipLaunchKernelGGL(k_degrid_thr, fr_elements(p->M * C, 256), dim3(256), lds, ctx->stream, s->traj, p->M,
                            p->dim, (int)p->N, p->kHW, p->L, p->lut, p->mfma_pairs, p->mfma_dacc, p->mfma_cidx, grid,
                            fr_plan_cells(p->dim, p->N, p->frames), C, out, p->frames);
         FR_HIP(ctx, hipGetLastError());
         return FR_OK;
     }
-    hipLaunchKernelGGL(k_degrid, dim3(nblk(p->M * C, 256)), dim3(256), 0, ctx->stream, s->traj, p->M, p->dim,
+    hipLaunchKernelGGL(k_degrid, fr_elements(p->M * C, 256), dim3(256), 0, ctx->stream, s->traj, p->M, p->dim,
                        (int)p->N, p->kHW, p->L, p->lut, grid, fr_plan_cells(p->dim, p->N, p->frames), C, out,
                        p->frames);
     FR_HIP(ctx, hipGetLastError());

@@ -410,7 +410,7 @@ fr_status pass(fr_fft *f, float2 *data, int64_t planes, int64_t count, int64_t s
     const size_t lds = sizeof(float2) * (d.N + ((size_t)(ROWS ? d.pitch : d.N) << d.ltc)) +
                        (sos ? sizeof(float) * ((size_t)sos->rc << d.ltc) : 0);
     const int64_t W = planes * tiles();
-    FR_CHECK(ctx, W < (int64_t(1) << 31), FR_ERR_UNSUPPORTED, "FFT launch of %lld workgroups", (long long)W);
+    FR_CHECK(ctx, (W + 8) * threads < (int64_t(1) << 32), FR_ERR_UNSUPPORTED, "FFT launch of %lld workgroups", (long long)W);
     const bool pos = f->sign > 0;
     auto kern = each == 1 ? (pos ? k_fft<ROWS, 1, 1, false> : k_fft<ROWS, 1, -1, false>)
                           : (pos ? k_fft<ROWS, 2, 1, false> : k_fft<ROWS, 2, -1, false>);

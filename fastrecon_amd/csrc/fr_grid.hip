@@ -466,7 +466,9 @@ fr_status launch(fr_plan *p, const fr_samples *s, float2 *out, float2 *partial)
     const size_t cells = fr_plan_cells(p->dim, p->N, p->frames);
     const int64_t light = p->nitems - p->nitems_front;
     const int64_t span = 8 * XCD_RUN;
-    dim3 grid((unsigned)(p->nitems_front + span * ((light + span - 1) / span)), chunks);
+    const int64_t W = p->nitems_front + span * ((light + span - 1) / span);
+    FR_CHECK(ctx, W * 64 < (int64_t(1) << 32), FR_ERR_UNSUPPORTED, "gridding launch of %lld workgroups", (long long)W);
+    dim3 grid((unsigned)W, chunks);
     if constexpr (ACC == FR_ACC_GATHER) {
         const size_t glds = sizeof(float) * (size_t)(GB + 1) * 64;
         hipLaunchKernelGGL(k_grid_gather<TS>, grid, dim3(64), glds, ctx->stream, p->items, p->nitems, p->units,

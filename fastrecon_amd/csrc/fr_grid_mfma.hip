@@ -407,6 +407,7 @@ fr_status launch_mfma_ct(fr_plan *p, const fr_samples *s, float2 *out, float2 *p
     constexpr int IPW = items_per_wg<NBLK>();
     const int64_t groups = (light + IPW - 1) / IPW, span = 8 * (XCD_RUN / IPW);
     const int64_t W = p->nitems_front + span * ((groups + span - 1) / span);
+    FR_CHECK(ctx, W * 64 < (int64_t(1) << 32), FR_ERR_UNSUPPORTED, "gridding launch of %lld workgroups", (long long)W);
     hipLaunchKernelGGL((k_grid_mfma<NBLK, NCB, PAIR, CT, FULL, TS>), dim3((unsigned)W, chunks), dim3(64), 0, ctx->stream,
                        p->items, p->nitems, p->units, p->hdrs, p->tstart, (const void *)p->taps, (const TS *)s->data,
                        s->dcf,

@@ -21,7 +21,7 @@ __global__ void k_fftshift(float2 *__restrict__ g, int dim, int N, int C, size_t
 {
     const int h = N / 2;
     const size_t half = cells / 2;                       // elements with slow coord < N/2
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t i = (size_t)fr_element();
     if (i >= half * C) return;
     const int c = (int)(i / half);
     const size_t r = i - (size_t)c * half;
@@ -168,7 +168,7 @@ extern "C" fr_status fr_fftshift(fr_ctx *ctx, fr_grids *g)
     const int batch = g->C * std::max(g->frames, 1);
     const size_t cells = g->frames > 0 ? (size_t)g->N * g->N : g->cells;
     const size_t n = cells / 2 * batch;
-    hipLaunchKernelGGL(k_fftshift, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, g->data, g->dim, (int)g->N, batch,
+    hipLaunchKernelGGL(k_fftshift, fr_elements(n, 256), dim3(256), 0, ctx->stream, g->data, g->dim, (int)g->N, batch,
                        cells);
     FR_HIP(ctx, hipGetLastError());
     return FR_OK;
@@ -287,7 +287,7 @@ __global__ void k_crop(const float2 *__restrict__ in, int dim, int N, int C, siz
                        float2 *__restrict__ out)
 {
     const size_t n = (size_t)rcx * rcy * rcz;
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t i = (size_t)fr_element();
     if (i >= n * C) return;
     const int c = (int)(i / n);
     const size_t o = i - (size_t)c * n;
@@ -377,7 +377,7 @@ extern "C" fr_status fr_crop(fr_ctx *ctx, const fr_grids *g, unsigned rcx, unsig
              FR_ERR_INVALID, "crop %ux%ux%u outside grid %u", rcx, rcy, rcz, g->N);
     const size_t n = (size_t)rcx * rcy * rcz * g->C;
     FR_EXTENT(ctx, out_dev, sizeof(float2) * n, "fr_crop output");
-    hipLaunchKernelGGL(k_crop, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, g->data, g->dim, (int)g->N, g->C,
+    hipLaunchKernelGGL(k_crop, fr_elements(n, 256), dim3(256), 0, ctx->stream, g->data, g->dim, (int)g->N, g->C,
                        g->cells, (int)rcx, (int)rcy, (int)rcz, (float2 *)out_dev);
     FR_HIP(ctx, hipGetLastError());
     return FR_OK;

@@ -327,6 +327,19 @@ void fr_pool_free(fr_ctx *ctx, void *p);
 bool fr_keep(fr_kept **list, void *p);
 void fr_free_kept(fr_ctx *ctx, fr_kept *list);
 
+// A launch of one thread an element, where the elements may be 2^32 and more
+// (samples times coils, cells times coils): a launch takes below 2^32
+// work-items along x and does nothing, without an error, beyond.
+static inline dim3 fr_elements(uint64_t n, unsigned b)
+{
+    const uint64_t blocks = (n + b - 1) / b, most = uint64_t(1) << 22;
+    return blocks <= most ? dim3((unsigned)blocks) : dim3((unsigned)most, (unsigned)((blocks + most - 1) / most));
+}
+static __device__ __forceinline__ int64_t fr_element()
+{
+    return ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
+}
+
 static inline size_t fr_cells(int dim, unsigned N)
 {
     return dim == 3 ? (size_t)N * N * N : (size_t)N * N;

@@ -105,3 +105,42 @@ def test_data_past_4_gib(ctx):
             h.close()
     for c in range(C):
         np.testing.assert_array_equal(grids[1][c], grids[0][0] * np.float32(2.0 ** (c % 7)))
+
+
+def test_degridding_of_2_32_values(ctx):
+    """More sample-coils than a launch has work-items along one axis, by the general kernel (a wide kernel)."""
+    rng = np.random.default_rng(3)
+    N, M, C, width, part = 16, 1 << 26, 66, 4.5, 1000
+    t = rng.integers(0, 16 * (N - 1), (part, 3)).astype(np.float32) / 16
+    all_t = np.empty((M, 3), np.float32)
+    all_t[:] = t[0]
+    all_t[:part] = all_t[-part:] = t
+    lut, _ = hip.kb_lut(width, 2.0, 64)
+    g = hip.Grids(ctx, 3, N, C)
+    for c in range(C):
+        g.upload(c, (rng.standard_normal(N ** 3) + 1j * rng.standard_normal(N ** 3)).astype(np.complex64))
+
+    def handle(points):
+        s = hip.Samples(ctx, 3, len(points), 1)
+        s.set_traj(points)
+        return s
+
+    s = handle(t)
+    small = hip.DeviceBuffer(ctx, 8 * part * C)
+    hip.degrid_execute(hip.Plan(ctx, s, N, width, lut, dict(accumulate=2)), s, g, small)
+    ref = small.to_host(np.int32)
+    s = handle(all_t)
+    plan = hip.Plan(ctx, s, N, width, lut)
+    out = hip.DeviceBuffer(ctx, 8 * M * C)
+    last = hip.DevicePtr(out, 8 * C * (M - part))
+    zero = np.zeros(2 * part * C, np.float32)
+    got = np.empty(2 * part * C, np.int32)
+    L = ctx.L
+    for p in (out.ptr, last.ptr):
+        ctx.check(L.fr_memcpy_h2d(ctx.h, p, zero.ctypes.data, zero.nbytes), "fr_memcpy_h2d")
+    hip.degrid_execute(plan, s, g, out)
+    for p in (out.ptr, last.ptr):
+        ctx.check(L.fr_memcpy_d2h(ctx.h, got.ctypes.data, p, got.nbytes), "fr_memcpy_d2h")
+        np.testing.assert_array_equal(got, ref)
+    for h in (out, plan, s, g):
+        h.close()

@@ -426,37 +426,36 @@ fr_status pass(fr_fft *f, float2 *data, int64_t planes, int64_t count, int64_t s
     return FR_OK;
 }
 
-// Where rocFFT's kernels are the faster ones.  It has kernels that transform
-// these sizes in one pass over a small 2D grid, or in one pass an axis without
-// transposes, and a launch or two less, or more threads at work in each
-// stage, beats these passes on few elements (4 x 240^2: 9.3 us against 11.5;
-// 16^2 to 48^2: half) and, where the radices of a size leave threads idle in
-// some stages (the 7s and 2 of 98), on many (8 x 98^3: 98 against 112).  At
-// the sizes not listed, of all that plan() takes up to 1000^2 and 400^3, these
-// passes were faster, or within 3%, from 1 grid to 2^26 elements (3D 2^27):
-// 0.45 to 0.95 of rocFFT's time.  A listed size is transformed here from
-// `from` to `to` thousand elements in all (measured at 10 to 23 batches each;
-// the lines lie between the two that they part).
+// Where rocFFT's kernels are the faster ones by more than 6% somewhere.  It
+// has kernels that transform these sizes in one pass over a small 2D grid, or
+// in one pass an axis without transposes, and a launch or two less, or more
+// threads at work in each stage, beats these passes on few elements (4 x 240^2:
+// 9.3 us against 11.5; 16^2 to 48^2: half) and, where the radices of a size
+// leave threads idle in some stages (the 7s and 2 of 98), on many (16 x 98^3: 175
+// against 199).  A listed size is transformed here from `from` to `to` thousand
+// elements in all (measured at 10 to 23 batches each, the lines between the two
+// that they part; where both are within 6%, here: rocFFT's plan takes 2 to 40
+// ms to make).  At the sizes not listed, of all that plan() takes up to 1000^2
+// and 400^3, these passes took 0.45 to 1.06 of rocFFT's time from 1 grid to 2^26
+// elements (3D 2^27), up to 1.15 (24^2: 1.2) at few elements of 12^2 to 24^2,
+// 70^2, 144^2, 224^2, 48^3 and 60^3.
 constexpr int64_t ALL = int64_t(1) << 40;
 struct window {
     int dim, N;
     int64_t from, to;
 };
 constexpr window windows[] = {
-    {2, 12, ALL, ALL}, {2, 14, 280, ALL}, {2, 15, ALL, ALL}, {2, 16, ALL, ALL}, {2, 18, ALL, ALL}, {2, 20, ALL, ALL},
-    {2, 21, 390, ALL}, {2, 24, ALL, ALL}, {2, 25, ALL, ALL}, {2, 27, ALL, ALL}, {2, 28, 490, ALL}, {2, 30, 100, ALL},
-    {2, 32, ALL, ALL}, {2, 35, ALL, ALL}, {2, 36, 290, ALL}, {2, 40, 250, ALL}, {2, 42, 390, ALL}, {2, 45, 320, ALL},
-    {2, 48, ALL, ALL}, {2, 49, 380, ALL}, {2, 50, 390, 1600}, {2, 54, 320, 1300}, {2, 56, 490, ALL},
-    {2, 60, 280, ALL}, {2, 63, 310, 5700}, {2, 64, 320, 5900}, {2, 70, 270, ALL}, {2, 72, 410, 2300},
-    {2, 75, 220, ALL}, {2, 80, 350, 4000}, {2, 81, 510, 2100}, {2, 84, 280, 2200}, {2, 98, 530, 1100},
-    {2, 100, 0, 780}, {2, 105, 310, 2400}, {2, 108, 460, 3700}, {2, 112, 490, 3900}, {2, 125, 310, ALL},
-    {2, 128, 450, 2600}, {2, 135, 0, 1400}, {2, 144, 230, ALL}, {2, 160, 280, 4000}, {2, 162, 320, 1800},
-    {2, 168, 200, ALL}, {2, 192, 260, ALL}, {2, 200, 280, 35000}, {2, 216, 320, ALL}, {2, 224, 170, ALL},
-    {2, 240, 400, 36000}, {2, 243, 410, ALL}, {2, 256, 450, ALL}, {2, 280, 350, ALL}, {2, 336, 390, ALL},
-    {2, 343, 410, ALL}, {2, 512, 370, ALL}, {3, 16, ALL, ALL}, {3, 25, ALL, ALL}, {3, 27, ALL, ALL},
-    {3, 32, 450, ALL}, {3, 48, 270, ALL}, {3, 60, 310, ALL}, {3, 64, 910, ALL}, {3, 72, 530, 1800},
-    {3, 80, 720, 5000}, {3, 81, 0, 7400}, {3, 84, 0, 2100}, {3, 98, 0, 2200}, {3, 108, 0, 12000}, {3, 112, 0, 2000},
-    {3, 125, 0, 38000}, {3, 162, 15000, 42000}};
+    {2, 14, 280, ALL}, {2, 15, ALL, ALL}, {2, 16, ALL, ALL}, {2, 18, ALL, ALL}, {2, 21, 280, ALL}, {2, 25, ALL, ALL},
+    {2, 27, ALL, ALL}, {2, 28, 250, ALL}, {2, 30, 100, ALL}, {2, 32, ALL, ALL}, {2, 35, ALL, ALL}, {2, 36, 290, ALL},
+    {2, 40, 130, ALL}, {2, 42, 390, ALL}, {2, 45, 220, ALL}, {2, 48, ALL, ALL}, {2, 49, 380, ALL},
+    {2, 50, 390, 1600}, {2, 54, 230, 1300}, {2, 56, 250, ALL}, {2, 60, 280, ALL}, {2, 63, 310, ALL},
+    {2, 64, 320, ALL}, {2, 72, 290, 2300}, {2, 75, 220, ALL}, {2, 80, 350, ALL}, {2, 81, 360, 2100},
+    {2, 84, 200, 2200}, {2, 98, 380, 1100}, {2, 100, 0, 780}, {2, 105, 220, 3000}, {2, 108, 320, 3700},
+    {2, 112, 350, 3900}, {2, 125, 310, ALL}, {2, 128, 320, 2600}, {2, 135, 0, 1400}, {2, 160, 180, 4000},
+    {2, 162, 320, 1800}, {2, 168, 200, ALL}, {2, 200, 280, ALL}, {2, 216, 320, ALL}, {2, 240, 400, ALL},
+    {2, 243, 410, ALL}, {2, 256, 450, ALL}, {2, 280, 350, ALL}, {2, 336, 280, ALL}, {2, 343, 410, ALL},
+    {2, 512, 370, ALL}, {3, 16, ALL, ALL}, {3, 25, ALL, ALL}, {3, 27, ALL, ALL}, {3, 32, 450, ALL},
+    {3, 64, 640, ALL}, {3, 72, 530, 1800}, {3, 84, 0, 2100}, {3, 98, 0, 4500}, {3, 108, 0, 12000}, {3, 112, 0, 2000}, {3, 125, 0, 38000}};
 
 }  // namespace
 

@@ -106,15 +106,16 @@ __device__ __forceinline__ void dft(float2 (&x)[R])
         x[2] = a - c;
         x[3] = sub_i(b, d);
     } else if constexpr (R == 5) {
-        // cos(2 pi / 5), cos(4 pi / 5) = -1/4 +- sqrt(5) / 4
-        constexpr real2 k = two(0.55901699437494742410), s1 = two(0.95105651629515357212), s2 = two(0.58778525229247312917);
+        // (cosines as -1/4 +- sqrt(5) / 4 take fewer products, but round once
+        // more: 160^3 1.66e-7 from FP64 against 1.6e-7)
+        constexpr real2 c1 = two(0.30901699437494742410), c2 = two(-0.80901699437494742410);
+        constexpr real2 s1 = two(0.95105651629515357212), s2 = two(0.58778525229247312917);
         constexpr real2 m1 = two(-0.95105651629515357212);
-        const float2 p1 = x[1] + x[4], p2 = x[2] + x[3], p = p1 + p2, t = scale(p1 - p2, k);
+        const float2 p1 = x[1] + x[4], p2 = x[2] + x[3];
         const float2 d1 = S > 0 ? x[1] - x[4] : x[4] - x[1], d2 = S > 0 ? x[2] - x[3] : x[3] - x[2];
-        const float2 m = make_float2(__builtin_fmaf(p.x, -0.25f, x[0].x), __builtin_fmaf(p.y, -0.25f, x[0].y));
-        const float2 a = m + t, b = m - t;
+        const float2 a = axpy(axpy(x[0], p1, c1), p2, c2), b = axpy(axpy(x[0], p1, c2), p2, c1);
         const float2 u = axpy(scale(d1, s1), d2, s2), v = axpy(scale(d1, s2), d2, m1);
-        x[0] = x[0] + p;
+        x[0] = x[0] + (p1 + p2);
         x[1] = add_i(a, u);
         x[4] = sub_i(a, u);
         x[2] = add_i(b, v);
@@ -307,7 +308,7 @@ __device__ __forceinline__ void transform(const fft_desc &d, const tile_at &t, f
 // TC of plane T / tiles, planes `plane` elements apart.  SOS: one plane, and
 // the image.
 template <bool ROWS, int NB, int S, bool SOS>
-__global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_eu(NB == 1 ? 6 : 4))) k_fft(
+__global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_eu(NB == 1 || ROWS ? 8 : SOS ? 6 : 7))) k_fft(
     float2 *data, const float2 *__restrict__ gtw, fft_desc d, int64_t count, uint32_t tiles, uint32_t all, int64_t step,
     int64_t plane, sos_out o)
 {

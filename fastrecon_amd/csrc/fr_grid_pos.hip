@@ -6,7 +6,7 @@
 // compact 16-cell box: a radius-2 kernel ball meets about 8 such boxes per
 // sample, against 10 for 8 x 2 x 1).  The plan lists, per unit, the samples
 // that have at least one accepted tap in it (ascending sample order, padded
-// to a multiple of 4 with a null sample).  Four records at a time are one
+// to a multiple of 16 with a null sample).  Four records at a time are one
 // dense product per 16 components
 //
 //     acc[16 cells][16 components] += A[16 cells][4 records] * B[4 records][16 components]
@@ -219,8 +219,8 @@ __device__ __forceinline__ void lane_cell(const item_box &b, int j, float &fx, f
 // 2^30), returns false.
 //
 // Records come in blocks of 64, one per lane: one load brings a block's
-// sample indices and one its positions and DCFs, which go through LDS (pbuf,
-// two blocks) to the 16 lanes that need each; the indices reach the lanes
+// sample indices and one its positions and DCFs, which go through LDS (pbuf)
+// to the 16 lanes that need each; the indices reach the lanes
 // that load a record's row by a lane exchange.  (Loaded where they are used,
 // each by 16 lanes, positions and indices took 16 times the load
 // instructions and return traffic of these.)  Software pipeline: while batch
@@ -231,9 +231,9 @@ __device__ __forceinline__ void lane_cell(const item_box &b, int j, float &fx, f
 // the waves that fit a SIMD, and at 32 coils by the traffic of the rows past
 // L2 as well: up to 16 coils, where six waves fit instead of five (a wave's
 // records and its write-out share their LDS, 80 VGPRs), 16 FP16 coils at
-// 384^3 went from 7.00 to 6.69 ms and 12 coils of 64 frames on 384^2 from
-// 1.19 to 1.13, while a third fewer VALU instructions a weight (squared
-// distances along each axis formed once a record) gained nothing: 7.01.  By
+// 384^3 went from 7.00 to 6.7 - 6.9 ms, by the run, and 12 coils of 64 frames
+// on 384^2 from 1.19 to 1.14, while a third fewer VALU instructions a weight
+// (squared distances along each axis formed once a record) gained nothing: 7.01.  By
 // blocks at all: 32 coils at 256^3 4.71 -> 4.13 ms (now 4.06), 16 FP16 coils
 // at 384^3 7.75 -> 7.12.  Rows fetched two or three batches ahead were slower
 // (the extra ones past an item's end cost as much as useful ones): 8.1 and
@@ -477,10 +477,10 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(po
     // ----------------------------------------------------------- pairs
     // One wave grids the two x-adjacent units of a pair one after the other,
     // the first unit's sums held in registers, and writes them out together:
-    // rows of 2 bx cells (64 bytes for 4-cell-wide units) instead of bx.  (Stored straight from the
-    // accumulators, 16 bytes of a row at a time, 32 coils at 256^3 took 4.87
-    // ms against 4.31 with an LDS transpose by 4-byte words and 4.13 with this
-    // one by 16-byte words.)
+    // rows of 2 bx cells (64 bytes for 4-cell-wide units) instead of bx.
+    // (Stored straight from the accumulators, 16 bytes of a row at a time, 32
+    // coils at 256^3 took 4.87 ms against 4.31 with an LDS transpose by 4-byte
+    // words and 4.13 with this one by 16-byte words.)
     if (bid >= front_wg && ntiles > 0) {
         const int64_t pidx = fr_sampled_tile(grp * PW + wv, tstride);   // (tstride 1: every pair)
         if (pidx >= ntiles) return;
@@ -534,7 +534,8 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(po
         const int cell = 2 * (lane & 15), x = cell & ((2 << lbx) - 1), row = cell >> (lbx + 1);
         const size_t go = ((size_t)(ba.oz + (row >> lby)) * N + (ba.oy + (row & ((1 << lby) - 1)))) * N + (ba.ox + x);
         // floats from the lane's first cell to its second and third: boxes
-        // less than 4 wide hold those in a next row
+        // less than 4 wide hold those in a next row (2 x 2 x 4, 32 coils on
+        // 128^3: 498 us, 883 as single units)
         const int d1 = lbx >= 1 ? 2 : 4, d2 = lbx >= 2 ? 4 : 8;
         constexpr int steps = NCB == 4 ? 2 : 1, ncs = NCB == 1 ? 8 : 16;
 #pragma unroll
@@ -594,7 +595,8 @@ __global__ void __launch_bounds__(64 * PW) __attribute__((amdgpu_waves_per_eu(po
     if (ipw > 1 && bid >= front_wg) {
         // A run of light items (one each a unit, their records consecutive)
         // as one record stream: at an item's end the pipeline keeps running
-        // while the unit is written out, from LDS beside the positions.
+        // while the unit is written out, from LDS beside the positions (4
+        // items a wave, 8 coils on 180^3: 283 us, drained at each item 317).
         // Units without records are written as zeros.
         auto next = [&]() __attribute__((always_inline)) {
             write_out(it, box);

@@ -988,7 +988,7 @@ extern "C" fr_status fr_plan_get_info(const fr_plan *p, fr_plan_info *info)
     info->tiles = (int)std::min<int64_t>(p->nunits, INT32_MAX);
     info->lds_bytes = 0;
     if (p->accumulate == FR_ACC_POS)
-        info->plan_bytes = (int64_t)sizeof(uint32_t) * (p->nrecs_padded + 64) + (int64_t)sizeof(float4) * (p->M + 1) +
+        info->plan_bytes = (int64_t)sizeof(uint32_t) * (p->nrecs_padded + FR_POS_PAD) + (int64_t)sizeof(float4) * (p->M + 1) +
                            (int64_t)sizeof(fr_unit) * p->nunits + (int64_t)sizeof(fr_item) * p->nitems;
     else
         info->plan_bytes = (int64_t)(sizeof(uint2) + sizeof(uint32_t)) * p->nrecords +

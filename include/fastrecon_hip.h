@@ -93,8 +93,10 @@ typedef struct {
                                     XCDs takes in launch order (0: 256)         */
     int stores;                  /* accumulate 6: grid stores 0: automatic
                                     (cached), 1: streaming (nontemporal), 2: cached */
-    int waves_per_simd;          /* accumulate 6: 0: automatic (4), 3 or 4 (the
-                                    kernel variant compiled for that occupancy) */
+    int waves_per_simd;          /* accumulate 6: 0: automatic (4), 3 or 4: the
+                                    kernel variant compiled to leave room for
+                                    that many waves above 16 coils (up to 16,
+                                    whose registers allow it, for 6)          */
     int tile_writes;             /* accumulate 6: 0: automatic (pairs), 1: four
                                     x-adjacent units per workgroup written out
                                     together in whole rows, 2: off (each unit
@@ -222,14 +224,18 @@ fr_status fr_grid_execute_noalloc(fr_plan *p, const fr_samples *s, fr_grids *out
  * orders its samples by grid tile on the first large call (not during a
  * capture, nor where there is no memory for it; or on the first
  * fr_dcf_pipe_menon) and keeps that order, about 16 bytes a sample, until
- * fr_plan_destroy. */
+ * fr_plan_destroy.  It serves the handle that the plan was built on, as long as
+ * its trajectory is not set again; other handles, and the same one from then on,
+ * take the general kernel (the same values, several times slower). */
 fr_status fr_degrid_execute(fr_plan *p, const fr_samples *s, const fr_grids *g, void *out_dev);
 
 /* -------------------------------------------------------------------- FFT */
 /* Replaces cuFFT (ImageFilter/cuFFT.cpp:15-37) and FFT (FFT.cpp:30-91):
- * one batched in-place C2C transform over all coils, unnormalised: sizes of
- * factors 2, 3, 5 and 7 up to 1024 (3D 800) by kernels of this library, the
- * others by rocFFT.
+ * one batched in-place C2C transform over all coils, unnormalised.  Kernels of
+ * this library take sizes up to 1024 (3D 800) that are products of at least two
+ * of 2 .. 8 and 10, none below N / 128 (so not 432, 576, 720, 768, 960 or 1024),
+ * but for sizes and batches that rocFFT is the faster one for (mostly small
+ * grids); rocFFT takes the others.
  * sign +1 is FFTW_BACKWARD / CUFFT_INVERSE, the reference default. */
 fr_status fr_fft_create(fr_ctx *ctx, int dim, unsigned N, int batch, int sign, fr_fft **out);
 fr_status fr_fft_destroy(fr_fft *f);

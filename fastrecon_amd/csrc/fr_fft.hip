@@ -13,10 +13,11 @@
 // writes.  Twiddles come from a table evaluated in FP64.
 //
 // Measured against rocFFT, whose plans of these sizes take strided passes and
-// transposes besides: 5 x 180^3 653 -> 315 us, 8 x 192^3 782 -> 709, 8 x 256^3
-// 1821 -> 1491, 8 x 96^3 94 -> 77, 8 x 512^2 31 -> 23 (about 4 TB/s where the
-// array is larger than the caches).  Relative L2 error 1.3e-7 .. 2.0e-7, up to
-// 17% below rocFFT's at each of 31 sizes from 96^2 to 288^3.
+// transposes besides: 4 x 180^3 466 -> 213 us, 8 x 192^3 738 -> 651, 8 x 256^3
+// 1799 -> 1451, 8 x 96^3 98 -> 74, 8 x 512^2 30 -> 21 (about 4 TB/s where the
+// array is larger than the caches).  White noise comes out 1.3e-7 .. 1.7e-7
+// from FP64, 4 to 18% nearer than rocFFT's at each of 34 sizes from 40^3 and
+// 96^2 to 288^3 and 640^2.
 #include "fr_internal.h"
 
 #include <algorithm>
@@ -43,9 +44,10 @@ __device__ __forceinline__ float2 cmul(float2 a, float2 b)
 // is the same relative error (1.8e-8 for sqrt(3) / 2) at every element of
 // every stage, which an image of several coils does not average out as it
 // does the elements' own roundings.  By the transform alone, 5 coils on 180^3
-// are 4.3e-8 from FP64 with both parts and 5.2e-8 with the first one (rocFFT
-// 5.5e-8); 5 x 250^2 5.0e-8 and 8.2e-8.  It costs nothing there that can be
-// seen (up to 4% at sizes of radix 10).
+// are 4.2e-8 from FP64 with both parts and 5.2e-8 with the first one (rocFFT
+// 5.5e-8).  The five-point butterfly's are in a form of fewer products, whose
+// one more rounding is not a bias; with it the pair costs nothing that can be
+// seen (up to 4% at 2D sizes of radix 10).
 struct real2 {
     float hi, lo;
 };
@@ -159,7 +161,8 @@ __device__ __forceinline__ void dft(float2 (&x)[R])
         constexpr double r3 = 0.86602540378443864676, C1 = 0.80901699437494742410, C2 = 0.30901699437494742410;
         constexpr double S1 = 0.58778525229247312917, S2 = 0.95105651629515357212;
         constexpr real2 wc[5] = {two(1.), two(R == 6 ? 0.5 : C1), two(R == 6 ? -0.5 : C2), two(-C2), two(-C1)};
-        constexpr real2 ws[5] = {two(0.), two(S * (R == 6 ? r3 : S1)), two(S * (R == 6 ? r3 : S2)), two(S * S2), two(S * S1)};
+        constexpr real2 ws[5] = {two(0.), two(S * (R == 6 ? r3 : S1)), two(S * (R == 6 ? r3 : S2)), two(S * S2),
+                                   two(S * S1)};
         constexpr real2 r2 = two(0.70710678118654752440);
 #pragma unroll
         for (int i = 0; i < H; ++i) {
@@ -308,9 +311,9 @@ __device__ __forceinline__ void transform(const fft_desc &d, const tile_at &t, f
 // TC of plane T / tiles, planes `plane` elements apart.  SOS: one plane, and
 // the image.
 template <bool ROWS, int NB, int S, bool SOS>
-__global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_eu(NB == 1 || ROWS ? 8 : SOS ? 6 : 7))) k_fft(
-    float2 *data, const float2 *__restrict__ gtw, fft_desc d, int64_t count, uint32_t tiles, uint32_t all, int64_t step,
-    int64_t plane, sos_out o)
+__global__ void __launch_bounds__(MAX_THREADS) __attribute__((amdgpu_waves_per_eu(NB == 1 || ROWS ? 8 : SOS ? 6 : 7)))
+k_fft(float2 *data, const float2 *__restrict__ gtw, fft_desc d, int64_t count, uint32_t tiles, uint32_t all,
+      int64_t step, int64_t plane, sos_out o)
 {
     extern __shared__ float2 sm[];              // twiddles [N], tile, sums
     float2 *buf = sm + d.N;
@@ -407,11 +410,13 @@ fr_status pass(fr_fft *f, float2 *data, int64_t planes, int64_t count, int64_t s
     while (d.nbmax << d.ltc > 2 * MAX_THREADS) --d.ltc;
     auto tiles = [&] { return (count + (1 << d.ltc) - 1) >> d.ltc; };
     while (d.ltc > 2 && planes * tiles() < (ROWS ? 4 : 1) * ctx->cu_count) --d.ltc;
-    const int work = d.nbmax << d.ltc, each = work > MAX_THREADS ? 2 : 1, threads = ((work + each - 1) / each + 63) & ~63;
+    const int work = d.nbmax << d.ltc, each = work > MAX_THREADS ? 2 : 1;
+    const int threads = ((work + each - 1) / each + 63) & ~63;
     const size_t lds = sizeof(float2) * (d.N + ((size_t)(ROWS ? d.pitch : d.N) << d.ltc)) +
                        (sos ? sizeof(float) * ((size_t)sos->rc << d.ltc) : 0);
     const int64_t W = planes * tiles();
-    FR_CHECK(ctx, (W + 8) * threads < (int64_t(1) << 32), FR_ERR_UNSUPPORTED, "FFT launch of %lld workgroups", (long long)W);
+    FR_CHECK(ctx, (W + 8) * threads < (int64_t(1) << 32), FR_ERR_UNSUPPORTED, "FFT launch of %lld workgroups",
+             (long long)W);
     const bool pos = f->sign > 0;
     auto kern = each == 1 ? (pos ? k_fft<ROWS, 1, 1, false> : k_fft<ROWS, 1, -1, false>)
                           : (pos ? k_fft<ROWS, 2, 1, false> : k_fft<ROWS, 2, -1, false>);
@@ -432,8 +437,8 @@ fr_status pass(fr_fft *f, float2 *data, int64_t planes, int64_t count, int64_t s
 // in one pass an axis without transposes, and a launch or two less, or more
 // threads at work in each stage, beats these passes on few elements (4 x 240^2:
 // 9.3 us against 11.5; 16^2 to 48^2: half) and, where the radices of a size
-// leave threads idle in some stages (the 7s and 2 of 98), on many (16 x 98^3: 175
-// against 199).  A listed size is transformed here from `from` to `to` thousand
+// leave threads idle in some stages (the 7s and 2 of 98), on many (16 x 98^3:
+// 175 against 199).  A listed size is transformed here from `from` to `to` thousand
 // elements in all (measured at 10 to 23 batches each, the lines between the two
 // that they part; where both are within 6%, here: rocFFT's plan takes 2 to 40
 // ms to make).  At the sizes not listed, of all that plan() takes up to 1000^2
@@ -456,7 +461,8 @@ constexpr window windows[] = {
     {2, 162, 320, 1800}, {2, 168, 200, ALL}, {2, 200, 280, ALL}, {2, 216, 320, ALL}, {2, 240, 400, ALL},
     {2, 243, 410, ALL}, {2, 256, 450, ALL}, {2, 280, 350, ALL}, {2, 336, 280, ALL}, {2, 343, 410, ALL},
     {2, 512, 370, ALL}, {3, 16, ALL, ALL}, {3, 25, ALL, ALL}, {3, 27, ALL, ALL}, {3, 32, 450, ALL},
-    {3, 64, 640, ALL}, {3, 72, 530, 1800}, {3, 84, 0, 2100}, {3, 98, 0, 4500}, {3, 108, 0, 12000}, {3, 112, 0, 2000}, {3, 125, 0, 38000}};
+    {3, 64, 640, ALL}, {3, 72, 530, 1800}, {3, 84, 0, 2100}, {3, 98, 0, 4500}, {3, 108, 0, 12000},
+    {3, 112, 0, 2000}, {3, 125, 0, 38000}};
 
 }  // namespace
 
